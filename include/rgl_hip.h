@@ -291,7 +291,7 @@ int rgl_mlp_train(rgl_gpu* gpu, const float* dev_samples, long long n, float* de
 /* No counterpart in the reference.  For callers that cannot allocate device
    memory (code under HIP graph capture, tight serving or training loops,
    harnesses that forbid hipMalloc): rgl_mlp_train with every training buffer
-   in one file-scope device array of 8.6 MB that each GPU holds until the
+   in one file-scope device array of 1.1 MB that each GPU holds until the
    process ends, so the call makes no hipMalloc, hipFree or other allocation.
    batch <= 4096 (RGL_E_CAPACITY beyond).  The last batch's loss goes to the
    device float *dev_loss_out (may be NULL) instead of host memory.  All

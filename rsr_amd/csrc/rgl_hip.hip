@@ -152,27 +152,19 @@ constexpr int kNumTimed = 9;
 // a StoreTrainingSamples request (no reference counterpart)
 struct SampleReq { float* out; uint32_t cap; uint32_t* count; float keep; uint32_t seed; };
 
-// device buffers of one training pass over a batch of B samples
-struct TrainBufs { float *X, *T, *H1, *H2, *H3, *Y, *dY, *dA, *dB, *Part, *Loss; };
+// device buffers of one training pass: the workgroups' partial gradient
+// sums, the batch's summed squared error and the weight image
+struct TrainBufs { float *Part, *Loss; uint16_t* Img; };
+
+// workgroups (and partial sums) of a training pass over B samples
+constexpr int train_groups(int B) { return (B + kTrChunk - 1) / kTrChunk; }
 
 // rgl_mlp_train_noalloc keeps its training buffers in one file-scope device
-// array, laid out for batches of at most kNoAllocMaxBatch samples; every
-// sub-buffer starts on a 256-byte boundary
+// array, laid out for batches of at most kNoAllocMaxBatch samples
 constexpr int kNoAllocMaxBatch = 4096;
-constexpr size_t kTrainChunk = 256;   // samples per split-K partial of the weight gradients
-constexpr size_t align64(size_t n) { return (n + 63) / 64 * 64; }
-constexpr size_t kScrX = 0;
-constexpr size_t kScrT = kScrX + align64(static_cast<size_t>(kNoAllocMaxBatch) * kMlpK1);
-constexpr size_t kScrH1 = kScrT + align64(static_cast<size_t>(kNoAllocMaxBatch) * 3);
-constexpr size_t kScrH2 = kScrH1 + align64(static_cast<size_t>(kNoAllocMaxBatch) * kMlpHid);
-constexpr size_t kScrH3 = kScrH2 + align64(static_cast<size_t>(kNoAllocMaxBatch) * kMlpHid);
-constexpr size_t kScrY = kScrH3 + align64(static_cast<size_t>(kNoAllocMaxBatch) * kMlpHid);
-constexpr size_t kScrdY = kScrY + align64(static_cast<size_t>(kNoAllocMaxBatch) * 3);
-constexpr size_t kScrdA = kScrdY + align64(static_cast<size_t>(kNoAllocMaxBatch) * 3);
-constexpr size_t kScrdB = kScrdA + align64(static_cast<size_t>(kNoAllocMaxBatch) * kMlpHid);
-constexpr size_t kScrPart = kScrdB + align64(static_cast<size_t>(kNoAllocMaxBatch) * kMlpHid);
-constexpr size_t kScrLoss = kScrPart + align64((kNoAllocMaxBatch + kTrainChunk - 1) / kTrainChunk * static_cast<size_t>(kMlpTrainable));
-constexpr size_t kScratchFloats = kScrLoss + 64;   // 8.6 MB
+constexpr size_t kScrLoss = static_cast<size_t>(train_groups(kNoAllocMaxBatch)) * kTrPart;
+constexpr size_t kScrImg = kScrLoss + 64;
+constexpr size_t kScratchFloats = kScrImg + (kTrImg + 1) / 2;   // 1.1 MB
 
 }  // namespace
 
@@ -232,7 +224,8 @@ struct rgl_gpu {
 	bool mlpShadeBlocksSet = false;
 	uint32_t mlpSegCap = 0;         // queue entries per segment
 	// training scratch
-	DevArray<float> tX, tT, tH1, tH2, tH3, tY, tdY, tdA, tdB, tPart, tLoss;
+	DevArray<float> tPart, tLoss;
+	DevArray<uint16_t> tImg;
 
 	// render target (GPU::Reset / Retile, rglv_gpu.cxx:50-87)
 	int W = 0, H = 0, tileW = 64, tileH = 64, tilesX = 0, tilesY = 0;
@@ -357,7 +350,8 @@ struct rgl_gpu {
 		tileDesc.release(); scanPart.release();
 		keys.release(); rec.release(); crec.release();
 		probeWant.release(); quadList.release();
-		for (auto* a : { &mlpQueue, &tX, &tT, &tH1, &tH2, &tH3, &tY, &tdY, &tdA, &tdB, &tPart, &tLoss }) a->release();
+		for (auto* a : { &mlpQueue, &tPart, &tLoss }) a->release();
+		tImg.release();
 		mlpImg.release(); fwdImg.release();
 		vpos.release(); vflags.release(); vvary.release(); trect.release(); tvert.release();
 		cvpos.release(); cvvary.release(); fcount.release(); frect.release(); dDraws.release(); dLite.release();
@@ -1215,62 +1209,34 @@ struct rgl_gpu {
 	static constexpr int kResetBlocks = 128;        // k_scatter blocks that reset the keys of multi-segment tiles
 
 	// ---- learned shading: one forward + backward pass over a batch ----
-	static void Gemm(hipStream_t ts, const float* A, const float* B, float* C, int M, int N, int K, int lda, int ldb, int ldc,
-	                 int tA, int tB, const float* bias, int relu, const float* mask, int ldm, int kChunk, int nz) {
-		GemmArgs g{ A, B, C, M, N, K, lda, ldb, ldc, tA, tB, bias, relu, mask, ldm, kChunk, kMlpTrainable };
-		k_gemm_bf16<<<dim3((N + 63) / 64, (M + 63) / 64, nz), 256, 0, ts>>>(g); }
-
-	// seed 0xffffffff: the first B samples in order.  lr > 0: Adam step on
-	// prm/opt; lr == 0: the summed gradient goes to gradOut.
 	// the training buffers of a batch of B samples, allocated on demand
 	int TrainBuffers(int B, TrainBufs& tb) {
 		hipError_t e;
-		const int nz = (B + static_cast<int>(kTrainChunk) - 1) / static_cast<int>(kTrainChunk);
-		for (auto* a : { &tX }) if ((e = a->ensure(static_cast<size_t>(B) * kMlpK1)) != hipSuccess) return hipfail(e, "hipMalloc training");
-		for (auto* a : { &tH1, &tH2, &tH3, &tdA, &tdB }) if ((e = a->ensure(static_cast<size_t>(B) * kMlpHid)) != hipSuccess) return hipfail(e, "hipMalloc training");
-		for (auto* a : { &tT, &tY, &tdY }) if ((e = a->ensure(static_cast<size_t>(B) * 3)) != hipSuccess) return hipfail(e, "hipMalloc training");
-		if ((e = tPart.ensure(static_cast<size_t>(nz) * kMlpTrainable)) != hipSuccess) return hipfail(e, "hipMalloc training");
+		if ((e = tPart.ensure(static_cast<size_t>(train_groups(B)) * kTrPart)) != hipSuccess) return hipfail(e, "hipMalloc training");
 		if ((e = tLoss.ensure(1)) != hipSuccess) return hipfail(e, "hipMalloc training");
-		tb = TrainBufs{ tX.p, tT.p, tH1.p, tH2.p, tH3.p, tY.p, tdY.p, tdA.p, tdB.p, tPart.p, tLoss.p };
+		if ((e = tImg.ensure(kTrImg)) != hipSuccess) return hipfail(e, "hipMalloc training");
+		tb = TrainBufs{ tPart.p, tLoss.p, tImg.p };
 		return 0; }
 
 	// the same buffers inside this device's `scratch` array (no allocation)
 	TrainBufs ScratchBuffers() const {
-		float* b = scratchDev;
-		return TrainBufs{ b + kScrX, b + kScrT, b + kScrH1, b + kScrH2, b + kScrH3, b + kScrY, b + kScrdY, b + kScrdA, b + kScrdB,
-		                  b + kScrPart, b + kScrLoss }; }
+		return TrainBufs{ scratchDev, scratchDev + kScrLoss, reinterpret_cast<uint16_t*>(scratchDev + kScrImg) }; }
+
+	// the weight image that the passes of one call start from
+	static void TrainImage(hipStream_t ts, const TrainBufs& tb, const float* prm) {
+		k_mlp_pack_train<<<(kMlpTrainable + 255) / 256, 256, 0, ts>>>(prm, tb.Img); }
 
 	// seed 0xffffffff: the first B samples in order.  lr > 0: Adam step on
 	// prm/opt; lr == 0: the summed gradient goes to gradOut.
 	int TrainPass(hipStream_t ts, const TrainBufs& tb, const float* samples, long long n, int B, float* prm, float* opt, float lr,
 	              float b1, float b2, int t, uint32_t seed, float* gradOut) {
 		hipError_t e;
-		const int kChunk = static_cast<int>(kTrainChunk);
-		const int nz = (B + kChunk - 1) / kChunk;
-		k_mlp_batch<<<(B + 255) / 256, 256, 0, ts>>>(samples, n, B, seed, static_cast<uint32_t>(t), prm, tb.X, tb.T);
-		// forward: H = relu(X W^T + b), Y = H3 W4^T + b4
-		Gemm(ts, tb.X, prm + kW1, tb.H1, B, kMlpHid, kMlpK1, kMlpK1, kMlpK1, kMlpHid, 0, 1, prm + kB1, 1, nullptr, 0, kMlpK1, 1);
-		Gemm(ts, tb.H1, prm + kW2, tb.H2, B, kMlpHid, kMlpHid, kMlpHid, kMlpHid, kMlpHid, 0, 1, prm + kB2, 1, nullptr, 0, kMlpHid, 1);
-		Gemm(ts, tb.H2, prm + kW3, tb.H3, B, kMlpHid, kMlpHid, kMlpHid, kMlpHid, kMlpHid, 0, 1, prm + kB3, 1, nullptr, 0, kMlpHid, 1);
-		Gemm(ts, tb.H3, prm + kW4, tb.Y, B, kMlpOut, kMlpHid, kMlpHid, kMlpHid, kMlpOut, 0, 1, prm + kB4, 0, nullptr, 0, kMlpHid, 1);
-		k_fill_u32<<<1, 64, 0, ts>>>(reinterpret_cast<uint32_t*>(tb.Loss), 1, 0u);
-		k_mlp_loss<<<(3 * B + 255) / 256, 256, 0, ts>>>(tb.Y, tb.T, B, tb.dY, tb.Loss);
-		// backward: weight gradients split over K = samples into nz partials
-		float* P = tb.Part;
-		Gemm(ts, tb.dY, tb.H3, P + kW4, kMlpOut, kMlpHid, B, kMlpOut, kMlpHid, kMlpHid, 1, 0, nullptr, 0, nullptr, 0, kChunk, nz);
-		k_mlp_colsum<<<nz, 64, 0, ts>>>(tb.dY, B, kMlpOut, kChunk, P + kB4, kMlpTrainable);
-		Gemm(ts, tb.dY, prm + kW4, tb.dA, B, kMlpHid, kMlpOut, kMlpOut, kMlpHid, kMlpHid, 0, 0, nullptr, 0, tb.H3, kMlpHid, kMlpOut, 1);
-		Gemm(ts, tb.dA, tb.H2, P + kW3, kMlpHid, kMlpHid, B, kMlpHid, kMlpHid, kMlpHid, 1, 0, nullptr, 0, nullptr, 0, kChunk, nz);
-		k_mlp_colsum<<<nz, 64, 0, ts>>>(tb.dA, B, kMlpHid, kChunk, P + kB3, kMlpTrainable);
-		Gemm(ts, tb.dA, prm + kW3, tb.dB, B, kMlpHid, kMlpHid, kMlpHid, kMlpHid, kMlpHid, 0, 0, nullptr, 0, tb.H2, kMlpHid, kMlpHid, 1);
-		Gemm(ts, tb.dB, tb.H1, P + kW2, kMlpHid, kMlpHid, B, kMlpHid, kMlpHid, kMlpHid, 1, 0, nullptr, 0, nullptr, 0, kChunk, nz);
-		k_mlp_colsum<<<nz, 64, 0, ts>>>(tb.dB, B, kMlpHid, kChunk, P + kB2, kMlpTrainable);
-		Gemm(ts, tb.dB, prm + kW2, tb.dA, B, kMlpHid, kMlpHid, kMlpHid, kMlpHid, kMlpHid, 0, 0, nullptr, 0, tb.H1, kMlpHid, kMlpHid, 1);
-		Gemm(ts, tb.dA, tb.X, P + kW1, kMlpHid, kMlpK1, B, kMlpHid, kMlpK1, kMlpK1, 1, 0, nullptr, 0, nullptr, 0, kChunk, nz);
-		k_mlp_colsum<<<nz, 64, 0, ts>>>(tb.dA, B, kMlpHid, kChunk, P + kB1, kMlpTrainable);
+		const int nz = train_groups(B);
+		k_mlp_pass<<<nz, kTrThreads, 0, ts>>>(samples, n, B, seed, static_cast<uint32_t>(t), prm,
+			reinterpret_cast<const uint4*>(tb.Img), tb.Part);
 		const float bc1 = 1.0F - std::pow(b1, static_cast<float>(t)), bc2 = 1.0F - std::pow(b2, static_cast<float>(t));
-		k_mlp_adam<<<(kMlpTrainable + 255) / 256, 256, 0, ts>>>(P, nz, prm, opt, opt ? opt + kMlpTrainable : nullptr,
-			lr, b1, b2, 1e-8F, bc1 > 0.0F ? bc1 : 1.0F, bc2 > 0.0F ? bc2 : 1.0F, gradOut);
+		k_mlp_update<<<kTrPart / 64, 64, 0, ts>>>(tb.Part, nz, prm, opt, opt ? opt + kMlpTrainable : nullptr,
+			lr, b1, b2, 1e-8F, bc1 > 0.0F ? bc1 : 1.0F, bc2 > 0.0F ? bc2 : 1.0F, gradOut, tb.Loss, tb.Img);
 		if ((e = hipGetLastError()) != hipSuccess) return hipfail(e, "training launch");
 		return 0; }
 
@@ -1672,6 +1638,7 @@ int rgl_mlp_gradient(rgl_gpu* g, const float* dev_samples, int n, float* dev_par
 	if (r != 0) return r;
 	TrainBufs tb;
 	if ((r = g->TrainBuffers(n, tb)) != 0) return r;
+	rgl_gpu::TrainImage(ms, tb, dev_params);
 	r = g->TrainPass(ms, tb, dev_samples, n, n, dev_params, nullptr, 0.0F, 0.9F, 0.999F, 1, 0xffffffffu, dev_grad);
 	if (r != 0) return r;
 	if ((r = g->AuxEnd(ms)) != 0) return r;
@@ -1693,6 +1660,7 @@ int rgl_mlp_train(rgl_gpu* g, const float* dev_samples, long long n, float* dev_
 	if (r != 0) return r;
 	TrainBufs tb;
 	if ((r = g->TrainBuffers(batch, tb)) != 0) return r;
+	rgl_gpu::TrainImage(ms, tb, dev_params);
 	for (int s = 0; s < steps; ++s) {
 		r = g->TrainPass(ms, tb, dev_samples, n, batch, dev_params, dev_opt, lr, 0.9F, 0.99F, step0 + s + 1,
 		                 seed == 0xffffffffu ? 0u : seed, nullptr);
@@ -1718,6 +1686,7 @@ int rgl_mlp_train_noalloc(rgl_gpu* g, const float* dev_samples, long long n, flo
 	int r = g->AuxBegin(ms);
 	if (r != 0) return r;
 	const TrainBufs tb = g->ScratchBuffers();
+	rgl_gpu::TrainImage(ms, tb, dev_params);
 	for (int s = 0; s < steps; ++s) {
 		r = g->TrainPass(ms, tb, dev_samples, n, batch, dev_params, dev_opt, lr, 0.9F, 0.99F, step0 + s + 1,
 		                 seed == 0xffffffffu ? 0u : seed, nullptr);

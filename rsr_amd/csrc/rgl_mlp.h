@@ -13,9 +13,9 @@
 // 64 per wave; the weights sit in LDS for the whole workgroup, and the
 // encoded inputs and layer activations stay in registers, in the lanes the
 // next product reads them from (the weight image's K columns are ordered
-// to match).  Training uses a generic bf16 MFMA
-// GEMM (operands rounded to bf16 when staged, FP32 accumulation) for the
-// forward and backward passes, split-K weight gradients and an Adam update.
+// to match).  Training runs a mini-batch forward and backward in one launch
+// (operands rounded to bf16 when staged in LDS, FP32 accumulation, partial
+// weight gradients per workgroup) and adds the partials up in the Adam update.
 // No part of this has a counterpart in the reference, whose shaders are
 // all analytic.
 #pragma once
@@ -141,20 +141,8 @@ __device__ inline void mlp_inputs(const ShadeInput& s, const float* norm, float 
 	x[9] = s.albedo[0]; x[10] = s.albedo[1]; x[11] = s.albedo[2];
 	x[12] = s.rough; }
 
-// frequency encoding, 9 values per input: x, then (sin, cos)(2^k pi x) for
-// k = 0..3 by the double-angle recurrence from sin(pi x), cos(pi x)
-__device__ inline float mlp_enc_value(const float x[kMlpFeat], int e) {
-	if (e >= kMlpEnc) return 0.0F;
-	const int i = e / 9, j = e - 9 * (e / 9);
-	const float xi = x[i];
-	if (j == 0) return xi;
-	float sn = __builtin_amdgcn_sinf(0.5F * xi), cs = __builtin_amdgcn_cosf(0.5F * xi);   // revolutions
-	const int kk = (j - 1) >> 1;
-	for (int q = 0; q < kk; ++q) { const float s2 = 2.0F * sn * cs, c2 = (cs - sn) * (cs + sn); sn = s2; cs = c2; }
-	return (j & 1) ? sn : cs; }
-
 // sin and cos of 2^k pi v, k = 0..3, by the double-angle recurrence from
-// sin(pi v), cos(pi v) (the operations of mlp_enc_value)
+// sin(pi v), cos(pi v)
 __device__ inline void enc_bands(float v, float sn[4], float cs[4]) {
 	sn[0] = __builtin_amdgcn_sinf(0.5F * v); cs[0] = __builtin_amdgcn_cosf(0.5F * v);   // revolutions
 #pragma unroll
@@ -656,131 +644,339 @@ __global__ __launch_bounds__(256) void k_mlp_samples(BatchDesc b, RasterArgs a, 
 // ---------------------------------------------------------------------------
 // training
 // ---------------------------------------------------------------------------
-// batch: encoded inputs X [B][128] (fp32) and targets T [B][3] for samples
-// chosen by hash (or in order when seed == 0xffffffff)
-__global__ void k_mlp_batch(const float* __restrict__ samples, long long n, int B, uint32_t seed, uint32_t step,
-                            const float* __restrict__ prm, float* __restrict__ X, float* __restrict__ T) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= B) return;
-	long long src;
-	if (seed == 0xffffffffu) src = i;
-	else src = static_cast<long long>(hash32(hash32(seed ^ (step * 0x9e3779b9u)) + static_cast<uint32_t>(i)) % static_cast<uint64_t>(n));
-	const float* r = samples + src * kMlpSample;
-	ShadeInput s;
-	s.n[0] = r[0]; s.n[1] = r[1]; s.n[2] = r[2]; s.v[0] = r[3]; s.v[1] = r[4]; s.v[2] = r[5];
-	s.p[0] = r[6]; s.p[1] = r[7]; s.p[2] = r[8]; s.albedo[0] = r[9]; s.albedo[1] = r[10]; s.albedo[2] = r[11];
-	s.rough = r[12];
-	float x[kMlpFeat];
-	mlp_inputs(s, prm + kNorm, x);
-	float* xo = X + static_cast<long long>(i) * kMlpK1;
-	for (int e = 0; e < kMlpK1; ++e) xo[e] = mlp_enc_value(x, e);
-	T[i * 3 + 0] = r[13]; T[i * 3 + 1] = r[14]; T[i * 3 + 2] = r[15]; }
+// A training call packs the weights into the image the pass keeps in LDS
+// (k_mlp_pack_train); each step is then two launches: k_mlp_pass runs a
+// mini-batch forward and backward and leaves partial sums of the gradient,
+// k_mlp_update adds them up, takes the Adam step and keeps the image.
+//
+// k_mlp_pass: a workgroup takes kTrChunk samples, kTrTile at a time, through
+// the whole network.  A layer is 64 wide, so a tile's activations, in both
+// orders the products read them (by sample and by unit), and the weights,
+// plain and transposed, fit the 160 KB of LDS; only the samples, the weight
+// image and the partial sums touch memory.  Every sum is taken in the order
+// of the plain split-K form (32 samples per MFMA step, 256 per partial,
+// partials and bias sums one after the other), so the result does not depend
+// on how the work is dealt out.  Bound: the nine short phases between
+// barriers of a tile (4.5 us), four tiles one after the other: 26 us, and a
+// step of 16384 samples 37 us.  As a launch per product (eleven 64 x 64-tile
+// products with every operand through memory), per column sum, loss, batch
+// and update a step took 448 us.  Partials of 64 samples spread over all CUs
+// took 31 us, but sum in another order, which Adam's early steps amplify.  In the backward
+// phases waves 0-3 hold the layer's gradient (all 64 samples of 16 units
+// each) while waves 4-7 take the weight gradients of the layer above.
+constexpr int kTrTile = 64;       // samples per tile
+constexpr int kTrChunk = 256;     // samples per workgroup, and per partial sum
+constexpr int kTrThreads = 512;
+constexpr int kTrPart = (kMlpTrainable + 1 + 63) / 64 * 64;   // floats of a partial: the gradient, then the squared error
+constexpr int kLdS = kTrTile + 8; // rows of 64 samples or units (padded as the weight image's rows are)
+constexpr int kLdY = 40;          // rows of the output layer's 3 values, padded to the MFMA K step
 
-// C = epilogue(op(A) op(B)) with op(A)(m,k) = transA ? A[k*lda+m] : A[m*lda+k]
-// and op(B)(k,n) = transB ? B[n*ldb+k] : B[k*ldb+n]; operands are rounded
-// to bf16 as they are staged in LDS, products accumulate in fp32.
-// blockIdx.z splits K into chunks of kChunk; chunk z writes C + z*zStride.
-struct GemmArgs {
-	const float* A; const float* B; float* C;
-	int M, N, K, lda, ldb, ldc, transA, transB;
-	const float* bias;     // + bias[n]
-	int relu;
-	const float* mask; int ldm;   // * (mask[m*ldm+n] > 0)
-	int kChunk; long long zStride;
-};
+// LDS offsets in uint16.  kTrRowB lies over kTrX (read by the first layer
+// only) and kTrDzB over kTrH3 (read by the output layer's gradient only).
+constexpr int kTrW1 = 0;                              // weights [out][in]
+constexpr int kTrW2 = kTrW1 + kMlpHid * kLd1;
+constexpr int kTrW3 = kTrW2 + kMlpHid * kLdS;
+constexpr int kTrW4 = kTrW3 + kMlpHid * kLdS;         // [16][kLdS], rows 3.. zero
+constexpr int kTrW2T = kTrW4 + 16 * kLdS;             // weights [in][out]
+constexpr int kTrW3T = kTrW2T + kMlpHid * kLdS;
+constexpr int kTrW4T = kTrW3T + kMlpHid * kLdS;       // [64][kLdY], columns 3.. zero
+constexpr int kTrImg = kTrW4T + kMlpHid * kLdY;       // the weight image ends here
+constexpr int kTrX = kTrImg;                          // X by sample [64][kLd1]
+constexpr int kTrRowB = kTrX;                         // activations by sample, second buffer [64][kLdS]
+constexpr int kTrXT = kTrX + kTrTile * kLd1;          // X by input [128][kLdS]
+constexpr int kTrH1 = kTrXT + kMlpK1 * kLdS;          // activations by unit [64][kLdS]
+constexpr int kTrH2 = kTrH1 + kMlpHid * kLdS;
+constexpr int kTrH3 = kTrH2 + kMlpHid * kLdS;
+constexpr int kTrDzB = kTrH3;                         // layer gradients by unit, second buffer
+constexpr int kTrDzA = kTrH3 + kMlpHid * kLdS;        // layer gradients by unit, first buffer [64][kLdS]
+constexpr int kTrRowA = kTrDzA + kMlpHid * kLdS;      // activations / gradients by sample, first buffer [64][kLdS]
+constexpr int kTrY = kTrRowA + kTrTile * kLdS;        // dY by sample [64][kLdY], columns 3.. zero
+constexpr int kTrYT = kTrY + kTrTile * kLdY;          // dY by output [16][kLdS], rows 3.. zero
+constexpr int kTrEnd = kTrYT + 16 * kLdS;
+static_assert(kTrImg % 8 == 0 && kTrEnd % 8 == 0, "16-byte copies");
 
-__global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
-	__shared__ __attribute__((aligned(16))) uint16_t As[64 * 40];
-	__shared__ __attribute__((aligned(16))) uint16_t Bs[64 * 40];
-	const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-	const int kb = blockIdx.z * g.kChunk, ke = min(g.K, kb + g.kChunk);
+__device__ inline uint16_t bf16_one(float v) { return static_cast<uint16_t>(bf16_pack(v, 0.0F)); }
+
+// the places of weight w (an index of the parameter block) in the image
+__device__ inline void train_image_put(uint16_t* img, int w, float v) {
+	const uint16_t h = bf16_one(v);
+	if (w < kB1) img[kTrW1 + (w >> 7) * kLd1 + (w & 127)] = h;
+	else if (w >= kW2 && w < kB2) {
+		const int i = w - kW2, o = i >> 6, k = i & 63;
+		img[kTrW2 + o * kLdS + k] = h; img[kTrW2T + k * kLdS + o] = h; }
+	else if (w >= kW3 && w < kB3) {
+		const int i = w - kW3, o = i >> 6, k = i & 63;
+		img[kTrW3 + o * kLdS + k] = h; img[kTrW3T + k * kLdS + o] = h; }
+	else if (w >= kW4 && w < kB4) {
+		const int i = w - kW4, o = i >> 6, k = i & 63;
+		img[kTrW4 + o * kLdS + k] = h; img[kTrW4T + k * kLdY + o] = h; }}
+
+// the image of the parameters, the padding of the output layer zeroed (the
+// other rows' padding is never read)
+__global__ __launch_bounds__(256) void k_mlp_pack_train(const float* __restrict__ prm, uint16_t* __restrict__ img) {
+	const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+	if (i < kMlpTrainable) train_image_put(img, i, prm[i]);
+	if (i < 13 * kMlpHid) img[kTrW4 + (kMlpOut + (i >> 6)) * kLdS + (i & 63)] = 0;
+	if (i < 29 * kMlpHid) img[kTrW4T + (i & 63) * kLdY + kMlpOut + (i >> 6)] = 0; }
+
+// acc[j] += A B_j^T over K = kK: 16 rows of A (this lane's at a, K values in
+// chunks of 32), and 16 rows of each of kN operands, bStep apart
+template <int kK, int kN>
+__device__ inline void tr_product(const uint16_t* a, const uint16_t* b, int bStep, f32x4_t (&acc)[kN]) {
+#pragma unroll
+	for (int c = 0; c < kK / 32; ++c) {
+		const bf16x8_t av = lds_bf16x8(a + 32 * c);
+#pragma unroll
+		for (int j = 0; j < kN; ++j) acc[j] = mfma_bf16(av, lds_bf16x8(b + j * bStep + 32 * c), acc[j]); }}
+
+// the same with kN A operands and one B
+template <int kK, int kN>
+__device__ inline void tr_product_rows(const uint16_t* a, int aStep, const uint16_t* b, f32x4_t (&acc)[kN]) {
+#pragma unroll
+	for (int c = 0; c < kK / 32; ++c) {
+		const bf16x8_t bv = lds_bf16x8(b + 32 * c);
+#pragma unroll
+		for (int i = 0; i < kN; ++i) acc[i] = mfma_bf16(lds_bf16x8(a + i * aStep + 32 * c), bv, acc[i]); }}
+
+// a value of a row of 16 lanes moved to the next row (3: to row 0)
+template <int kRow>
+__device__ inline float next_row(float v) {
+	const uint32_t u = f2u(v);
+	const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);   // rows 0 0 2 2, rows 1 1 3 3
+	if constexpr (kRow == 0 || kRow == 2) return u2f(s[0]);
+	const auto t = __builtin_amdgcn_permlane32_swap(s[1], s[1], false, false);   // rows 0 1 0 1, rows 2 3 2 3
+	if constexpr (kRow == 1) return u2f(t[0]);
+	return u2f(t[1]); }
+
+__global__ __launch_bounds__(kTrThreads) void k_mlp_pass(const float* __restrict__ samples, long long n, int B, uint32_t seed,
+		uint32_t step, const float* __restrict__ prm, const uint4* __restrict__ img, float* __restrict__ part) {
+	__shared__ __attribute__((aligned(16))) uint16_t L[kTrEnd];
+	__shared__ float sbias[3 * kMlpHid + 4];     // b1 b2 b3 b4
+	__shared__ float sT[3 * kTrTile];            // the tile's targets
+	__shared__ __attribute__((aligned(16))) float sDY[kMlpOut][kTrTile];   // dY in fp32
+	__shared__ uint8_t smask[3][4][64];          // waves 4-7's units above zero
+	__shared__ float sLoss[4];
 	const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, r16 = lane & 15, q = lane >> 4;
-	const int wm = (wv & 1) * 32, wn = (wv >> 1) * 32;
-	f32x4_t acc[2][2];
+	const int ug = (wv & 3) * 16, sh = (wv >> 2) * 32;   // the wave's units of a layer and (forward) its samples
+	// the tile's samples: chosen by hash, or in order when seed ==
+	// 0xffffffff; rows past the batch take its last sample and no gradient.
+	// A thread reads features wv and wv + 8 of sample `lane` (wave 6: its
+	// targets too), a tile ahead.
+	float fx[2], ft[kMlpOut];
+	auto fetch = [&](int t0) {
+		const int i = min(t0 + lane, B - 1);
+		const long long src = seed == 0xffffffffu ? i : static_cast<long long>(
+			hash32(hash32(seed ^ (step * 0x9e3779b9u)) + static_cast<uint32_t>(i)) % static_cast<uint64_t>(n));
+		const float* row = samples + src * kMlpSample;
+		fx[0] = row[wv];
+		fx[1] = wv + 8 < kMlpFeat ? row[wv + 8] : 0.0F;
+		if (wv == 6) for (int c = 0; c < kMlpOut; ++c) ft[c] = row[kMlpFeat + c]; };
+	const int s0 = static_cast<int>(blockIdx.x) * kTrChunk, s1 = min(s0 + kTrChunk, B);
+	fetch(s0);
+	for (int i = tid; i < kTrImg / 8; i += kTrThreads) reinterpret_cast<uint4*>(L)[i] = img[i];
+	for (int i = tid; i < 3 * kMlpHid + kMlpOut; i += kTrThreads)
+		sbias[i] = i < 3 * kMlpHid ? prm[kB1 + (i >> 6) * (kMlpHid + kMlpHid * kMlpHid) + (i & 63)] : prm[kB4 + i - 3 * kMlpHid];
+	// what is read and never written again
+	for (int i = tid; i < 16 * kMlpHid; i += kTrThreads) L[kTrYT + (i >> 6) * kLdS + (i & 63)] = 0;
+	for (int i = tid; i < kTrTile * 32; i += kTrThreads) L[kTrY + (i >> 5) * kLdY + (i & 31)] = 0;
+	for (int i = tid; i < (kMlpK1 - kMlpEnc) * kTrTile; i += kTrThreads) L[kTrXT + (kMlpEnc + (i >> 6)) * kLdS + (i & 63)] = 0;
+	const float n0 = prm[kNorm], n1 = prm[kNorm + 1], n2 = prm[kNorm + 2], ninv = prm[kNorm + 3];
+	const float dscale = 2.0F / (3.0F * static_cast<float>(B));
+	const f32x4_t zero = { 0.0F, 0.0F, 0.0F, 0.0F };
+	// waves 4-7: rows ug of the weight gradients (W4: its columns ug)
+	f32x4_t g1[8] = { zero, zero, zero, zero, zero, zero, zero, zero }, g2[4] = { zero, zero, zero, zero }, g3[4] = { zero, zero, zero, zero }, g4[1] = { zero };
+	// waves 0-3: bias gradients of units ug (lane row 0); wave 7: b4's (lanes 0..2)
+	float gb[3] = { 0.0F, 0.0F, 0.0F }, gb4 = 0.0F, loss = 0.0F;
+
+	// two 16-sample tiles of a hidden layer: relu(A W^T + b), stored by unit
+	// (T) and by sample (R); bit 4 i + r: sample sh + 16 i + 4 q + r above zero
+	auto forward = [&](const f32x4_t (&acc)[2], const float* bias, uint16_t* T, uint16_t* R) {
+		uint32_t m = 0;
+		const int u = ug + r16;
+		const float bu = bias[u];
 #pragma unroll
-	for (int i = 0; i < 2; ++i)
-#pragma unroll
-		for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{ 0.0F, 0.0F, 0.0F, 0.0F };
-	for (int k0 = kb; k0 < ke; k0 += 32) {
-		// stage 64 x 32 of op(A) and op(B) as [row][k] bf16
-#pragma unroll
-		for (int e = 0; e < 8; ++e) {
-			const int idx = e * 256 + tid;
-			int r, k;
-			if (g.transA) { k = idx >> 6; r = idx & 63; } else { r = idx >> 5; k = idx & 31; }
-			const int gm = m0 + r, gk = k0 + k;
-			float v = 0.0F;
-			if (gm < g.M && gk < ke) v = g.transA ? g.A[static_cast<long long>(gk) * g.lda + gm] : g.A[static_cast<long long>(gm) * g.lda + gk];
-			As[r * 40 + k] = bf16_bits(v); }
-#pragma unroll
-		for (int e = 0; e < 8; ++e) {
-			const int idx = e * 256 + tid;
-			int r, k;
-			if (g.transB) { r = idx >> 5; k = idx & 31; } else { k = idx >> 6; r = idx & 63; }
-			const int gn = n0 + r, gk = k0 + k;
-			float v = 0.0F;
-			if (gn < g.N && gk < ke) v = g.transB ? g.B[static_cast<long long>(gn) * g.ldb + gk] : g.B[static_cast<long long>(gk) * g.ldb + gn];
-			Bs[r * 40 + k] = bf16_bits(v); }
-		__syncthreads();
-		bf16x8_t a[2], b[2];
-#pragma unroll
-		for (int i = 0; i < 2; ++i) a[i] = lds_bf16x8(As + (wm + 16 * i + r16) * 40 + q * 8);
-#pragma unroll
-		for (int j = 0; j < 2; ++j) b[j] = lds_bf16x8(Bs + (wn + 16 * j + r16) * 40 + q * 8);
-#pragma unroll
-		for (int i = 0; i < 2; ++i)
-#pragma unroll
-			for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(a[i], b[j], acc[i][j]);
-		__syncthreads(); }
-	float* C = g.C + blockIdx.z * g.zStride;
-#pragma unroll
-	for (int i = 0; i < 2; ++i)
-#pragma unroll
-		for (int j = 0; j < 2; ++j)
+		for (int i = 0; i < 2; ++i) {
+			float v[4];
 #pragma unroll
 			for (int r = 0; r < 4; ++r) {
-				const int m = m0 + wm + 16 * i + 4 * q + r, n = n0 + wn + 16 * j + r16;
-				if (m >= g.M || n >= g.N) continue;
-				float v = acc[i][j][r];
-				if (g.bias) v += g.bias[n];
-				if (g.relu) v = v > 0.0F ? v : 0.0F;
-				if (g.mask && !(g.mask[static_cast<long long>(m) * g.ldm + n] > 0.0F)) v = 0.0F;
-				C[static_cast<long long>(m) * g.ldc + n] = v; }}
+				v[r] = acc[i][r] + bu;
+				const bool on = v[r] > 0.0F;
+				v[r] = on ? v[r] : 0.0F;
+				m |= (on ? 1u : 0u) << (4 * i + r); }
+			const uint32_t lo = bf16_pack(v[0], v[1]), hi = bf16_pack(v[2], v[3]);
+			const int s = sh + 16 * i + 4 * q;
+			*reinterpret_cast<uint2*>(T + u * kLdS + s) = make_uint2(lo, hi);
+			uint16_t* o = R + s * kLdS + u;
+			o[0] = static_cast<uint16_t>(lo); o[kLdS] = static_cast<uint16_t>(lo >> 16);
+			o[2 * kLdS] = static_cast<uint16_t>(hi); o[3 * kLdS] = static_cast<uint16_t>(hi >> 16); }
+		return m; };
+	// a layer's gradient (waves 0-3: all samples of units ug), zero where the
+	// unit was, kept in v and stored by unit and (R not null) by sample
+	auto backward = [&](const f32x4_t (&acc)[4], uint32_t m, f32x4_t (&v)[4], uint16_t* T, uint16_t* R) {
+		const int u = ug + r16;
+#pragma unroll
+		for (int i = 0; i < 4; ++i) {
+#pragma unroll
+			for (int r = 0; r < 4; ++r) v[i][r] = (m >> (4 * i + r)) & 1u ? acc[i][r] : 0.0F;
+			const uint32_t lo = bf16_pack(v[i][0], v[i][1]), hi = bf16_pack(v[i][2], v[i][3]);
+			const int s = 16 * i + 4 * q;
+			*reinterpret_cast<uint2*>(T + u * kLdS + s) = make_uint2(lo, hi);
+			if (R) {
+				uint16_t* o = R + s * kLdS + u;
+				o[0] = static_cast<uint16_t>(lo); o[kLdS] = static_cast<uint16_t>(lo >> 16);
+				o[2 * kLdS] = static_cast<uint16_t>(hi); o[3 * kLdS] = static_cast<uint16_t>(hi >> 16); }}};
 
-// dY = 2 (Y - T) / (3 B); loss partial sums of squared error
-__global__ void k_mlp_loss(const float* __restrict__ Y, const float* __restrict__ T, int B, float* __restrict__ dY,
-                           float* __restrict__ lossSum) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	float se = 0.0F;
-	if (i < 3 * B) {
-		const float d = Y[i] - T[i];
-		dY[i] = d * (2.0F / (3.0F * static_cast<float>(B)));
-		se = d * d; }
-	for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
-	if ((threadIdx.x & 63) == 0 && se != 0.0F) atomicAdd(lossSum, se); }
+	for (int t0 = s0; t0 < s1; t0 += kTrTile) {   // uniform
+		// frequency encoding: features wv and wv + 8 of sample `lane`
+#pragma unroll
+		for (int k = 0; k < 2; ++k) {
+			const int f = wv + 8 * k;
+			if (f >= kMlpFeat) break;   // uniform over the wave
+			float x = fx[k];
+			if (f >= 6 && f < 9) x = (x - (f == 6 ? n0 : f == 7 ? n1 : n2)) * ninv;
+			float sn[4], cs[4];
+			enc_bands(x, sn, cs);
+			const float v[9] = { x, sn[0], cs[0], sn[1], cs[1], sn[2], cs[2], sn[3], cs[3] };
+#pragma unroll
+			for (int j = 0; j < 9; ++j) {
+				const uint16_t h = bf16_one(v[j]);
+				L[kTrX + lane * kLd1 + 9 * f + j] = h;
+				L[kTrXT + (9 * f + j) * kLdS + lane] = h; }}
+		if (wv == 5) for (int k = kMlpEnc; k < kMlpK1; ++k) L[kTrX + lane * kLd1 + k] = 0;
+		if (wv == 6) for (int c = 0; c < kMlpOut; ++c) sT[3 * lane + c] = ft[c];
+		__syncthreads();
+		if (t0 + kTrTile < s1) fetch(t0 + kTrTile);
+		uint32_t m[3];
+		{
+			f32x4_t acc[2] = { zero, zero };
+			tr_product_rows<kMlpK1, 2>(L + kTrX + (sh + r16) * kLd1 + 8 * q, 16 * kLd1, L + kTrW1 + (ug + r16) * kLd1 + 8 * q, acc);
+			m[0] = forward(acc, sbias, L + kTrH1, L + kTrRowA);
+		}
+		__syncthreads();
+		{
+			f32x4_t acc[2] = { zero, zero };
+			tr_product_rows<kMlpHid, 2>(L + kTrRowA + (sh + r16) * kLdS + 8 * q, 16 * kLdS, L + kTrW2 + (ug + r16) * kLdS + 8 * q, acc);
+			m[1] = forward(acc, sbias + kMlpHid, L + kTrH2, L + kTrRowB);
+		}
+		__syncthreads();
+		{
+			f32x4_t acc[2] = { zero, zero };
+			tr_product_rows<kMlpHid, 2>(L + kTrRowB + (sh + r16) * kLdS + 8 * q, 16 * kLdS, L + kTrW3 + (ug + r16) * kLdS + 8 * q, acc);
+			m[2] = forward(acc, sbias + 2 * kMlpHid, L + kTrH3, L + kTrRowA);
+		}
+		if (wv >= 4)
+#pragma unroll
+			for (int l = 0; l < 3; ++l) smask[l][wv - 4][lane] = static_cast<uint8_t>(m[l]);
+		__syncthreads();
+		// outputs (lane columns r16 < 3) of 16 samples per wave, squared error
+		// and dY = 2 (Y - T) / (3 B)
+		if (wv < 4) {
+			f32x4_t acc[1] = { zero };
+			tr_product<kMlpHid, 1>(L + kTrRowA + (ug + r16) * kLdS + 8 * q, L + kTrW4 + r16 * kLdS + 8 * q, 0, acc);
+			if (r16 < kMlpOut) {
+				float dy[4];
+				const int s = ug + 4 * q;
+#pragma unroll
+				for (int r = 0; r < 4; ++r) {
+					const float d = (acc[0][r] + sbias[3 * kMlpHid + r16]) - sT[3 * (s + r) + r16];
+					const bool on = t0 + s + r < s1;
+					dy[r] = on ? d * dscale : 0.0F;
+					loss += on ? d * d : 0.0F;
+					sDY[r16][s + r] = dy[r];
+					L[kTrY + (s + r) * kLdY + r16] = bf16_one(dy[r]); }
+				*reinterpret_cast<uint2*>(L + kTrYT + r16 * kLdS + s) = make_uint2(bf16_pack(dy[0], dy[1]), bf16_pack(dy[2], dy[3])); }
+#pragma unroll
+			for (int l = 0; l < 3; ++l) m[l] |= static_cast<uint32_t>(smask[l][wv][lane]) << 8; }
+		__syncthreads();
+		f32x4_t d3[4], d2[4], d1[4];
+		if (wv < 4) {   // layer 3's gradient dY W4
+			f32x4_t acc[4] = { zero, zero, zero, zero };
+			tr_product_rows<32, 4>(L + kTrY + r16 * kLdY + 8 * q, 16 * kLdY, L + kTrW4T + (ug + r16) * kLdY + 8 * q, acc);
+			backward(acc, m[2], d3, L + kTrDzA, L + kTrRowA); }
+		else {          // W4's dY^T H3
+			tr_product<kTrTile, 1>(L + kTrYT + r16 * kLdS + 8 * q, L + kTrH3 + (ug + r16) * kLdS + 8 * q, 0, g4);
+			if (wv == 7 && lane < kMlpOut)
+#pragma unroll
+				for (int s = 0; s < kTrTile; s += 4) {
+					const float4 v = *reinterpret_cast<const float4*>(&sDY[lane][s]);
+					gb4 = (((gb4 + v.x) + v.y) + v.z) + v.w; }}
+		__syncthreads();
+		if (wv < 4) {
+			f32x4_t acc[4] = { zero, zero, zero, zero };
+			tr_product_rows<kMlpHid, 4>(L + kTrRowA + r16 * kLdS + 8 * q, 16 * kLdS, L + kTrW3T + (ug + r16) * kLdS + 8 * q, acc);
+			backward(acc, m[1], d2, L + kTrDzB, L + kTrRowB); }
+		else tr_product<kTrTile, 4>(L + kTrDzA + (ug + r16) * kLdS + 8 * q, L + kTrH2 + r16 * kLdS + 8 * q, 16 * kLdS, g3);
+		__syncthreads();
+		if (wv < 4) {
+			f32x4_t acc[4] = { zero, zero, zero, zero };
+			tr_product_rows<kMlpHid, 4>(L + kTrRowB + r16 * kLdS + 8 * q, 16 * kLdS, L + kTrW2T + (ug + r16) * kLdS + 8 * q, acc);
+			backward(acc, m[0], d1, L + kTrDzA, nullptr); }
+		else tr_product<kTrTile, 4>(L + kTrDzB + (ug + r16) * kLdS + 8 * q, L + kTrH1 + r16 * kLdS + 8 * q, 16 * kLdS, g2);
+		__syncthreads();
+		if (wv < 4) {
+			// bias gradients: a unit's 64 samples one after the other, lane row
+			// by lane row (the running sums are right in the row whose turn it is)
+			auto rows = [&](f32x4_t a, f32x4_t b, f32x4_t c, auto hop) {
+				gb[0] = hop((((gb[0] + a[0]) + a[1]) + a[2]) + a[3]);
+				gb[1] = hop((((gb[1] + b[0]) + b[1]) + b[2]) + b[3]);
+				gb[2] = hop((((gb[2] + c[0]) + c[1]) + c[2]) + c[3]); };
+#pragma unroll
+			for (int i = 0; i < 4; ++i) {
+				rows(d1[i], d2[i], d3[i], [](float v) { return next_row<0>(v); });
+				rows(d1[i], d2[i], d3[i], [](float v) { return next_row<1>(v); });
+				rows(d1[i], d2[i], d3[i], [](float v) { return next_row<2>(v); });
+				rows(d1[i], d2[i], d3[i], [](float v) { return next_row<3>(v); }); }}
+		else tr_product<kTrTile, 8>(L + kTrDzA + (ug + r16) * kLdS + 8 * q, L + kTrXT + r16 * kLdS + 8 * q, 16 * kLdS, g1);
+		__syncthreads(); }
 
-// column sums of dZ [rows][cols] over row chunks -> partial z of a bias gradient
-__global__ void k_mlp_colsum(const float* __restrict__ dZ, int rows, int cols, int rowChunk, float* __restrict__ out,
-                             long long zStride) {
-	const int c = threadIdx.x;
-	if (c >= cols) return;
-	const int r0 = blockIdx.x * rowChunk, r1 = min(rows, r0 + rowChunk);
-	float s = 0.0F;
-	for (int r = r0; r < r1; ++r) s += dZ[static_cast<long long>(r) * cols + c];
-	out[blockIdx.x * zStride + c] = s; }
+	// the partial sums: a gradient tile's lane holds rows 4 q .. 4 q + 3 of column r16
+	float* P = part + static_cast<long long>(blockIdx.x) * kTrPart;
+	if (wv >= 4) {
+		auto put = [&](float* w, int ld, int col, const f32x4_t& g) {
+#pragma unroll
+			for (int r = 0; r < 4; ++r) w[(ug + 4 * q + r) * ld + col + r16] = g[r]; };
+#pragma unroll
+		for (int j = 0; j < 8; ++j) put(P + kW1, kMlpK1, 16 * j, g1[j]);
+#pragma unroll
+		for (int j = 0; j < 4; ++j) { put(P + kW2, kMlpHid, 16 * j, g2[j]); put(P + kW3, kMlpHid, 16 * j, g3[j]); }
+		if (q == 0)
+#pragma unroll
+			for (int r = 0; r < kMlpOut; ++r) P[kW4 + r * kMlpHid + ug + r16] = g4[0][r];
+		if (wv == 7 && lane < kMlpOut) P[kB4 + lane] = gb4; }
+	else {
+		if (q == 0) { P[kB1 + ug + r16] = gb[0]; P[kB2 + ug + r16] = gb[1]; P[kB3 + ug + r16] = gb[2]; }
+		for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
+		if (lane == 0) sLoss[wv] = loss; }
+	__syncthreads();
+	if (tid == 0) P[kMlpTrainable] = (sLoss[0] + sLoss[1]) + (sLoss[2] + sLoss[3]); }
 
-// sums the split partials; Adam update when lr > 0, else writes the gradient
-__global__ void k_mlp_adam(const float* __restrict__ part, int nz, float* __restrict__ prm, float* __restrict__ mom,
+// adds up the nz partials of a parameter, one after the other (a thread's
+// loads are in flight together); Adam update of the parameter and its place
+// in the weight image, or the gradient when gradOut is set.  The word after
+// the gradient is the squared error.  One wave per workgroup, so that the
+// 16,771 parameters' loads come from all CUs.
+__global__ __launch_bounds__(64) void k_mlp_update(const float* __restrict__ part, int nz, float* __restrict__ prm, float* __restrict__ mom,
                            float* __restrict__ vel, float lr, float b1, float b2, float eps, float bc1, float bc2,
-                           float* __restrict__ gradOut) {
-	const int p = blockIdx.x * blockDim.x + threadIdx.x;
-	if (p >= kMlpTrainable) return;
-	float gsum = 0.0F;
-	for (int z = 0; z < nz; ++z) gsum += part[static_cast<long long>(z) * kMlpTrainable + p];
-	if (gradOut) { gradOut[p] = gsum; return; }
-	const float m = b1 * mom[p] + (1.0F - b1) * gsum;
-	const float v = b2 * vel[p] + (1.0F - b2) * gsum * gsum;
+                           float* __restrict__ gradOut, float* __restrict__ lossSum, uint16_t* __restrict__ img) {
+	const int p = static_cast<int>(blockIdx.x) * 64 + static_cast<int>(threadIdx.x);
+	if (p > kMlpTrainable) return;
+	const float* src = part + p;
+	float g = 0.0F;
+	int z = 0;
+	for (; z + 16 <= nz; z += 16) {
+		float v[16];
+#pragma unroll
+		for (int k = 0; k < 16; ++k) v[k] = src[static_cast<long long>(z + k) * kTrPart];
+#pragma unroll
+		for (int k = 0; k < 16; ++k) g += v[k]; }
+	for (; z < nz; ++z) g += src[static_cast<long long>(z) * kTrPart];
+	if (p == kMlpTrainable) { lossSum[0] = g; return; }
+	if (gradOut) { gradOut[p] = g; return; }
+	const float m = b1 * mom[p] + (1.0F - b1) * g;
+	const float v = b2 * vel[p] + (1.0F - b2) * g * g;
 	mom[p] = m; vel[p] = v;
-	prm[p] -= lr * (m / bc1) / (__builtin_sqrtf(v / bc2) + eps); }
+	const float w = prm[p] - lr * (m / bc1) / (__builtin_sqrtf(v / bc2) + eps);
+	prm[p] = w;
+	train_image_put(img, p, w); }
 
 }  // namespace rgl

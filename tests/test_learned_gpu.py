@@ -335,3 +335,18 @@ def test_learned_frame_graph_replay_matches_eager():
     gpu.set_learned_shading(None, 0.0)
     other.close()
     gpu.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 1000])
+def test_gradient_at_tile_edges(n):
+    # batches around the pass's 64-sample tiles and 256-sample partials
+    s, p = _samples(n, 3), _params(4)
+    gpu = rgl.GPU(0)
+    ds, dp = torch.from_numpy(s).to(DEV), torch.from_numpy(p).to(DEV)
+    g = torch.zeros(learned.TRAINABLE, dtype=torch.float32, device=DEV)
+    loss = gpu.mlp_gradient(ds.data_ptr(), n, dp.data_ptr(), g.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    ref_loss, want = learned.ref_gradient(s, p)
+    assert abs(loss - ref_loss) <= 1e-3 * ref_loss
+    for a, b in zip(learned.layers(g.cpu().numpy().astype(np.float64)), learned.layers(want)):
+        assert np.linalg.norm(a - b) < 2e-2 * max(np.linalg.norm(b), 1e-12)
+    gpu.close()

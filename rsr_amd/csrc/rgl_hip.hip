@@ -264,7 +264,8 @@ struct rgl_gpu {
 	std::vector<uint8_t> lastIo;
 	int nIo = 0, nIoTiles = 0, nIoBlocks = 0;
 	DevArray<uint32_t> order;
-	DevArray<int4> ioBoxes;         // the pixel rect of every 64 sorted records of an in-order tile
+	DevArray<unsigned long long> ioMasks;   // per region of an in-order tile, a bit per sorted record that can touch it
+	int ioRegions = 1;              // the most regions per tile of the batch's in-order frames
 	DevArray<unsigned long long> skeys0, skeys1;
 	int segPairs = kSegPairs;       // (triangle, tile) pairs per visibility work item
 	int splitQuads = kSplitQuads;   // quad work per quadrant from which visibility regions are halved
@@ -363,7 +364,7 @@ struct rgl_gpu {
 		dFrames.release();
 		if (hOps) (void)hipHostFree(hOps);
 		if (hIo) (void)hipHostFree(hIo);
-		dOps.release(); dIo.release(); order.release(); ioBoxes.release(); skeys0.release(); skeys1.release();
+		dOps.release(); dIo.release(); order.release(); ioMasks.release(); skeys0.release(); skeys1.release();
 		if (auxDone) (void)hipEventDestroy(auxDone);
 		if (graphExec) (void)hipGraphExecDestroy(graphExec);
 		if (capStream) (void)hipStreamDestroy(capStream);
@@ -737,13 +738,15 @@ struct rgl_gpu {
 			f.blocksX = (f.W + kResolveW - 1) / kResolveW;
 			tileBase += f.nTiles;
 			keyBase += static_cast<long long>(f.W) * f.H;
-			blockBase += f.blocksX * ((f.H + kResolveH - 1) / kResolveH); }
+			// frames drawn in order store their own pixels: no resolve blocks
+			if (!f.inOrder) blockBase += f.blocksX * ((f.H + kResolveH - 1) / kResolveH); }
 		if (n > 1) for (int i = 0; i < n; ++i)
 			if (!recs[i]->sampleReqs.empty()) return fail(RGL_E_UNSUPPORTED, "training samples are stored from single-frame runs");
 		// the in-order frames: one k_tile_order block per tile, one k_inorder
 		// block per kRegionDim x kRegionDim region of a tile
 		std::vector<IoFrame> io;
 		int ioTiles = 0, ioBlocks = 0;
+		ioRegions = 1;
 		for (int i = 0; i < n; ++i) {
 			if (!frames[i].inOrder) continue;
 			IoFrame e;
@@ -752,6 +755,7 @@ struct rgl_gpu {
 			e.regionsX = (frames[i].tileW + kRegionDim - 1) / kRegionDim;
 			e.regionsY = (frames[i].tileH + kRegionDim - 1) / kRegionDim;
 			io.push_back(e);
+			ioRegions = std::max(ioRegions, e.regionsX * e.regionsY);
 			ioTiles += frames[i].nTiles;
 			ioBlocks += frames[i].nTiles * e.regionsX * e.regionsY; }
 		BatchDesc b;
@@ -784,7 +788,8 @@ struct rgl_gpu {
 		if (!io.empty()) {
 			const size_t nl = static_cast<size_t>(listCap) + clistCap;
 			if ((e = Grow(order, nl)) != hipSuccess) return hipfail(e, "hipMalloc tile order");
-			if ((e = Grow(ioBoxes, nl)) != hipSuccess) return hipfail(e, "hipMalloc tile order rects");
+			if ((e = Grow(ioMasks, (nl / 64 + static_cast<size_t>(ioTiles) + 1) * static_cast<size_t>(ioRegions))) != hipSuccess)
+				return hipfail(e, "hipMalloc record masks");
 			if ((e = Grow(skeys0, nl)) != hipSuccess) return hipfail(e, "hipMalloc sort keys");
 			if ((e = Grow(skeys1, nl)) != hipSuccess) return hipfail(e, "hipMalloc sort keys"); }
 		if (!dOps.p) {
@@ -1012,7 +1017,7 @@ struct rgl_gpu {
 		const void* ptrs[] = { vpos.p, vflags.p, vvary.p, trect.p, tvert.p, tileCount.p, tileCursor.p, tileOff.p, clipq.p, clipqOf.p,
 		                       cvpos.p, cvvary.p, fcount.p, frect.p, clipHist.p, clipOff.p, clipCursor.p, itemTile.p, tileDesc.p, scanPart.p, tileCost.p,
 		                       keys.p, rec.p, crec.p, mlpImg.p, probeWant.p, quadList.p, mlpQueue.p, qCount.p, mlpParams,
-		                       dOps.p, dIo.p, order.p, ioBoxes.p, skeys0.p, skeys1.p };
+		                       dOps.p, dIo.p, order.p, ioMasks.p, skeys0.p, skeys1.p };
 		mix(ptrs, sizeof(ptrs));
 		const uint32_t caps[] = { listCap, clipCap, clistCap, mlpSegCap, static_cast<uint32_t>(items), learned ? 1u : 0u,
 		                          static_cast<uint32_t>(mlpShadeBlocks) };
@@ -1070,7 +1075,7 @@ struct rgl_gpu {
 		template <class P> void run() { launch<ProgramList<P>>(); }
 		template <class L> void launch() {
 			k_inorder<L><<<g.nIoBlocks, kIoThreads, lds, g.stream>>>(b, ra, g.dIo.p, g.nIo, b.frames, g.dOps.p, g.dDraws.p, g.dLite.p, g.tileDesc.p,
-				g.rec.p, g.crec.p, g.order.p, g.ioBoxes.p); }};
+				g.rec.p, g.crec.p, g.order.p, g.ioMasks.p, g.ioRegions); }};
 	struct ResolveLaunch {
 		rgl_gpu& g; const BatchDesc& b; const RasterArgs& ra; unsigned rblocks; const DrawLite* lite; const DrawDesc* dd;
 		template <class P> void run() {
@@ -1143,7 +1148,7 @@ struct rgl_gpu {
 			k_scatter<<<(fusedScan ? 1 : 0) + b.units + kClipScatterBlocks + kResetBlocks, kUnitThreads, b.unitWindow * sizeof(uint32_t),
 				stream>>>(b, dLite.p, sa); }
 		Mark(5);
-		if (b.nTiles > 0) {
+		if (nIo < b.nFrames) {
 			// one workgroup per work item, sized from the last completed frame;
 			// the kernel strides over any remainder
 			Dispatch(0, k_vis, dim3(std::min(items, 1 << 20)), dim3(kRasterThreads), 0, b, ra,
@@ -1153,8 +1158,8 @@ struct rgl_gpu {
 		// every tile region walks them (before k_resolve, whose first block
 		// publishes the frame's counters)
 		if (nIo > 0)
-			k_tile_order<<<nIoTiles, 256, 0, stream>>>(b, dIo.p, nIo, b.frames, tileDesc.p, rec.p, crec.p, order.p, skeys0.p, skeys1.p,
-				ioBoxes.p);
+			k_tile_order<<<nIoTiles, kSortThreads, 0, stream>>>(b, dIo.p, nIo, b.frames, tileDesc.p, rec.p, crec.p, order.p, skeys0.p,
+				skeys1.p, ioMasks.p, ioRegions);
 		// everything above writes this executor's buffers alone; what
 		// follows writes or samples the caller's, after the previous
 		// double-buffered frame has finished

@@ -9,17 +9,17 @@
 // more drawing).
 //
 //   k_tile_order  one workgroup per tile: the tile's (triangle, tile) setup
-//                 records, inline and clipped, sorted by submission slot (an
-//                 LDS bitonic sort; above kSortCap records, LDS-sorted runs
-//                 merged in global memory).
-//   k_inorder     one workgroup per 16 x 16-pixel region of a tile, one
-//                 thread per 2x2 quad: the quad's colour, depth and
-//                 primitive id stay in registers while the workgroup steps
-//                 through the tile's triangles (from LDS, 64 at a time) and
-//                 frame commands in slot order, applying
-//                 TriangleProgram::Render (rglv_gpu_impl.hxx:166-222) to the
-//                 quad: coverage, scissor, early or late depth test, depth
-//                 write, shading, alpha blend, masked colour store.
+//                 records, inline and clipped, sorted by submission slot, and
+//                 per region of the tile a bit per sorted record that can
+//                 touch it.
+//   k_inorder     one wave per 8 x 8-pixel region of a tile, one lane per
+//                 pixel: the pixel's colour, depth and primitive id stay in
+//                 registers while the wave steps through the region's
+//                 triangles (64 at a time) and the frame commands in slot
+//                 order, applying TriangleProgram::Render
+//                 (rglv_gpu_impl.hxx:166-222): coverage, scissor, early or
+//                 late depth test, depth write, shading, alpha blend, masked
+//                 colour store.
 #pragma once
 
 #include "rgl_kernels.h"
@@ -63,8 +63,11 @@ struct alignas(16) IoFrame {
 constexpr int kAttachColorDepth = 0, kAttachRGBF32 = 1;
 
 constexpr int kSortCap = 4096;       // records a tile sorts in LDS in one piece
-constexpr int kRegionDim = 16;       // k_inorder region: 16 x 16 pixels, 8 x 8 quads
-constexpr int kIoThreads = (kRegionDim / 2) * (kRegionDim / 2);   // one thread per quad of the region
+constexpr int kSortThreads = 1024;   // k_tile_order workgroup
+constexpr int kRegionDim = 8;        // k_inorder region: 8 x 8 pixels, a lane each; 4 x 4 quads
+constexpr int kRegionQuads = (kRegionDim / 2) * (kRegionDim / 2);
+constexpr int kIoThreads = kRegionDim * kRegionDim;
+static_assert(kIoThreads == 64, "a region is one wave, its record masks one word per 64 records");
 
 __device__ inline int find_io(const IoFrame* io, int n, int blk, bool tiles) {
 	int lo = 0, hi = n - 1;
@@ -73,96 +76,123 @@ __device__ inline int find_io(const IoFrame* io, int n, int blk, bool tiles) {
 		if ((tiles ? io[mid].tileStart : io[mid].blockStart) <= blk) lo = mid; else hi = mid - 1; }
 	return lo; }
 
-// ascending bitonic sort of m (a power of two) keys in LDS by the workgroup
-__device__ inline void bitonic_sort(unsigned long long* s, uint32_t m) {
-	for (uint32_t k = 2; k <= m; k <<= 1)
+// the wave's 64 keys, one per lane, in ascending order (a bitonic network)
+__device__ inline unsigned long long wave_sort(unsigned long long v) {
+	const uint32_t lane = threadIdx.x & 63;
+#pragma unroll
+	for (uint32_t k = 2; k <= 64; k <<= 1)
+#pragma unroll
 		for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-			for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) {
-				const uint32_t ixj = i ^ j;
-				if (ixj > i) {
-					const unsigned long long x = s[i], y = s[ixj];
-					if ((x > y) == ((i & k) == 0)) { s[i] = y; s[ixj] = x; }}}
-			__syncthreads(); }}
+			const unsigned long long o = __shfl_xor(v, static_cast<int>(j), 64);
+			const bool low = (lane & j) == 0, up = (lane & k) == 0;
+			if ((low == up) ? o < v : o > v) v = o; }
+	return v; }
 
-// The pixel rect of the quads of every kIoThreads consecutive records of a
-// tile's sorted list (one wave each): a k_inorder region skips the batches
-// whose rect misses it.  boxes[ob + k] holds the rect of records k ..
-// k + kIoThreads - 1 as (x0, y0, x1, y1), x1 and y1 exclusive.
-static_assert(kIoThreads == 64, "a batch's rect is one wave's reduction");
-__device__ inline void batch_boxes(uint32_t n, uint32_t ninl, const VisTile& d, uint32_t ob, const VisRec* __restrict__ rec,
-                                   const VisRec* __restrict__ crec, const uint32_t* __restrict__ order, int4* __restrict__ boxes) {
+// one merge pass over n distinct keys in sorted runs of `run`: each key's
+// place in its merged run of 2 run is its index in its own run plus its
+// rank (binary search) in the other
+__device__ inline void merge_runs(const unsigned long long* src, unsigned long long* dst, uint32_t n, uint32_t run) {
+	for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+		const uint32_t a0 = i & ~(2 * run - 1);
+		const uint32_t a1 = min(a0 + run, n), b1 = min(a0 + 2 * run, n);
+		const unsigned long long key = src[i];
+		const bool inA = i < a1;
+		uint32_t lo = inA ? a1 : a0, hi = inA ? b1 : a1;
+		const uint32_t own = inA ? i - a0 : i - a1, base = lo;
+		while (lo < hi) { const uint32_t mid = (lo + hi) >> 1; if (src[mid] < key) lo = mid + 1; else hi = mid; }
+		dst[a0 + own + (lo - base)] = key; }}
+
+// The word of a tile's record masks: masks[mask_word(...) + region * nb + k]
+// holds a bit per record 64 k .. 64 k + 63 of the tile's sorted list (nb =
+// ceil(n / 64) words per region) whose quads reach the region.  ob: the
+// tile's first position of order[], blk its index among the in-order tiles;
+// maxRegions: the most regions per tile of the batch's in-order frames.
+// Ranges of different tiles are disjoint.
+__device__ inline long long mask_word(uint32_t ob, int blk, int maxRegions) {
+	return (static_cast<long long>(ob >> 6) + blk) * maxRegions; }
+
+// a tile's record masks, one wave per 64 sorted records: a ballot per region
+__device__ inline void record_masks(uint32_t n, uint32_t ninl, const VisTile& d, uint32_t ob, const Rect& R, int regionsX, int regionsY,
+                                    const VisRec* __restrict__ rec, const VisRec* __restrict__ crec, const uint32_t* __restrict__ order,
+                                    unsigned long long* __restrict__ masks) {
 	__syncthreads();   // the workgroup's order[] stores
 	const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-	for (uint32_t k0 = wv * 64u; k0 < n; k0 += nw * 64u) {   // uniform over the wave
-		int x0 = 0x7fffffff, y0 = 0x7fffffff, x1 = -0x7fffffff, y1 = -0x7fffffff;
-		if (k0 + lane < n) {
-			const uint32_t p = order[ob + k0 + lane];
+	const uint32_t nb = (n + 63) >> 6;
+	for (uint32_t k = wv; k < nb; k += nw) {   // uniform over the wave
+		int gx0 = 1, gx1 = 0, gy0 = 1, gy1 = 0;   // the regions the record's quads reach (none)
+		if (64 * k + lane < n) {
+			const uint32_t p = order[ob + 64 * k + lane];
 			const VisRec& r = p < ninl ? rec[d.ib + p] : crec[d.cb + (p - ninl)];
-			const int minx = static_cast<int>(r.minxy & 0xffffu), miny = static_cast<int>(r.minxy >> 16);
-			x0 = minx; y0 = miny;
-			x1 = minx + 2 * static_cast<int>(r.nq & 0xffffu); y1 = miny + 2 * static_cast<int>(r.nq >> 16); }
-		for (int o = 32; o > 0; o >>= 1) {
-			x0 = min(x0, __shfl_xor(x0, o, 64)); y0 = min(y0, __shfl_xor(y0, o, 64));
-			x1 = max(x1, __shfl_xor(x1, o, 64)); y1 = max(y1, __shfl_xor(y1, o, 64)); }
-		if (lane == 0) boxes[ob + k0] = make_int4(x0, y0, x1, y1); }}
+			const uint2 v = *reinterpret_cast<const uint2*>(&r.minxy);   // minxy, nq
+			const int minx = static_cast<int>(v.x & 0xffffu) - R.x0, miny = static_cast<int>(v.x >> 16) - R.y0;
+			const int nqx = static_cast<int>(v.y & 0xffffu), nqy = static_cast<int>(v.y >> 16);
+			if (nqx > 0 && nqy > 0) {
+				gx0 = minx / kRegionDim; gx1 = (minx + 2 * nqx - 1) / kRegionDim;
+				gy0 = miny / kRegionDim; gy1 = (miny + 2 * nqy - 1) / kRegionDim; }}
+		unsigned long long mine = 0;
+		int reg = 0;
+		for (int gy = 0; gy < regionsY; ++gy)
+			for (int gx = 0; gx < regionsX; ++gx, ++reg) {
+				const unsigned long long m = __ballot(gx0 <= gx && gx <= gx1 && gy0 <= gy && gy <= gy1);
+				if ((reg & 63) == static_cast<int>(lane)) mine = m;
+				if ((reg & 63) == 63) masks[static_cast<long long>(reg - 63 + static_cast<int>(lane)) * nb + k] = mine; }
+		const int rest = reg & 63;
+		if (static_cast<int>(lane) < rest) masks[static_cast<long long>(reg - rest + static_cast<int>(lane)) * nb + k] = mine; }}
 
 // A tile's records in submission order.  Keys are (slot << 32 | p), p the
 // record's position in the tile (inline records first, then clipped); every
 // (triangle, tile) pair has its own slot, so keys are distinct.  order[ob +
 // k] receives the k-th record's p, ob = the tile's first inline + first
-// clipped list position (the tiles' ranges are disjoint).
-__global__ __launch_bounds__(256) void k_tile_order(BatchDesc b, const IoFrame* __restrict__ io, int nIo,
+// clipped list position (the tiles' ranges are disjoint).  Runs of 64 are
+// sorted in the lanes of a wave, then merged in LDS (up to kSortCap records,
+// and above that in global memory), each pass a binary search per key:
+// six passes of LDS latency for 4,096 records, where a bitonic network in
+// LDS took 78 passes and barriers (71 -> 31 us with tiles of up to 1,800).
+__global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, const IoFrame* __restrict__ io, int nIo,
 		const FrameDesc* __restrict__ frames, const VisTile* __restrict__ tileDesc, const VisRec* __restrict__ rec,
 		const VisRec* __restrict__ crec, uint32_t* __restrict__ order, unsigned long long* __restrict__ skeys0,
-		unsigned long long* __restrict__ skeys1, int4* __restrict__ boxes) {
-	__shared__ unsigned long long s[kSortCap];
+		unsigned long long* __restrict__ skeys1, unsigned long long* __restrict__ masks, int maxRegions) {
+	__shared__ unsigned long long s[2][kSortCap];
 	const int blk = static_cast<int>(blockIdx.x);
 	const IoFrame e = io[find_io(io, nIo, blk, true)];
 	const FrameDesc& f = frames[e.frame];
-	const int tile = f.tileBase + (blk - e.tileStart);
+	const int lt = blk - e.tileStart, tile = f.tileBase + lt;
+	const Rect R = tile_rect(f, lt);
 	const VisTile d = tileDesc[tile];
 	const uint32_t n = d.ntot, ninl = d.ninl, ob = d.ib + d.cb;
-	const uint32_t t = threadIdx.x;
+	const uint32_t t = threadIdx.x, lane = t & 63;
 	auto key_of = [&](uint32_t p) -> unsigned long long {
 		const uint32_t slot = p < ninl ? rec[d.ib + p].slot : crec[d.cb + (p - ninl)].slot;
 		return (static_cast<unsigned long long>(slot) << 32) | p; };
-	if (n <= static_cast<uint32_t>(kSortCap)) {
-		uint32_t m = 1;
-		while (m < n) m <<= 1;
-		for (uint32_t i = t; i < m; i += blockDim.x) s[i] = i < n ? key_of(i) : ~0ull;
+	// records c0 .. c0 + cn - 1 sorted in LDS; returns the buffer they end in
+	auto sort_lds = [&](uint32_t c0, uint32_t cn) {
+		for (uint32_t i0 = t & ~63u; i0 < cn; i0 += kSortThreads) {   // uniform over the wave
+			const unsigned long long v = wave_sort(i0 + lane < cn ? key_of(c0 + i0 + lane) : ~0ull);
+			if (i0 + lane < cn) s[0][i0 + lane] = v; }
 		__syncthreads();
-		bitonic_sort(s, m);
-		for (uint32_t i = t; i < n; i += blockDim.x) order[ob + i] = static_cast<uint32_t>(s[i]);
-		batch_boxes(n, ninl, d, ob, rec, crec, order, boxes);
+		int cur = 0;
+		for (uint32_t run = 64; run < cn; run <<= 1, cur ^= 1) { merge_runs(s[cur], s[cur ^ 1], cn, run); __syncthreads(); }
+		return cur; };
+	unsigned long long* const tm = masks + mask_word(ob, blk, maxRegions);
+	if (n <= static_cast<uint32_t>(kSortCap)) {
+		const unsigned long long* v = s[sort_lds(0, n)];
+		for (uint32_t i = t; i < n; i += kSortThreads) order[ob + i] = static_cast<uint32_t>(v[i]);
+		record_masks(n, ninl, d, ob, R, e.regionsX, e.regionsY, rec, crec, order, tm);
 		return; }
-	// runs of kSortCap sorted in LDS, then merged pairwise: each key's place
-	// in the merged run is its index in its own run plus its rank (binary
-	// search) in the other
 	unsigned long long* src = skeys0 + ob;
 	unsigned long long* dst = skeys1 + ob;
 	for (uint32_t c0 = 0; c0 < n; c0 += kSortCap) {
 		const uint32_t cn = min(static_cast<uint32_t>(kSortCap), n - c0);
 		__syncthreads();
-		for (uint32_t i = t; i < static_cast<uint32_t>(kSortCap); i += blockDim.x) s[i] = i < cn ? key_of(c0 + i) : ~0ull;
-		__syncthreads();
-		bitonic_sort(s, kSortCap);
-		for (uint32_t i = t; i < cn; i += blockDim.x) src[c0 + i] = s[i]; }
+		const unsigned long long* v = s[sort_lds(c0, cn)];
+		for (uint32_t i = t; i < cn; i += kSortThreads) src[c0 + i] = v[i]; }
 	__syncthreads();
 	for (uint32_t run = kSortCap; run < n; run <<= 1) {
-		for (uint32_t i = t; i < n; i += blockDim.x) {
-			const uint32_t a0 = i / (2 * run) * (2 * run);
-			const uint32_t a1 = min(a0 + run, n), b1 = min(a0 + 2 * run, n);
-			const unsigned long long key = src[i];
-			const bool inA = i < a1;
-			uint32_t lo = inA ? a1 : a0, hi = inA ? b1 : a1;
-			const uint32_t own = inA ? i - a0 : i - a1;
-			const uint32_t base = inA ? a1 : a0;
-			while (lo < hi) { const uint32_t mid = (lo + hi) >> 1; if (src[mid] < key) lo = mid + 1; else hi = mid; }
-			dst[a0 + own + (lo - base)] = key; }
+		merge_runs(src, dst, n, run);
 		__syncthreads();
 		unsigned long long* x = src; src = dst; dst = x; }
-	for (uint32_t i = t; i < n; i += blockDim.x) order[ob + i] = static_cast<uint32_t>(src[i]);
-	batch_boxes(n, ninl, d, ob, rec, crec, order, boxes); }
+	for (uint32_t i = t; i < n; i += kSortThreads) order[ob + i] = static_cast<uint32_t>(src[i]);
+	record_masks(n, ninl, d, ob, R, e.regionsX, e.regionsY, rec, crec, order, tm); }
 
 // ShadeFragment of program P for a quad at (qx, qy): perspective-correct BP
 // from BS and the vertices' 1/w (Render, rglv_gpu_impl.hxx:187-191),
@@ -206,6 +236,43 @@ struct ShadeQuad {
 __device__ inline bool depth_pass(int func, float frag, float dest) {
 	return func == 0 ? frag < dest : func == 1 ? frag <= dest : frag == dest; }
 
+// the k-th (from 0) set bit of m, which has more than k
+__device__ inline uint32_t select_bit(unsigned long long m, uint32_t k) {
+	uint32_t at = 0;
+	uint32_t w = static_cast<uint32_t>(m);
+	uint32_t c = static_cast<uint32_t>(__popc(w));
+	if (k >= c) { k -= c; at = 32; w = static_cast<uint32_t>(m >> 32); }
+#pragma unroll
+	for (uint32_t h = 16; h > 0; h >>= 1) {
+		c = static_cast<uint32_t>(__popc(w & ((1u << h) - 1u)));
+		if (k >= c) { k -= c; at += h; w >>= h; }}
+	return at; }
+
+// what the shading reads of a batch's triangle
+struct alignas(16) IoTri {
+	int32_t c1, c2, c3;
+	int32_t dx12, dy12, dx23, dy23, dx31, dy31;
+	uint32_t minxy;
+	float scale;
+	uint32_t slot;
+};
+static_assert(sizeof(IoTri) == 48, "three 16-byte rows");
+
+// A region's triangles come 64 at a time (the set bits of its record masks,
+// in order), and their (triangle, quad) pairs inside the region, at most 16
+// each, in windows of 64.  Shade: each lane takes one pair: coverage,
+// scissor, the program on the quad (programs have no side effects, so this
+// runs before the depth test); its bit goes into its quad's word.  Apply:
+// each lane walks the set bits of its pixel's quad, in slot order, with the
+// frame's commands between them.
+//
+// Bound: the chain of dependent fetches of a window (vertex ids, positions,
+// varyings, texels, about 3 us), times the windows of the heaviest region.
+// 8 x 8 regions of one wave each keep that chain short and need no barrier;
+// 16 x 16 regions, which walked all triangles of a batch per quad and all
+// batches of the tile, took 471 us on 327,680 blended triangles at
+// 1920x1080 where these take 219 us.
+//
 // L: the programs the draws may use (a frame of one program compiles only
 // that program's shading, which keeps the registers, and so the resident
 // waves that hide each triangle's texture fetches, of that program alone)
@@ -213,25 +280,25 @@ template <class L>
 __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs a, const IoFrame* __restrict__ io, int nIo,
 		const FrameDesc* __restrict__ frames, const FrameOp* __restrict__ ops, const DrawDesc* __restrict__ draws,
 		const DrawLite* __restrict__ lite, const VisTile* __restrict__ tileDesc, const VisRec* __restrict__ rec,
-		const VisRec* __restrict__ crec, const uint32_t* __restrict__ order, const int4* __restrict__ boxes) {
-	__shared__ VisRec srec[kIoThreads];
-	__shared__ int sdraw[kIoThreads];
-	__shared__ uint32_t sfrag[kIoThreads / 64];
-	// each batch triangle's source triangle (bit 31: a clipped fan)
-	__shared__ uint32_t ssrc[kIoThreads];
-	__shared__ uint32_t scan_sh[kIoThreads / 64 + 1];
-	// a window of kIoThreads (triangle, quad) pairs, shaded in parallel: the
-	// lanes' depths and colours, the live and kept lanes; qoff[j]: the first
-	// pair of batch triangle j
-	__shared__ float wfd[kIoThreads][4];
-	__shared__ float4 wcol[kIoThreads][4];
-	__shared__ uint32_t wmask[kIoThreads];
-	__shared__ uint32_t qoff[kIoThreads + 1];
-	// per batch triangle, for the ordered pass: its draw's fragment state
-	// (bit 0 depth test, 1 depth write, 2-3 depth function, 4 colour write,
-	// 5 blend, 6 early depth test), its primitive id, and its pair rect in
-	// the region (x0 | y0 << 16, cx | cy << 16)
-	__shared__ uint32_t sstate[kIoThreads], sprim[kIoThreads], sxy[kIoThreads], scxy[kIoThreads];
+		const VisRec* __restrict__ crec, const uint32_t* __restrict__ order, const unsigned long long* __restrict__ masks,
+		int maxRegions) {
+	// 64 words of the region's record masks and the set bits before each
+	__shared__ unsigned long long smask[64];
+	__shared__ uint32_t spre[65];
+	// the batch's triangles: setup; draw | fragment state << 16 (bit 0 depth
+	// test, 1 depth write, 2-3 depth function, 4 colour write, 5 blend, 6
+	// early depth test); source triangle (bit 31: a clipped fan); primitive
+	// id; pair rect in the region's quads (x0 | y0 << 4 | cx << 8)
+	__shared__ IoTri stri[64];
+	__shared__ uint32_t smeta[64], ssrc[64], sprim[64], srect[64], qoff[64];
+	// a window of pairs: its triangles, the lanes' depths and colours, the
+	// lanes (bits 0-3: live lanes the program keeps, 4-7: live lanes); per
+	// quad of the region the window's pairs with a live lane
+	__shared__ uint8_t wtri[64];
+	__shared__ uint8_t wmask[64];
+	__shared__ __attribute__((aligned(16))) float wfd[64][4];
+	__shared__ float4 wcol[64][4];
+	__shared__ unsigned long long qpairs[kRegionQuads];
 	const int vs = a.varyStride;
 	const int blk = static_cast<int>(blockIdx.x);
 	const IoFrame e = io[find_io(io, nIo, blk, false)];
@@ -242,19 +309,20 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	const int tile = f.tileBase + lt;
 	const Rect R = tile_rect(f, lt);
 	const int rgy = reg / e.regionsX, rgx = reg - rgy * e.regionsX;
+	const int rx0 = R.x0 + rgx * kRegionDim, ry0 = R.y0 + rgy * kRegionDim;
+	if (rx0 >= R.x1 || ry0 >= R.y1) return;   // beyond the target (uniform): no quad starts here
 	const int t = static_cast<int>(threadIdx.x);
-	// this thread's quad: top-left pixel (qx, qy); lane l = (l & 1, l >> 1)
-	const int qx = R.x0 + rgx * kRegionDim + 2 * (t % (kRegionDim / 2));
-	const int qy = R.y0 + rgy * kRegionDim + 2 * (t / (kRegionDim / 2));
-	bool onScreen[4];
-#pragma unroll
-	for (int l = 0; l < 4; ++l) onScreen[l] = qx + (l & 1) < R.x1 && qy + (l >> 1) < R.y1;
+	// this lane's pixel: lane l = (l & 1, l >> 1) of quad `quad` at (qx, qy)
+	const int l = t & 3, quad = t >> 2;
+	const int qx = rx0 + 2 * (quad & 3), qy = ry0 + 2 * (quad >> 2);
+	const int x = qx + (l & 1), y = qy + (l >> 1);
+	const bool onScreen = x < R.x1 && y < R.y1;
+	const bool quadOnScreen = qx < R.x1 && qy < R.y1;
 	// the tile buffers start zeroed (the oracle's convention for a tile not
 	// yet cleared; the reference leaves the previous tile's contents)
-	float cr[4] = { 0.0F, 0.0F, 0.0F, 0.0F }, cg[4] = { 0.0F, 0.0F, 0.0F, 0.0F }, cb[4] = { 0.0F, 0.0F, 0.0F, 0.0F };
-	float dz[4] = { 0.0F, 0.0F, 0.0F, 0.0F };
-	float ca[4] = { 0.0F, 0.0F, 0.0F, 0.0F };   // RB_RGBAF32's alpha: set by clears, never drawn
-	uint32_t pid[4] = { 0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu };
+	float cr = 0.0F, cg = 0.0F, cb = 0.0F, dz = 0.0F;
+	float ca = 0.0F;   // RB_RGBAF32's alpha: set by clears, never drawn
+	uint32_t pid = 0xffffffffu;
 	uint32_t frags = 0;
 	const VisTile vt = tileDesc[tile];
 	const uint32_t n = vt.ntot, ninl = vt.ninl, ob = vt.ib + vt.cb;
@@ -262,130 +330,110 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	const uint32_t ope = static_cast<uint32_t>(f.opBase + f.nOps);
 	uint32_t nextOp = opi < ope ? ops[opi].pos : 0xffffffffu;   // the position of the next frame command
 
+	// the four lanes of a quad run it together
 	auto apply_op = [&](const FrameOp& op) {
 		if (op.kind == kOpClear) {
-			if (op.bits & 1) {
-#pragma unroll
-				for (int l = 0; l < 4; ++l) {
-					cr[l] = op.color[0]; cg[l] = op.color[1]; cb[l] = op.color[2]; ca[l] = op.color[3]; pid[l] = 0xffffffffu; }}
-			if (op.bits & 2) {
-#pragma unroll
-				for (int l = 0; l < 4; ++l) dz[l] = op.depth; }}
-		else if (op.kind == kOpStoreColorHalf || op.kind == kOpStoreColorQuads) {
-			// one output per quad whose top-left pixel lies in the tile
-			// rect (the reference's loops step 2 x 2 over the rect)
-			if (!onScreen[0]) return;
-			const long long q = static_cast<long long>(qy >> 1) * op.stride + (qx >> 1);
-			if (op.kind == kOpStoreColorHalf) {
-				// Downsample (rglr_algorithm.cxx:118-165): the transposed
-				// quad's pixels summed in lane order, times 1/4; alpha 0
-				const float z = ((0.0F + 0.0F) + 0.0F) + 0.0F;
-				static_cast<float4*>(op.ptr)[q] = make_float4((((cr[0] + cr[1]) + cr[2]) + cr[3]) * 0.25F,
-				                                              (((cg[0] + cg[1]) + cg[2]) + cg[3]) * 0.25F,
-				                                              (((cb[0] + cb[1]) + cb[2]) + cb[3]) * 0.25F, z * 0.25F); }
-			else {
-				// Copy to a QFloat4Canvas (rglr_algorithm.cxx:320-368): alpha 1
-				// from RB_RGBF32, the fourth channel (RB_COLOR_DEPTH: the depth)
-				// otherwise
-				float4* o = static_cast<float4*>(op.ptr) + 4 * q;
-				float a[4];
-#pragma unroll
-				for (int l = 0; l < 4; ++l) a[l] = op.attach == kAttachRGBF32 ? 1.0F : op.attach == kAttachColorDepth ? dz[l] : ca[l];
-				o[0] = make_float4(cr[0], cr[1], cr[2], cr[3]);
-				o[1] = make_float4(cg[0], cg[1], cg[2], cg[3]);
-				o[2] = make_float4(cb[0], cb[1], cb[2], cb[3]);
-				o[3] = make_float4(a[0], a[1], a[2], a[3]); }}
+			if (op.bits & 1) { cr = op.color[0]; cg = op.color[1]; cb = op.color[2]; ca = op.color[3]; pid = 0xffffffffu; }
+			if (op.bits & 2) dz = op.depth; }
+		else if (op.kind == kOpStoreColorHalf) {
+			// Downsample (rglr_algorithm.cxx:118-165): one output per quad whose
+			// top-left pixel lies in the tile rect (the reference's loops step
+			// 2 x 2 over the rect), the transposed quad's pixels summed in lane
+			// order, times 1/4; alpha 0
+			auto mean = [&](float v) {
+				const float v1 = __shfl(v, (t & ~3) + 1, 64), v2 = __shfl(v, (t & ~3) + 2, 64), v3 = __shfl(v, (t & ~3) + 3, 64);
+				return (((v + v1) + v2) + v3) * 0.25F; };
+			const float r = mean(cr), g = mean(cg), bl = mean(cb);
+			const float z = ((0.0F + 0.0F) + 0.0F) + 0.0F;
+			if (quadOnScreen && l == 0)
+				static_cast<float4*>(op.ptr)[static_cast<long long>(qy >> 1) * op.stride + (qx >> 1)] = make_float4(r, g, bl, z * 0.25F); }
+		else if (op.kind == kOpStoreColorQuads) {
+			// Copy to a QFloat4Canvas (rglr_algorithm.cxx:320-368): alpha 1
+			// from RB_RGBF32, the fourth channel (RB_COLOR_DEPTH: the depth)
+			// otherwise
+			if (!quadOnScreen) return;
+			float* o = static_cast<float*>(op.ptr) + 16 * (static_cast<long long>(qy >> 1) * op.stride + (qx >> 1)) + l;
+			o[0] = cr; o[4] = cg; o[8] = cb;
+			o[12] = op.attach == kAttachRGBF32 ? 1.0F : op.attach == kAttachColorDepth ? dz : ca; }
 		else {
-#pragma unroll
-			for (int l = 0; l < 4; ++l) {
-				if (!onScreen[l]) continue;
-				const long long o = static_cast<long long>(qy + (l >> 1)) * f.W + qx + (l & 1);
-				if (op.kind == kOpStoreColor) {
-					float c[3] = { cr[l], cg[l], cb[l] };
-					if (op.post != 1)
-						post_shade(op.post, op.exposure, c, f.W, f.H, R.x0, R.y0, qx + (l & 1), qy + (l >> 1));
-					const uint32_t px = op.gamma
-						? ((to_srgb8(c[0]) << 16) | (to_srgb8(c[1]) << 8) | to_srgb8(c[2]))
-						: ((to_linear8(c[0]) << 16) | (to_linear8(c[1]) << 8) | to_linear8(c[2]));
-					static_cast<uint32_t*>(op.ptr)[o] = px; }
-				else if (op.kind == kOpStoreDepth) static_cast<float*>(op.ptr)[o] = dz[l];
-				else if (op.kind == kOpStoreColorFP)   // Copy to a FloatingPointCanvas (rglr_algorithm.cxx:194-280): alpha 0
-					static_cast<float4*>(op.ptr)[static_cast<long long>(qy + (l >> 1)) * op.stride + qx + (l & 1)] =
-						make_float4(cr[l], cg[l], cb[l], 0.0F);
-				else static_cast<uint32_t*>(op.ptr)[o] = pid[l]; }}};
+			if (!onScreen) return;
+			const long long o = static_cast<long long>(y) * f.W + x;
+			if (op.kind == kOpStoreColor) {
+				float c[3] = { cr, cg, cb };
+				if (op.post != 1) post_shade(op.post, op.exposure, c, f.W, f.H, R.x0, R.y0, x, y);
+				const uint32_t px = op.gamma
+					? ((to_srgb8(c[0]) << 16) | (to_srgb8(c[1]) << 8) | to_srgb8(c[2]))
+					: ((to_linear8(c[0]) << 16) | (to_linear8(c[1]) << 8) | to_linear8(c[2]));
+				static_cast<uint32_t*>(op.ptr)[o] = px; }
+			else if (op.kind == kOpStoreDepth) static_cast<float*>(op.ptr)[o] = dz;
+			else if (op.kind == kOpStoreColorFP)   // Copy to a FloatingPointCanvas (rglr_algorithm.cxx:194-280): alpha 0
+				static_cast<float4*>(op.ptr)[static_cast<long long>(y) * op.stride + x] = make_float4(cr, cg, cb, 0.0F);
+			else static_cast<uint32_t*>(op.ptr)[o] = pid; }};
 
-	// the region's pixel rect: records whose quads miss it are dropped when
-	// a batch is loaded (the rest keep their order), so the workgroup steps
-	// only through the triangles that can touch its pixels
-	const int rx0 = R.x0 + rgx * kRegionDim, ry0 = R.y0 + rgy * kRegionDim;
-	const int rx1 = min(rx0 + kRegionDim, R.x1), ry1 = min(ry0 + kRegionDim, R.y1);
-	for (uint32_t base = 0; base < n; base += kIoThreads) {
-		// a batch whose records' quads all miss the region (uniform)
-		const int4 bb = boxes[ob + base];
-		if (bb.x >= rx1 || bb.z <= rx0 || bb.y >= ry1 || bb.w <= ry0) continue;
+	const uint32_t nb = (n + 63) >> 6;   // words of the region's record masks
+	const unsigned long long* rm = masks + mask_word(ob, e.tileStart + lt, maxRegions) + static_cast<long long>(reg) * nb;
+	if (t < kRegionQuads) qpairs[t] = 0;
+	for (uint32_t k0 = 0; k0 < nb; k0 += 64) {   // 64 words, 4,096 records, at a time
+		const unsigned long long mw = k0 + t < nb ? rm[k0 + t] : 0ull;
+		uint32_t hits = static_cast<uint32_t>(__popcll(mw));
+		for (int o = 1; o < 64; o <<= 1) {
+			const uint32_t v = __shfl_up(hits, o, 64);
+			if (t >= o) hits += v; }
+		const uint32_t nh = __shfl(hits, 63, 64);
+		if (nh == 0) continue;   // uniform
 		__syncthreads();
-		VisRec rr;
-		bool hit = false;
-		if (base + static_cast<uint32_t>(t) < n) {
-			const uint32_t p = order[ob + base + t];
-			rr = p < ninl ? rec[vt.ib + p] : crec[vt.cb + (p - ninl)];
-			const int minx = static_cast<int>(rr.minxy & 0xffffu), miny = static_cast<int>(rr.minxy >> 16);
-			const int nqx = static_cast<int>(rr.nq & 0xffffu), nqy = static_cast<int>(rr.nq >> 16);
-			hit = minx < rx1 && minx + 2 * nqx > rx0 && miny < ry1 && miny + 2 * nqy > ry0; }
-		uint32_t cnt;
-		const uint32_t at = block_exclusive_scan(hit ? 1u : 0u, scan_sh, cnt);
-		if (hit) {
-			const uint32_t t2 = at;   // the record's place among the batch's hits
-			srec[t2] = rr;
-			const int di = find_draw_slot(lite, b.nDraws, rr.slot);
-			sdraw[t2] = di;
-			const DrawLite& dl = lite[di];
-			const uint32_t rel = rr.slot - dl.slotBase;
-			const uint32_t nTri = static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
-			const uint32_t srcTri = rel < nTri ? rel : (rel - nTri) / kFanMax;
-			ssrc[t2] = srcTri | (rel < nTri ? 0u : 0x80000000u);
-			const DrawDesc& dd = draws[di];
-			sstate[t2] = (dd.depthTest ? 1u : 0u) | (dd.depthWrite ? 2u : 0u) | (static_cast<uint32_t>(dd.depthFunc) << 2) |
-			             (dd.colorWrite ? 16u : 0u) | (dd.blend ? 32u : 0u) | (program_info(dd.program).earlyZ ? 64u : 0u);
-			sprim[t2] = dl.primBase + srcTri; }
+		smask[t] = mw;
+		spre[t + 1] = hits;
+		if (t == 0) spre[0] = 0;
 		__syncthreads();
-		// the batch's (triangle, quad) pairs inside the region, triangle by
-		// triangle in order: triangle j's quads of its quad rect that lie in
-		// the region's quads (both grids step 2 from even origins)
-		auto pair_rect = [&](int j, int& x0, int& y0, int& cx, int& cy) {
-			const int minx = static_cast<int>(srec[j].minxy & 0xffffu), miny = static_cast<int>(srec[j].minxy >> 16);
-			const int nqx = static_cast<int>(srec[j].nq & 0xffffu), nqy = static_cast<int>(srec[j].nq >> 16);
-			x0 = max(minx, rx0); y0 = max(miny, ry0);
-			const int x1 = min(minx + 2 * nqx, rx0 + kRegionDim), y1 = min(miny + 2 * nqy, ry0 + kRegionDim);
-			cx = x1 > x0 ? (x1 - x0 + 1) >> 1 : 0;
-			cy = y1 > y0 ? (y1 - y0 + 1) >> 1 : 0; };
-		uint32_t np = 0;
-		if (static_cast<uint32_t>(t) < cnt) {
-			int x0, y0, cx, cy;
-			pair_rect(t, x0, y0, cx, cy);
-			np = static_cast<uint32_t>(cx * cy);
-			sxy[t] = static_cast<uint32_t>(x0) | (static_cast<uint32_t>(y0) << 16);
-			scxy[t] = static_cast<uint32_t>(cx) | (static_cast<uint32_t>(cy) << 16); }
-		uint32_t total;
-		const uint32_t poff = block_exclusive_scan(np, scan_sh, total);
-		if (static_cast<uint32_t>(t) < cnt) qoff[t] = poff;
-		if (t == 0) qoff[cnt] = total;
-		__syncthreads();
-		for (uint32_t w0 = 0; w0 < total; w0 += kIoThreads) {
-			// shade: thread t takes pair w0 + t (coverage, scissor, the
-			// program), in parallel over the window
-			{
-				const uint32_t p = w0 + static_cast<uint32_t>(t);
-				uint32_t pm = 0;   // bits 0-3: live lanes the program keeps, bits 4-7: live lanes
-				if (p < total) {
-					int lo = 0, hi = static_cast<int>(cnt) - 1;   // the last triangle whose pairs start at or before p
-					while (lo < hi) { const int mid = (lo + hi + 1) >> 1; if (qoff[mid] <= p) lo = mid; else hi = mid - 1; }
-					const int j = lo;
-					int x0, y0, cx, cy;
-					pair_rect(j, x0, y0, cx, cy);
-					const int k = static_cast<int>(p - qoff[j]), iy = k / cx, ix = k - iy * cx;
-					const int px = x0 + 2 * ix, py = y0 + 2 * iy;
-					const VisRec& r = srec[j];
+		for (uint32_t h0 = 0; h0 < nh; h0 += 64) {
+			// the batch: lane t takes the region's (h0 + t)-th record of these
+			const uint32_t cnt = min(64u, nh - h0);
+			uint32_t np = 0;
+			if (static_cast<uint32_t>(t) < cnt) {
+				const uint32_t h = h0 + static_cast<uint32_t>(t);
+				uint32_t lo = 0;   // the word with spre[lo] <= h < spre[lo + 1]
+#pragma unroll
+				for (uint32_t st = 32; st > 0; st >>= 1) if (spre[lo + st] <= h) lo += st;
+				const uint32_t p = order[ob + 64 * (k0 + lo) + select_bit(smask[lo], h - spre[lo])];
+				const VisRec rr = p < ninl ? rec[vt.ib + p] : crec[vt.cb + (p - ninl)];
+				stri[t] = IoTri{ rr.c1, rr.c2, rr.c3, rr.dx12, rr.dy12, rr.dx23, rr.dy23, rr.dx31, rr.dy31, rr.minxy, rr.scale, rr.slot };
+				const int di = find_draw_slot(lite, b.nDraws, rr.slot);
+				const DrawLite& dl = lite[di];
+				const uint32_t rel = rr.slot - dl.slotBase;
+				const uint32_t nTri = static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
+				const uint32_t srcTri = rel < nTri ? rel : (rel - nTri) / kFanMax;
+				ssrc[t] = srcTri | (rel < nTri ? 0u : 0x80000000u);
+				const DrawDesc& dd = draws[di];
+				smeta[t] = static_cast<uint32_t>(di) |
+				           ((dd.depthTest ? 1u : 0u) | (dd.depthWrite ? 2u : 0u) | (static_cast<uint32_t>(dd.depthFunc) << 2) |
+				            (dd.colorWrite ? 16u : 0u) | (dd.blend ? 32u : 0u) | (program_info(dd.program).earlyZ ? 64u : 0u)) << 16;
+				sprim[t] = dl.primBase + srcTri;
+				// its quads among the region's (both grids step 2 from even origins)
+				const int minx = static_cast<int>(rr.minxy & 0xffffu), miny = static_cast<int>(rr.minxy >> 16);
+				const int x0 = max(minx - rx0, 0) >> 1, y0 = max(miny - ry0, 0) >> 1;
+				const int x1 = min((minx - rx0) / 2 + static_cast<int>(rr.nq & 0xffffu), kRegionDim / 2);
+				const int y1 = min((miny - ry0) / 2 + static_cast<int>(rr.nq >> 16), kRegionDim / 2);
+				np = static_cast<uint32_t>((x1 - x0) * (y1 - y0));
+				srect[t] = static_cast<uint32_t>(x0) | (static_cast<uint32_t>(y0) << 4) | (static_cast<uint32_t>(x1 - x0) << 8); }
+			uint32_t pend = np;   // pairs up to and with this lane's triangle
+			for (int o = 1; o < 64; o <<= 1) {
+				const uint32_t v = __shfl_up(pend, o, 64);
+				if (t >= o) pend += v; }
+			const uint32_t total = __shfl(pend, 63, 64), pbeg = pend - np;
+			qoff[t] = pbeg;
+			for (uint32_t w0 = 0; w0 < total; w0 += 64) {
+				// the window's pairs name their triangles
+				for (uint32_t p = max(pbeg, w0), pe = min(pend, w0 + 64u); p < pe; ++p) wtri[p - w0] = static_cast<uint8_t>(t);
+				__syncthreads();
+				// shade: lane t takes pair w0 + t (coverage, scissor, the program)
+				if (w0 + static_cast<uint32_t>(t) < total) {
+					const int j = wtri[t];
+					const uint32_t k = w0 + static_cast<uint32_t>(t) - qoff[j], rc = srect[j], cx = rc >> 8;
+					const uint32_t iy = (k * (cx == 3u ? 22u : 64u >> (cx >> 1))) >> 6;   // k / cx for k < 16, cx <= 4
+					const uint32_t wx = (rc & 15u) + k - iy * cx, wy = ((rc >> 4) & 15u) + iy;
+					const int px = rx0 + 2 * static_cast<int>(wx), py = ry0 + 2 * static_cast<int>(wy);
+					const IoTri r = stri[j];
 					const int kx = (px - static_cast<int>(r.minxy & 0xffffu)) >> 1, ky = (py - static_cast<int>(r.minxy >> 16)) >> 1;
 					// the quad's lanes (c, c+dy, c+dx, c+dx+dy), stepped as the
 					// rasteriser loops step (rglv_triangle.hxx:253-304)
@@ -397,8 +445,8 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 					const int32_t e3[4] = { q3, wadd(q3, r.dy31), wadd(q3, r.dx31), wadd(wadd(q3, r.dx31), r.dy31) };
 					uint32_t live = 0;
 #pragma unroll
-					for (int l = 0; l < 4; ++l) live |= ((e1[l] | e2[l] | e3[l]) >= 0 ? 1u : 0u) << l;
-					const int di = sdraw[j];
+					for (int i = 0; i < 4; ++i) live |= ((e1[i] | e2[i] | e3[i]) >= 0 ? 1u : 0u) << i;
+					const int di = static_cast<int>(smeta[j] & 0xffffu);
 					const DrawDesc& dd = draws[di];
 					if (live && dd.scissorOn) {
 						// the scissor flags of the rasteriser loops mask exactly
@@ -406,21 +454,12 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 						// are even)
 						const Rect S = draw_tile_rect(lite[di], (R.x0 / f.tileW), (R.y0 / f.tileH));
 #pragma unroll
-						for (int l = 0; l < 4; ++l) {
-							const int x = px + (l & 1), y = py + (l >> 1);
-							if (x < S.x0 || x >= S.x1 || y < S.y0 || y >= S.y1) live &= ~(1u << l); }}
+						for (int i = 0; i < 4; ++i) {
+							const int sx = px + (i & 1), sy = py + (i >> 1);
+							if (sx < S.x0 || sx >= S.x1 || sy < S.y0 || sy >= S.y1) live &= ~(1u << i); }}
 					if (live) {
 						frags += static_cast<uint32_t>(__popc(live));
-						float bx[4], by[4], bz[4], fd[4];
-#pragma unroll
-						for (int l = 0; l < 4; ++l) {
-							bx[l] = itof(e2[l]) * r.scale;
-							bz[l] = itof(e1[l]) * r.scale;
-							by[l] = (1.0F - bx[l]) - bz[l];
-							fd[l] = (bx[l] * r.z0 + by[l] * r.z1) + bz[l] * r.z2; }
-						// the program on the triangle's vertices (1/w, varyings) from
-						// LDS: it has no side effects, so it runs before the quad's
-						// depth test, which the ordered pass below applies
+						// the triangle's vertices (depth, 1/w, varyings)
 						const DrawLite& dl = lite[di];
 						const uint32_t src = ssrc[j], srcTri = src & 0x7fffffffu;
 						TriVerts tr;
@@ -432,83 +471,62 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 							const uint32_t fslot = r.slot - dl.slotBase - static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
 							clipped_verts(a.clipqOf[dl.triBase + srcTri] * kFanMax + (fslot - srcTri * kFanMax), a.cvpos, tr, vs);
 							vary = a.cvvary; }
+						float bx[4], by[4], bz[4], fd[4];
+#pragma unroll
+						for (int i = 0; i < 4; ++i) {
+							bx[i] = itof(e2[i]) * r.scale;
+							bz[i] = itof(e1[i]) * r.scale;
+							by[i] = (1.0F - bx[i]) - bz[i];
+							fd[i] = (bx[i] * tr.z[0] + by[i] * tr.z[1]) + bz[i] * tr.z[2]; }
 						float col[4][4];
 						ShadeQuad sq{ dd, tr.w, vary + tr.vary[0], vary + tr.vary[1], vary + tr.vary[2],
 						              bx, by, bz, fd, px, py, f.H, tr.clipped, col, 0xfu, true };
 						dispatch_program(dd.program, sq, L{});
-						pm = (live & sq.keep) | (live << 4);
+						wmask[t] = static_cast<uint8_t>((live & sq.keep) | (live << 4));
+						*reinterpret_cast<float4*>(wfd[t]) = make_float4(fd[0], fd[1], fd[2], fd[3]);
 #pragma unroll
-						for (int l = 0; l < 4; ++l) {
-							wfd[t][l] = fd[l];
-							wcol[t][l] = make_float4(col[l][0], col[l][1], col[l][2], col[l][3]); }}}
-				wmask[t] = pm;
-			}
-			__syncthreads();
-			// apply: each thread walks its quad's pairs of the window in
-			// triangle order with the frame commands between them:
-			// TriangleProgram::Render's early or late depth test and depth
-			// write around the program, then blend and the masked colour store
-			int jb = 0, je = static_cast<int>(cnt) - 1;   // the first triangle whose pairs end after w0
-			while (jb < je) { const int mid = (jb + je) >> 1; if (qoff[mid + 1] > w0) je = mid; else jb = mid + 1; }
-			for (int j = jb; j < static_cast<int>(cnt) && qoff[j] < w0 + kIoThreads; ++j) {
-				const uint32_t slot = srec[j].slot;
-				while (nextOp <= slot) { apply_op(ops[opi]); ++opi; nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
-				const uint32_t xy = sxy[j], cxy = scxy[j];
-				const int x0 = static_cast<int>(xy & 0xffffu), y0 = static_cast<int>(xy >> 16);
-				const int cx = static_cast<int>(cxy & 0xffffu), cy = static_cast<int>(cxy >> 16);
-				if (qx < x0 || qy < y0) continue;
-				const int ix = (qx - x0) >> 1, iy = (qy - y0) >> 1;
-				if (ix >= cx || iy >= cy) continue;
-				const uint32_t p = qoff[j] + static_cast<uint32_t>(iy * cx + ix);
-				if (p < w0 || p >= w0 + kIoThreads) continue;
-				const int wi = static_cast<int>(p - w0);
-				const uint32_t pm = wmask[wi];
-				uint32_t mask = pm >> 4;
-				if (!mask) continue;
-				const uint32_t st = sstate[j];
-				const bool depthTest = (st & 1u) != 0u, depthWrite = (st & 2u) != 0u, earlyZ = (st & 64u) != 0u;
-				const int depthFunc = static_cast<int>((st >> 2) & 3u);
-				float fd[4];
-#pragma unroll
-				for (int l = 0; l < 4; ++l) fd[l] = wfd[wi][l];
-				if (depthTest && earlyZ) {
-#pragma unroll
-					for (int l = 0; l < 4; ++l) if (!depth_pass(depthFunc, fd[l], dz[l])) mask &= ~(1u << l);
-					if (!mask) continue; }
-				if (depthWrite && earlyZ) {
-#pragma unroll
-					for (int l = 0; l < 4; ++l) if (mask & (1u << l)) dz[l] = fd[l]; }
-				mask &= pm & 0xfu;   // gl_triMask after ShadeFragment
-				if (depthTest && !earlyZ) {
-#pragma unroll
-					for (int l = 0; l < 4; ++l) if (!depth_pass(depthFunc, fd[l], dz[l])) mask &= ~(1u << l);
-					if (!mask) continue; }
-				if (depthWrite && !earlyZ) {
-#pragma unroll
-					for (int l = 0; l < 4; ++l) if (mask & (1u << l)) dz[l] = fd[l]; }
-				if (st & 16u) {
-#pragma unroll
-					for (int l = 0; l < 4; ++l) {
-						if (!(mask & (1u << l))) continue;
-						const float4 c = wcol[wi][l];
-						if (st & 32u) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
-							const float al = c.w, om = 1.0F - al;
-							cr[l] = c.x * al + cr[l] * om;
-							cg[l] = c.y * al + cg[l] * om;
-							cb[l] = c.z * al + cb[l] * om; }
-						else { cr[l] = c.x; cg[l] = c.y; cb[l] = c.z; }}}
-				const uint32_t prim = sprim[j];
-#pragma unroll
-				for (int l = 0; l < 4; ++l) if (mask & (1u << l)) pid[l] = prim; }
+						for (int i = 0; i < 4; ++i) wcol[t][i] = make_float4(col[i][0], col[i][1], col[i][2], col[i][3]);
+						atomicOr(&qpairs[wy * (kRegionDim / 2) + wx], 1ull << t); }}
+				__syncthreads();
+				// apply: the pairs of this pixel's quad in triangle order with the
+				// frame commands between them: TriangleProgram::Render's early or
+				// late depth test and depth write around the program, then blend
+				// and the masked colour store
+				unsigned long long todo = qpairs[quad];
+				while (todo) {
+					const int w = __ffsll(static_cast<long long>(todo)) - 1;
+					todo &= todo - 1;
+					const int j = wtri[w];
+					const uint32_t st = smeta[j] >> 16, pm = wmask[w];
+					const float fd = wfd[w][l];
+					const float4 c = wcol[w][l];
+					const uint32_t slot = stri[j].slot;
+					while (nextOp <= slot) { apply_op(ops[opi]); ++opi; nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
+					bool on = ((pm >> (4 + l)) & 1u) != 0u;
+					const bool keep = ((pm >> l) & 1u) != 0u;   // gl_triMask after ShadeFragment
+					const bool pass = !(st & 1u) || depth_pass(static_cast<int>((st >> 2) & 3u), fd, dz);
+					if (st & 64u) {   // early depth test and write
+						on = on && pass;
+						if (on && (st & 2u)) dz = fd;
+						on = on && keep; }
+					else {
+						on = on && keep && pass;
+						if (on && (st & 2u)) dz = fd; }
+					if (on) {
+						if (st & 16u) {
+							if (st & 32u) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
+								const float al = c.w, om = 1.0F - al;
+								cr = c.x * al + cr * om;
+								cg = c.y * al + cg * om;
+								cb = c.z * al + cb * om; }
+							else { cr = c.x; cg = c.y; cb = c.z; }}
+						pid = sprim[j]; }}
+				__syncthreads();
+				if (t < kRegionQuads) qpairs[t] = 0; }
 			__syncthreads(); }}
 	while (opi < ope) { apply_op(ops[opi]); ++opi; }
-	// fragments that reached the depth test, one atomic per workgroup
+	// fragments that reached the depth test, one atomic per region
 	for (int o = 32; o > 0; o >>= 1) frags += __shfl_xor(frags, o, 64);
-	if ((t & 63) == 0) sfrag[t >> 6] = frags;
-	__syncthreads();
-	if (t == 0) {
-		unsigned long long sum = 0;
-		for (int w = 0; w < kIoThreads / 64; ++w) sum += sfrag[w];
-		if (sum) atomicAdd(&a.ctr->slot[blockIdx.x % kCtrSlots].fragments, sum); }}
+	if (t == 0 && frags) atomicAdd(&a.ctr->slot[blockIdx.x % kCtrSlots].fragments, static_cast<unsigned long long>(frags)); }
 
 }  // namespace rgl

@@ -64,8 +64,7 @@ constexpr int kAttachColorDepth = 0, kAttachRGBF32 = 1;
 
 constexpr int kSortCap = 4096;       // records a tile sorts in LDS in one piece
 constexpr int kSortThreads = 1024;   // k_tile_order workgroup
-constexpr int kRegionDim = 8;        // k_inorder region: 8 x 8 pixels, a lane each; 4 x 4 quads
-constexpr int kRegionQuads = (kRegionDim / 2) * (kRegionDim / 2);
+constexpr int kRegionDim = 8;        // k_inorder region: 8 x 8 pixels, a lane each
 constexpr int kIoThreads = kRegionDim * kRegionDim;
 static_assert(kIoThreads == 64, "a region is one wave, its record masks one word per 64 records");
 
@@ -194,42 +193,15 @@ __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, const 
 	for (uint32_t i = t; i < n; i += kSortThreads) order[ob + i] = static_cast<uint32_t>(src[i]);
 	record_masks(n, ninl, d, ob, R, e.regionsX, e.regionsY, rec, crec, order, tm); }
 
-// ShadeFragment of program P for a quad at (qx, qy): perspective-correct BP
-// from BS and the vertices' 1/w (Render, rglv_gpu_impl.hxx:187-191),
-// varyings, gl_FragCoord and gl_FragDepth, the quad's texture LOD from
-// lanes 0 and 1; colour with alpha per lane, and the lanes the program
-// keeps (discard clears them)
-template <class P>
-__device__ inline uint32_t shade_quad(const DrawDesc& d, const float w[3], const float* v0, const float* v1, const float* v2,
-                                      const float bx[4], const float by[4], const float bz[4], const float fd[4], int qx, int qy,
-                                      int h, bool clipped, float col[4][4]) {
-	float vv[4][P::kVary];
-	FragCoord fc[4];
-#pragma unroll
-	for (int l = 0; l < 4; ++l) {
-		const float fragW = oneover((bx[l] * w[0] + by[l] * w[1]) + bz[l] * w[2]);
-		const float p0 = (w[0] * bx[l]) * fragW;
-		const float p2 = (w[2] * bz[l]) * fragW;
-		const float p1 = (1.0F - p0) - p2;
-#pragma unroll
-		for (int k = 0; k < P::kVary; ++k) vv[l][k] = (p0 * v0[k] + p1 * v1[k]) + p2 * v2[k];
-		fc[l] = frag_coord(qx, qy, l, h, clipped, fd[l]); }
-	int lod = 0;
-	float u0, w0, u1, w1;
-	if (lod_texcoord<P>(d, vv[0], fc[0], u0, w0) && lod_texcoord<P>(d, vv[1], fc[1], u1, w1))
-		lod = texture_lod(d.tu0, u0, u1, w0, w1);
-	uint32_t keep = 0;
-#pragma unroll
-	for (int l = 0; l < 4; ++l) keep |= (P::fragment(d, vv[l], lod, fc[l], col[l]) ? 1u : 0u) << l;
-	return keep; }
-
-struct ShadeQuad {
-	const DrawDesc& d; const float* w; const float* v0; const float* v1; const float* v2;
-	const float* bx; const float* by; const float* bz; const float* fd; int qx, qy, h; bool clipped;
-	float (*col)[4]; uint32_t keep; bool earlyZ;
+// the draw's program on one lane of a quad, the vertices' varyings loaded
+// with the triangle's vertex ids
+struct ShadeFrag {
+	const DrawDesc& d; const TriSetup& t; const TriVerts& tr; const float* vary;
+	int kx, ky, lane, h; float* col; float depth; bool keep;
 	template <class P> __device__ void run() {
-		keep = shade_quad<P>(d, w, v0, v1, v2, bx, by, bz, fd, qx, qy, h, clipped, col);
-		earlyZ = P::kEarlyZ; }};
+		typename ShadeOne<P>::Vary vy;
+		ShadeOne<P>::load(vary, tr, vy);
+		keep = shade_lane<P>(d, t, tr, vy.v[0], vy.v[1], vy.v[2], kx, ky, lane, kRcpMantissa, col, depth, h); }};
 
 // depth functions of the fragment state (DepthLT / DepthLE / DepthEQ,
 // rglv_gpu_impl.hxx:64-74)
@@ -248,30 +220,31 @@ __device__ inline uint32_t select_bit(unsigned long long m, uint32_t k) {
 		if (k >= c) { k -= c; at += h; w >>= h; }}
 	return at; }
 
-// what the shading reads of a batch's triangle
+// what the coverage and shading read of a batch's triangle
 struct alignas(16) IoTri {
-	int32_t c1, c2, c3;
-	int32_t dx12, dy12, dx23, dy23, dx31, dy31;
+	int32_t c1, c2, dx12, dy12, dx23, dy23;
 	uint32_t minxy;
 	float scale;
+	int32_t c3, dx31, dy31;   // coverage only
 	uint32_t slot;
 };
 static_assert(sizeof(IoTri) == 48, "three 16-byte rows");
 
 // A region's triangles come 64 at a time (the set bits of its record masks,
 // in order), and their (triangle, quad) pairs inside the region, at most 16
-// each, in windows of 64.  Shade: each lane takes one pair: coverage,
-// scissor, the program on the quad (programs have no side effects, so this
-// runs before the depth test); its bit goes into its quad's word.  Apply:
-// each lane walks the set bits of its pixel's quad, in slot order, with the
-// frame's commands between them.
+// each, in windows of 64.  Cover: each lane takes one pair and lists its
+// covered fragments.  Shade: each lane takes one fragment of the list and
+// runs the program (programs have no side effects, so this runs before the
+// depth test); its pair's bit goes into its pixel's word.  Apply: each lane
+// walks the set bits of its pixel, in slot order, with the frame's commands
+// between them.
 //
-// Bound: the chain of dependent fetches of a window (vertex ids, positions,
-// varyings, texels, about 3 us), times the windows of the heaviest region.
-// 8 x 8 regions of one wave each keep that chain short and need no barrier;
-// 16 x 16 regions, which walked all triangles of a batch per quad and all
-// batches of the tile, took 471 us on 327,680 blended triangles at
-// 1920x1080 where these take 219 us.
+// Bound: VALU issue (the program per fragment), and the two dependent fetches
+// of a window (positions with varyings, texels) in the heaviest regions.
+// 327,680 blended triangles at 1920x1080 take 144 us; a lane per quad in
+// the shading, three of whose four lanes are often not covered, took 219 us,
+// and 16 x 16 regions that walked all triangles of a batch per quad and all
+// batches of the tile 471 us.
 //
 // L: the programs the draws may use (a frame of one program compiles only
 // that program's shading, which keeps the registers, and so the resident
@@ -287,18 +260,19 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	__shared__ uint32_t spre[65];
 	// the batch's triangles: setup; draw | fragment state << 16 (bit 0 depth
 	// test, 1 depth write, 2-3 depth function, 4 colour write, 5 blend, 6
-	// early depth test); source triangle (bit 31: a clipped fan); primitive
-	// id; pair rect in the region's quads (x0 | y0 << 4 | cx << 8)
+	// early depth test, 7 the program runs); vertices (bit 31 of the first: in
+	// the clipped arrays); primitive id; pair rect in the region's quads (x0 |
+	// y0 << 4 | cx << 8)
 	__shared__ IoTri stri[64];
-	__shared__ uint32_t smeta[64], ssrc[64], sprim[64], srect[64], qoff[64];
-	// a window of pairs: its triangles, the lanes' depths and colours, the
-	// lanes (bits 0-3: live lanes the program keeps, 4-7: live lanes); per
-	// quad of the region the window's pairs with a live lane
-	__shared__ uint8_t wtri[64];
-	__shared__ uint8_t wmask[64];
-	__shared__ __attribute__((aligned(16))) float wfd[64][4];
+	__shared__ uint32_t smeta[64], sv0[64], sv1[64], sv2[64], sprim[64], srect[64], qoff[64];
+	// a window of pairs: its triangles and quads (x | y << 2), its covered
+	// fragments (pair | lane << 6), their depths, colours and whether the
+	// program kept them; per pixel of the region the pairs that cover it
+	__shared__ uint8_t wtri[64], wquad[64], flist[256];
+	__shared__ uint8_t wkeep[64][4];
+	__shared__ float wfd[64][4];
 	__shared__ float4 wcol[64][4];
-	__shared__ unsigned long long qpairs[kRegionQuads];
+	__shared__ unsigned long long ppairs[64];
 	const int vs = a.varyStride;
 	const int blk = static_cast<int>(blockIdx.x);
 	const IoFrame e = io[find_io(io, nIo, blk, false)];
@@ -370,9 +344,33 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				static_cast<float4*>(op.ptr)[static_cast<long long>(y) * op.stride + x] = make_float4(cr, cg, cb, 0.0F);
 			else static_cast<uint32_t*>(op.ptr)[o] = pid; }};
 
+	auto apply_pair = [&](int w) {
+		const int j = wtri[w];
+		const uint32_t st = smeta[j] >> 16;
+		const float fd = wfd[w][l];
+		const float4 c = wcol[w][l];
+		const bool keep = wkeep[w][l] != 0;   // gl_triMask after ShadeFragment
+		const bool pass = !(st & 1u) || depth_pass(static_cast<int>((st >> 2) & 3u), fd, dz);
+		bool on;
+		if (st & 64u) {   // early depth test and write
+			if (pass && (st & 2u)) dz = fd;
+			on = pass && keep; }
+		else {
+			on = keep && pass;
+			if (on && (st & 2u)) dz = fd; }
+		if (on) {
+			if (st & 16u) {
+				if (st & 32u) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
+					const float al = c.w, om = 1.0F - al;
+					cr = c.x * al + cr * om;
+					cg = c.y * al + cg * om;
+					cb = c.z * al + cb * om; }
+				else { cr = c.x; cg = c.y; cb = c.z; }}
+			pid = sprim[j]; }};
+
 	const uint32_t nb = (n + 63) >> 6;   // words of the region's record masks
 	const unsigned long long* rm = masks + mask_word(ob, e.tileStart + lt, maxRegions) + static_cast<long long>(reg) * nb;
-	if (t < kRegionQuads) qpairs[t] = 0;
+	ppairs[t] = 0;
 	for (uint32_t k0 = 0; k0 < nb; k0 += 64) {   // 64 words, 4,096 records, at a time
 		const unsigned long long mw = k0 + t < nb ? rm[k0 + t] : 0ull;
 		uint32_t hits = static_cast<uint32_t>(__popcll(mw));
@@ -397,17 +395,24 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				for (uint32_t st = 32; st > 0; st >>= 1) if (spre[lo + st] <= h) lo += st;
 				const uint32_t p = order[ob + 64 * (k0 + lo) + select_bit(smask[lo], h - spre[lo])];
 				const VisRec rr = p < ninl ? rec[vt.ib + p] : crec[vt.cb + (p - ninl)];
-				stri[t] = IoTri{ rr.c1, rr.c2, rr.c3, rr.dx12, rr.dy12, rr.dx23, rr.dy23, rr.dx31, rr.dy31, rr.minxy, rr.scale, rr.slot };
+				stri[t] = IoTri{ rr.c1, rr.c2, rr.dx12, rr.dy12, rr.dx23, rr.dy23, rr.minxy, rr.scale, rr.c3, rr.dx31, rr.dy31, rr.slot };
 				const int di = find_draw_slot(lite, b.nDraws, rr.slot);
 				const DrawLite& dl = lite[di];
 				const uint32_t rel = rr.slot - dl.slotBase;
 				const uint32_t nTri = static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
 				const uint32_t srcTri = rel < nTri ? rel : (rel - nTri) / kFanMax;
-				ssrc[t] = srcTri | (rel < nTri ? 0u : 0x80000000u);
+				if (rel < nTri) {
+					const uint4 tv = a.tvert[dl.triBase + srcTri];
+					sv0[t] = tv.x; sv1[t] = tv.y; sv2[t] = tv.z; }
+				else {   // the fan triangle's vertices (clipped_verts)
+					const uint32_t v0 = a.clipqOf[dl.triBase + srcTri] * kClipVerts, fj = rel - nTri - srcTri * kFanMax;
+					sv0[t] = v0 | 0x80000000u; sv1[t] = v0 + fj + 1; sv2[t] = v0 + fj + 2; }
 				const DrawDesc& dd = draws[di];
+				const ProgramInfo info = program_info(dd.program);
 				smeta[t] = static_cast<uint32_t>(di) |
 				           ((dd.depthTest ? 1u : 0u) | (dd.depthWrite ? 2u : 0u) | (static_cast<uint32_t>(dd.depthFunc) << 2) |
-				            (dd.colorWrite ? 16u : 0u) | (dd.blend ? 32u : 0u) | (program_info(dd.program).earlyZ ? 64u : 0u)) << 16;
+				            (dd.colorWrite ? 16u : 0u) | (dd.blend ? 32u : 0u) | (info.earlyZ ? 64u : 0u) |
+				            (dd.colorWrite || info.discard ? 128u : 0u)) << 16;
 				sprim[t] = dl.primBase + srcTri;
 				// its quads among the region's (both grids step 2 from even origins)
 				const int minx = static_cast<int>(rr.minxy & 0xffffu), miny = static_cast<int>(rr.minxy >> 16);
@@ -422,16 +427,21 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				if (t >= o) pend += v; }
 			const uint32_t total = __shfl(pend, 63, 64), pbeg = pend - np;
 			qoff[t] = pbeg;
+			__syncthreads();
+			// a frame command at or before the batch's last triangle
+			const bool anyOp = __any(nextOp <= stri[cnt - 1].slot);
 			for (uint32_t w0 = 0; w0 < total; w0 += 64) {
 				// the window's pairs name their triangles
 				for (uint32_t p = max(pbeg, w0), pe = min(pend, w0 + 64u); p < pe; ++p) wtri[p - w0] = static_cast<uint8_t>(t);
 				__syncthreads();
-				// shade: lane t takes pair w0 + t (coverage, scissor, the program)
+				// cover: lane t takes pair w0 + t
+				uint32_t live = 0;
 				if (w0 + static_cast<uint32_t>(t) < total) {
 					const int j = wtri[t];
 					const uint32_t k = w0 + static_cast<uint32_t>(t) - qoff[j], rc = srect[j], cx = rc >> 8;
 					const uint32_t iy = (k * (cx == 3u ? 22u : 64u >> (cx >> 1))) >> 6;   // k / cx for k < 16, cx <= 4
 					const uint32_t wx = (rc & 15u) + k - iy * cx, wy = ((rc >> 4) & 15u) + iy;
+					wquad[t] = static_cast<uint8_t>(wx | (wy << 2));
 					const int px = rx0 + 2 * static_cast<int>(wx), py = ry0 + 2 * static_cast<int>(wy);
 					const IoTri r = stri[j];
 					const int kx = (px - static_cast<int>(r.minxy & 0xffffu)) >> 1, ky = (py - static_cast<int>(r.minxy >> 16)) >> 1;
@@ -443,86 +453,93 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 					const int32_t e1[4] = { q1, wadd(q1, r.dy12), wadd(q1, r.dx12), wadd(wadd(q1, r.dx12), r.dy12) };
 					const int32_t e2[4] = { q2, wadd(q2, r.dy23), wadd(q2, r.dx23), wadd(wadd(q2, r.dx23), r.dy23) };
 					const int32_t e3[4] = { q3, wadd(q3, r.dy31), wadd(q3, r.dx31), wadd(wadd(q3, r.dx31), r.dy31) };
-					uint32_t live = 0;
 #pragma unroll
 					for (int i = 0; i < 4; ++i) live |= ((e1[i] | e2[i] | e3[i]) >= 0 ? 1u : 0u) << i;
-					const int di = static_cast<int>(smeta[j] & 0xffffu);
-					const DrawDesc& dd = draws[di];
-					if (live && dd.scissorOn) {
+					const DrawLite& dl = lite[smeta[j] & 0xffffu];
+					if (live && dl.scissorOn) {
 						// the scissor flags of the rasteriser loops mask exactly
 						// the lanes outside the clipped raster rect (tile origins
 						// are even)
-						const Rect S = draw_tile_rect(lite[di], (R.x0 / f.tileW), (R.y0 / f.tileH));
+						const Rect S = draw_tile_rect(dl, (R.x0 / f.tileW), (R.y0 / f.tileH));
 #pragma unroll
 						for (int i = 0; i < 4; ++i) {
 							const int sx = px + (i & 1), sy = py + (i >> 1);
-							if (sx < S.x0 || sx >= S.x1 || sy < S.y0 || sy >= S.y1) live &= ~(1u << i); }}
-					if (live) {
-						frags += static_cast<uint32_t>(__popc(live));
-						// the triangle's vertices (depth, 1/w, varyings)
-						const DrawLite& dl = lite[di];
-						const uint32_t src = ssrc[j], srcTri = src & 0x7fffffffu;
-						TriVerts tr;
-						const float* vary;
-						if (!(src >> 31)) {
-							inline_verts(a.tvert[dl.triBase + srcTri], a.vpos, tr, vs);
-							vary = a.vvary; }
-						else {
-							const uint32_t fslot = r.slot - dl.slotBase - static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
-							clipped_verts(a.clipqOf[dl.triBase + srcTri] * kFanMax + (fslot - srcTri * kFanMax), a.cvpos, tr, vs);
-							vary = a.cvvary; }
-						float bx[4], by[4], bz[4], fd[4];
+							if (sx < S.x0 || sx >= S.x1 || sy < S.y0 || sy >= S.y1) live &= ~(1u << i); }}}
+				const uint32_t nlive = static_cast<uint32_t>(__popc(live));
+				frags += nlive;
+				uint32_t fend = nlive;   // covered fragments up to and with this lane's pair
+				for (int o = 1; o < 64; o <<= 1) {
+					const uint32_t v = __shfl_up(fend, o, 64);
+					if (t >= o) fend += v; }
+				const uint32_t nf = __shfl(fend, 63, 64);
+				uint32_t fat = fend - nlive;
 #pragma unroll
-						for (int i = 0; i < 4; ++i) {
-							bx[i] = itof(e2[i]) * r.scale;
-							bz[i] = itof(e1[i]) * r.scale;
-							by[i] = (1.0F - bx[i]) - bz[i];
-							fd[i] = (bx[i] * tr.z[0] + by[i] * tr.z[1]) + bz[i] * tr.z[2]; }
-						float col[4][4];
-						ShadeQuad sq{ dd, tr.w, vary + tr.vary[0], vary + tr.vary[1], vary + tr.vary[2],
-						              bx, by, bz, fd, px, py, f.H, tr.clipped, col, 0xfu, true };
-						dispatch_program(dd.program, sq, L{});
-						wmask[t] = static_cast<uint8_t>((live & sq.keep) | (live << 4));
-						*reinterpret_cast<float4*>(wfd[t]) = make_float4(fd[0], fd[1], fd[2], fd[3]);
-#pragma unroll
-						for (int i = 0; i < 4; ++i) wcol[t][i] = make_float4(col[i][0], col[i][1], col[i][2], col[i][3]);
-						atomicOr(&qpairs[wy * (kRegionDim / 2) + wx], 1ull << t); }}
+				for (int i = 0; i < 4; ++i) if ((live >> i) & 1u) flist[fat++] = static_cast<uint8_t>(t | (i << 6));
 				__syncthreads();
-				// apply: the pairs of this pixel's quad in triangle order with the
+				// shade: lane t takes fragment f0 + t
+				for (uint32_t f0 = 0; f0 < nf; f0 += 64) {
+					if (f0 + static_cast<uint32_t>(t) >= nf) continue;
+					const uint32_t en = flist[f0 + static_cast<uint32_t>(t)];
+					const int w = static_cast<int>(en & 63u), fl = static_cast<int>(en >> 6), j = wtri[w], wq = wquad[w];
+					const IoTri& r = stri[j];
+					TriSetup ts;
+					ts.c1 = r.c1; ts.c2 = r.c2; ts.dx12 = r.dx12; ts.dy12 = r.dy12; ts.dx23 = r.dx23; ts.dy23 = r.dy23;
+					ts.minx = static_cast<int>(r.minxy & 0xffffu); ts.miny = static_cast<int>(r.minxy >> 16); ts.scale = r.scale;
+					const int kx = (rx0 + 2 * (wq & 3) - ts.minx) >> 1, ky = (ry0 + 2 * (wq >> 2) - ts.miny) >> 1;
+					const uint32_t v0 = sv0[j];
+					const bool clipped = (v0 >> 31) != 0u;
+					const uint32_t vi[3] = { v0 & 0x7fffffffu, sv1[j], sv2[j] };
+					const float4* vp = clipped ? a.cvpos : a.vpos;
+					TriVerts tr;
+					tr.clipped = clipped;
+#pragma unroll
+					for (int i = 0; i < 3; ++i) {
+						const float4 p = vp[vi[i]];
+						tr.z[i] = p.z; tr.w[i] = p.w;
+						tr.vary[i] = static_cast<long long>(vi[i]) * vs; }
+					const uint32_t meta = smeta[j];
+					const DrawDesc& dd = draws[meta & 0xffffu];
+					float col[4] = { 0.0F, 0.0F, 0.0F, 0.0F }, fd;
+					bool keep = true;
+					if (meta & (128u << 16)) {
+						ShadeFrag sf{ dd, ts, tr, clipped ? a.cvvary : a.vvary, kx, ky, fl, f.H, col, 0.0F, true };
+						dispatch_program(dd.program, sf, L{});
+						fd = sf.depth; keep = sf.keep; }
+					else {   // neither its colour nor its discard is used: the depth alone
+						const int32_t q1 = wadd(wadd(ts.c1, wmul(kx, wmul(ts.dy12, 2))), wmul(ky, wmul(ts.dx12, 2)));
+						const int32_t q2 = wadd(wadd(ts.c2, wmul(kx, wmul(ts.dy23, 2))), wmul(ky, wmul(ts.dx23, 2)));
+						const int32_t e1 = wadd(q1, wadd((fl & 1) ? ts.dy12 : 0, (fl & 2) ? ts.dx12 : 0));
+						const int32_t e2 = wadd(q2, wadd((fl & 1) ? ts.dy23 : 0, (fl & 2) ? ts.dx23 : 0));
+						const float bx = itof(e2) * ts.scale, bz = itof(e1) * ts.scale, by = (1.0F - bx) - bz;
+						fd = (bx * tr.z[0] + by * tr.z[1]) + bz * tr.z[2]; }
+					wkeep[w][fl] = keep ? 1 : 0;
+					wfd[w][fl] = fd;
+					wcol[w][fl] = make_float4(col[0], col[1], col[2], col[3]);
+					atomicOr(&ppairs[4 * wq + fl], 1ull << w); }
+				__syncthreads();
+				// apply: the pairs covering this pixel in triangle order with the
 				// frame commands between them: TriangleProgram::Render's early or
 				// late depth test and depth write around the program, then blend
 				// and the masked colour store
-				unsigned long long todo = qpairs[quad];
-				while (todo) {
-					const int w = __ffsll(static_cast<long long>(todo)) - 1;
-					todo &= todo - 1;
-					const int j = wtri[w];
-					const uint32_t st = smeta[j] >> 16, pm = wmask[w];
-					const float fd = wfd[w][l];
-					const float4 c = wcol[w][l];
-					const uint32_t slot = stri[j].slot;
-					while (nextOp <= slot) { apply_op(ops[opi]); ++opi; nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
-					bool on = ((pm >> (4 + l)) & 1u) != 0u;
-					const bool keep = ((pm >> l) & 1u) != 0u;   // gl_triMask after ShadeFragment
-					const bool pass = !(st & 1u) || depth_pass(static_cast<int>((st >> 2) & 3u), fd, dz);
-					if (st & 64u) {   // early depth test and write
-						on = on && pass;
-						if (on && (st & 2u)) dz = fd;
-						on = on && keep; }
-					else {
-						on = on && keep && pass;
-						if (on && (st & 2u)) dz = fd; }
-					if (on) {
-						if (st & 16u) {
-							if (st & 32u) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
-								const float al = c.w, om = 1.0F - al;
-								cr = c.x * al + cr * om;
-								cg = c.y * al + cg * om;
-								cb = c.z * al + cb * om; }
-							else { cr = c.x; cg = c.y; cb = c.z; }}
-						pid = sprim[j]; }}
-				__syncthreads();
-				if (t < kRegionQuads) qpairs[t] = 0; }
+				unsigned long long todo = ppairs[t];
+				ppairs[t] = 0;
+				if (anyOp) {
+					// a quad's lanes meet the frame commands together: before the
+					// first pair of any of them that the command precedes
+					unsigned long long qt = todo | __shfl_xor(todo, 1, 64);
+					qt |= __shfl_xor(qt, 2, 64);
+					while (qt) {
+						const int w = __ffsll(static_cast<long long>(qt)) - 1;
+						qt &= qt - 1;
+						const uint32_t slot = stri[wtri[w]].slot;
+						while (nextOp <= slot) { apply_op(ops[opi]); ++opi; nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
+						if ((todo >> w) & 1ull) apply_pair(w); }}
+				else
+					while (todo) {
+						const int w = __ffsll(static_cast<long long>(todo)) - 1;
+						todo &= todo - 1;
+						apply_pair(w); }
+				__syncthreads(); }
 			__syncthreads(); }}
 	while (opi < ope) { apply_op(ops[opi]); ++opi; }
 	// fragments that reached the depth test, one atomic per region

@@ -1215,12 +1215,13 @@ __device__ inline FragCoord frag_coord(int qx, int qy, int l, int h, bool clippe
 	fc.depth = depth;
 	return fc; }
 
-// shade one pixel (lane `lane` of quad (kx, ky)) of a winning triangle;
-// h = the target's height (gl_FragCoord)
+// the program on lane `lane` of quad (kx, ky) of a triangle: RGBA colour and
+// depth, false when the program discards it; h = the target's height
+// (gl_FragCoord)
 template <class P>
-__device__ inline void shade_pixel(const DrawDesc& d, const TriSetup& t, const TriVerts& tr, const float* v0, const float* v1,
-                                   const float* v2, int kx, int ky, int lane, const uint32_t* rcpTab, float color[3], float& depth,
-                                   int h = 0) {
+__device__ inline bool shade_lane(const DrawDesc& d, const TriSetup& t, const TriVerts& tr, const float* v0, const float* v1,
+                                  const float* v2, int kx, int ky, int lane, const uint32_t* rcpTab, float color[4], float& depth,
+                                  int h) {
 	const int32_t q1 = wadd(wadd(t.c1, wmul(kx, wmul(t.dy12, 2))), wmul(ky, wmul(t.dx12, 2)));
 	const int32_t q2 = wadd(wadd(t.c2, wmul(kx, wmul(t.dy23, 2))), wmul(ky, wmul(t.dx23, 2)));
 	// lane offsets of the rasteriser's quad: (c, c+dy, c+dx, c+dx+dy) (rglv_triangle.hxx:253-258)
@@ -1245,8 +1246,15 @@ __device__ inline void shade_pixel(const DrawDesc& d, const TriSetup& t, const T
 		lod_texcoord<P>(d, a0, frag_coord(qx, qy, 0, h, tr.clipped, l0.depth), u0, w0);
 		lod_texcoord<P>(d, a1, frag_coord(qx, qy, 1, h, tr.clipped, l1.depth), u1, w1);
 		lod = texture_lod(d.tu0, u0, u1, w0, w1); }
+	return P::fragment(d, vv, lod, fc, color); }
+
+// shade one pixel (lane `lane` of quad (kx, ky)) of a winning triangle
+template <class P>
+__device__ inline void shade_pixel(const DrawDesc& d, const TriSetup& t, const TriVerts& tr, const float* v0, const float* v1,
+                                   const float* v2, int kx, int ky, int lane, const uint32_t* rcpTab, float color[3], float& depth,
+                                   int h = 0) {
 	float c4[4];
-	(void)P::fragment(d, vv, lod, fc, c4);
+	(void)shade_lane<P>(d, t, tr, v0, v1, v2, kx, ky, lane, rcpTab, c4, depth, h);
 	color[0] = c4[0]; color[1] = c4[1]; color[2] = c4[2]; }
 
 // resolve shaders: one program known at compile time, or a switch over

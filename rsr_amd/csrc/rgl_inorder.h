@@ -274,7 +274,12 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	__shared__ float4 wcol[64][4];
 	__shared__ unsigned long long ppairs[64];
 	const int vs = a.varyStride;
-	const int blk = static_cast<int>(blockIdx.x);
+	// Workgroups are dealt round-robin over the eight XCDs: runs of 64 regions
+	// (a 64-pixel tile's) go to one XCD, whose L2 then reads the tile's
+	// records, vertices and texels once.
+	constexpr int kRun = 64 * kXcds;
+	const int wg = static_cast<int>(blockIdx.x);
+	const int blk = wg < static_cast<int>(gridDim.x) / kRun * kRun ? wg / kRun * kRun + (wg % kXcds) * 64 + (wg / kXcds) % 64 : wg;
 	const IoFrame e = io[find_io(io, nIo, blk, false)];
 	const FrameDesc& f = frames[e.frame];
 	const int rpt = e.regionsX * e.regionsY;

@@ -263,7 +263,7 @@ struct rgl_gpu {
 	DevArray<IoFrame> dIo;
 	std::vector<uint8_t> lastIo;
 	int nIo = 0, nIoTiles = 0, nIoBlocks = 0;
-	DevArray<uint32_t> order;
+	DevArray<IoRec> ioRec;          // the in-order tiles' records in submission order
 	DevArray<unsigned long long> ioMasks;   // per region of an in-order tile, a bit per sorted record that can touch it
 	int ioRegions = 1;              // the most regions per tile of the batch's in-order frames
 	DevArray<unsigned long long> skeys0, skeys1;
@@ -364,7 +364,7 @@ struct rgl_gpu {
 		dFrames.release();
 		if (hOps) (void)hipHostFree(hOps);
 		if (hIo) (void)hipHostFree(hIo);
-		dOps.release(); dIo.release(); order.release(); ioMasks.release(); skeys0.release(); skeys1.release();
+		dOps.release(); dIo.release(); ioRec.release(); ioMasks.release(); skeys0.release(); skeys1.release();
 		if (auxDone) (void)hipEventDestroy(auxDone);
 		if (graphExec) (void)hipGraphExecDestroy(graphExec);
 		if (capStream) (void)hipStreamDestroy(capStream);
@@ -787,7 +787,7 @@ struct rgl_gpu {
 		if (r != 0) return r;
 		if (!io.empty()) {
 			const size_t nl = static_cast<size_t>(listCap) + clistCap;
-			if ((e = Grow(order, nl)) != hipSuccess) return hipfail(e, "hipMalloc tile order");
+			if ((e = Grow(ioRec, nl)) != hipSuccess) return hipfail(e, "hipMalloc sorted records");
 			if ((e = Grow(ioMasks, (nl / 64 + static_cast<size_t>(ioTiles) + 1) * static_cast<size_t>(ioRegions))) != hipSuccess)
 				return hipfail(e, "hipMalloc record masks");
 			if ((e = Grow(skeys0, nl)) != hipSuccess) return hipfail(e, "hipMalloc sort keys");
@@ -1017,7 +1017,7 @@ struct rgl_gpu {
 		const void* ptrs[] = { vpos.p, vflags.p, vvary.p, trect.p, tvert.p, tileCount.p, tileCursor.p, tileOff.p, clipq.p, clipqOf.p,
 		                       cvpos.p, cvvary.p, fcount.p, frect.p, clipHist.p, clipOff.p, clipCursor.p, itemTile.p, tileDesc.p, scanPart.p, tileCost.p,
 		                       keys.p, rec.p, crec.p, mlpImg.p, probeWant.p, quadList.p, mlpQueue.p, qCount.p, mlpParams,
-		                       dOps.p, dIo.p, order.p, ioMasks.p, skeys0.p, skeys1.p };
+		                       dOps.p, dIo.p, ioRec.p, ioMasks.p, skeys0.p, skeys1.p };
 		mix(ptrs, sizeof(ptrs));
 		const uint32_t caps[] = { listCap, clipCap, clistCap, mlpSegCap, static_cast<uint32_t>(items), learned ? 1u : 0u,
 		                          static_cast<uint32_t>(mlpShadeBlocks) };
@@ -1075,7 +1075,7 @@ struct rgl_gpu {
 		template <class P> void run() { launch<ProgramList<P>>(); }
 		template <class L> void launch() {
 			k_inorder<L><<<g.nIoBlocks, kIoThreads, lds, g.stream>>>(b, ra, g.dIo.p, g.nIo, b.frames, g.dOps.p, g.dDraws.p, g.dLite.p, g.tileDesc.p,
-				g.rec.p, g.crec.p, g.order.p, g.ioMasks.p, g.ioRegions); }};
+				g.ioRec.p, g.ioMasks.p, g.ioRegions); }};
 	struct ResolveLaunch {
 		rgl_gpu& g; const BatchDesc& b; const RasterArgs& ra; unsigned rblocks; const DrawLite* lite; const DrawDesc* dd;
 		template <class P> void run() {
@@ -1158,8 +1158,8 @@ struct rgl_gpu {
 		// every tile region walks them (before k_resolve, whose first block
 		// publishes the frame's counters)
 		if (nIo > 0)
-			k_tile_order<<<nIoTiles, kSortThreads, 0, stream>>>(b, dIo.p, nIo, b.frames, tileDesc.p, rec.p, crec.p, order.p, skeys0.p,
-				skeys1.p, ioMasks.p, ioRegions);
+			k_tile_order<<<nIoTiles, kSortThreads, 0, stream>>>(b, ra, dIo.p, nIo, b.frames, dDraws.p, dLite.p, tileDesc.p, rec.p, crec.p, ioRec.p,
+				skeys0.p, skeys1.p, ioMasks.p, ioRegions);
 		// everything above writes this executor's buffers alone; what
 		// follows writes or samples the caller's, after the previous
 		// double-buffered frame has finished

@@ -9,8 +9,9 @@
 // more drawing).
 //
 //   k_tile_order  one workgroup per tile: the tile's (triangle, tile) setup
-//                 records, inline and clipped, sorted by submission slot, and
-//                 per region of the tile a bit per sorted record that can
+//                 records, inline and clipped, sorted by submission slot and
+//                 written in that order with their draw's state and vertices,
+//                 and per region of the tile a bit per sorted record that can
 //                 touch it.
 //   k_inorder     one wave per 8 x 8-pixel region of a tile, one lane per
 //                 pixel: the pixel's colour, depth and primitive id stay in
@@ -101,56 +102,77 @@ __device__ inline void merge_runs(const unsigned long long* src, unsigned long l
 		while (lo < hi) { const uint32_t mid = (lo + hi) >> 1; if (src[mid] < key) lo = mid + 1; else hi = mid; }
 		dst[a0 + own + (lo - base)] = key; }}
 
+// A tile's record as k_inorder reads it: the setup (dx31 = -(dx12 + dx23)
+// and dy31 likewise, in the wrapping arithmetic of the setup), its
+// triangle's vertices and its draw's fragment state, so that a region takes
+// a triangle with one 64-byte load.
+struct alignas(16) IoRec {
+	int32_t c1, c2, c3;
+	int32_t dx12, dy12, dx23, dy23;
+	uint32_t minxy;       // minx | miny << 16
+	float scale;
+	uint32_t slot;
+	uint32_t v0, v1, v2;  // vertices (bit 31 of v0: in the clipped arrays)
+	uint32_t meta;        // draw | state << 8 | quads across << 16 | quads down << 24
+	uint32_t prim;        // primitive id
+	uint32_t pad;
+};
+static_assert(sizeof(IoRec) == 64 && kMaxDraws <= 256 && kMaxAnyTileDim / 2 <= 255, "four 16-byte loads; the fields of meta");
+// the fragment state in IoRec::meta >> 8: depth test, depth write, depth
+// function (two bits), colour write, blend, early depth test, and whether
+// the program runs (its colour or its discard is used)
+constexpr uint32_t kStDepthTest = 1u, kStDepthWrite = 2u, kStDepthFunc = 2, kStColor = 16u, kStBlend = 32u, kStEarlyZ = 64u, kStProgram = 128u;
+
+__device__ inline IoRec make_io_rec(const VisRec& r, const DrawLite* __restrict__ lite, const DrawDesc* __restrict__ draws, int nDraws,
+                                    const uint4* __restrict__ tvert, const uint32_t* __restrict__ clipqOf) {
+	const int di = find_draw_slot(lite, nDraws, r.slot);
+	const DrawLite& dl = lite[di];
+	const DrawDesc& dd = draws[di];
+	const ProgramInfo info = program_info(dd.program);
+	const uint32_t rel = r.slot - dl.slotBase;
+	const uint32_t nTri = static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
+	const uint32_t srcTri = rel < nTri ? rel : (rel - nTri) / kFanMax;
+	IoRec o;
+	o.c1 = r.c1; o.c2 = r.c2; o.c3 = r.c3;
+	o.dx12 = r.dx12; o.dy12 = r.dy12; o.dx23 = r.dx23; o.dy23 = r.dy23;
+	o.minxy = r.minxy; o.scale = r.scale; o.slot = r.slot;
+	if (rel < nTri) {
+		const uint4 tv = tvert[dl.triBase + srcTri];
+		o.v0 = tv.x; o.v1 = tv.y; o.v2 = tv.z; }
+	else {   // the fan triangle's vertices (clipped_verts)
+		const uint32_t v0 = clipqOf[dl.triBase + srcTri] * kClipVerts, fj = rel - nTri - srcTri * kFanMax;
+		o.v0 = v0 | 0x80000000u; o.v1 = v0 + fj + 1; o.v2 = v0 + fj + 2; }
+	const uint32_t st = (dd.depthTest ? kStDepthTest : 0u) | (dd.depthWrite ? kStDepthWrite : 0u) |
+	                    (static_cast<uint32_t>(dd.depthFunc) << kStDepthFunc) | (dd.colorWrite ? kStColor : 0u) |
+	                    (dd.blend ? kStBlend : 0u) | (info.earlyZ ? kStEarlyZ : 0u) | (dd.colorWrite || info.discard ? kStProgram : 0u);
+	o.meta = static_cast<uint32_t>(di) | (st << 8) | ((r.nq & 0xffu) << 16) | ((r.nq >> 16) << 24);
+	o.prim = dl.primBase + srcTri;
+	o.pad = 0u;
+	return o; }
+
 // The word of a tile's record masks: masks[mask_word(...) + region * nb + k]
 // holds a bit per record 64 k .. 64 k + 63 of the tile's sorted list (nb =
 // ceil(n / 64) words per region) whose quads reach the region.  ob: the
-// tile's first position of order[], blk its index among the in-order tiles;
+// tile's first sorted record, blk its index among the in-order tiles;
 // maxRegions: the most regions per tile of the batch's in-order frames.
 // Ranges of different tiles are disjoint.
 __device__ inline long long mask_word(uint32_t ob, int blk, int maxRegions) {
 	return (static_cast<long long>(ob >> 6) + blk) * maxRegions; }
 
-// a tile's record masks, one wave per 64 sorted records: a ballot per region
-__device__ inline void record_masks(uint32_t n, uint32_t ninl, const VisTile& d, uint32_t ob, const Rect& R, int regionsX, int regionsY,
-                                    const VisRec* __restrict__ rec, const VisRec* __restrict__ crec, const uint32_t* __restrict__ order,
-                                    unsigned long long* __restrict__ masks) {
-	__syncthreads();   // the workgroup's order[] stores
-	const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-	const uint32_t nb = (n + 63) >> 6;
-	for (uint32_t k = wv; k < nb; k += nw) {   // uniform over the wave
-		int gx0 = 1, gx1 = 0, gy0 = 1, gy1 = 0;   // the regions the record's quads reach (none)
-		if (64 * k + lane < n) {
-			const uint32_t p = order[ob + 64 * k + lane];
-			const VisRec& r = p < ninl ? rec[d.ib + p] : crec[d.cb + (p - ninl)];
-			const uint2 v = *reinterpret_cast<const uint2*>(&r.minxy);   // minxy, nq
-			const int minx = static_cast<int>(v.x & 0xffffu) - R.x0, miny = static_cast<int>(v.x >> 16) - R.y0;
-			const int nqx = static_cast<int>(v.y & 0xffffu), nqy = static_cast<int>(v.y >> 16);
-			if (nqx > 0 && nqy > 0) {
-				gx0 = minx / kRegionDim; gx1 = (minx + 2 * nqx - 1) / kRegionDim;
-				gy0 = miny / kRegionDim; gy1 = (miny + 2 * nqy - 1) / kRegionDim; }}
-		unsigned long long mine = 0;
-		int reg = 0;
-		for (int gy = 0; gy < regionsY; ++gy)
-			for (int gx = 0; gx < regionsX; ++gx, ++reg) {
-				const unsigned long long m = __ballot(gx0 <= gx && gx <= gx1 && gy0 <= gy && gy <= gy1);
-				if ((reg & 63) == static_cast<int>(lane)) mine = m;
-				if ((reg & 63) == 63) masks[static_cast<long long>(reg - 63 + static_cast<int>(lane)) * nb + k] = mine; }
-		const int rest = reg & 63;
-		if (static_cast<int>(lane) < rest) masks[static_cast<long long>(reg - rest + static_cast<int>(lane)) * nb + k] = mine; }}
-
 // A tile's records in submission order.  Keys are (slot << 32 | p), p the
 // record's position in the tile (inline records first, then clipped); every
-// (triangle, tile) pair has its own slot, so keys are distinct.  order[ob +
-// k] receives the k-th record's p, ob = the tile's first inline + first
-// clipped list position (the tiles' ranges are disjoint).  Runs of 64 are
-// sorted in the lanes of a wave, then merged in LDS (up to kSortCap records,
-// and above that in global memory), each pass a binary search per key:
-// six passes of LDS latency for 4,096 records, where a bitonic network in
-// LDS took 78 passes and barriers (71 -> 31 us with tiles of up to 1,800).
-__global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, const IoFrame* __restrict__ io, int nIo,
-		const FrameDesc* __restrict__ frames, const VisTile* __restrict__ tileDesc, const VisRec* __restrict__ rec,
-		const VisRec* __restrict__ crec, uint32_t* __restrict__ order, unsigned long long* __restrict__ skeys0,
-		unsigned long long* __restrict__ skeys1, unsigned long long* __restrict__ masks, int maxRegions) {
+// (triangle, tile) pair has its own slot, so keys are distinct.  sorted[ob +
+// k] receives the k-th record, ob = the tile's first inline + first clipped
+// list position (the tiles' ranges are disjoint).  Runs of 64 are sorted in
+// the lanes of a wave, then merged in LDS (up to kSortCap records, and above
+// that in global memory), each pass a binary search per key: six passes of
+// LDS latency for 4,096 records, where a bitonic network in LDS took 78
+// passes and barriers (71 -> 31 us with tiles of up to 1,800).
+__global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, RasterArgs a, const IoFrame* __restrict__ io, int nIo,
+		const FrameDesc* __restrict__ frames, const DrawDesc* __restrict__ draws, const DrawLite* __restrict__ lite,
+		const VisTile* __restrict__ tileDesc, const VisRec* __restrict__ rec, const VisRec* __restrict__ crec,
+		IoRec* __restrict__ sorted, unsigned long long* __restrict__ skeys0, unsigned long long* __restrict__ skeys1,
+		unsigned long long* __restrict__ masks, int maxRegions) {
 	__shared__ unsigned long long s[2][kSortCap];
 	const int blk = static_cast<int>(blockIdx.x);
 	const IoFrame e = io[find_io(io, nIo, blk, true)];
@@ -172,26 +194,45 @@ __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, const 
 		int cur = 0;
 		for (uint32_t run = 64; run < cn; run <<= 1, cur ^= 1) { merge_runs(s[cur], s[cur ^ 1], cn, run); __syncthreads(); }
 		return cur; };
+	const unsigned long long* keys;   // the tile's sorted keys
+	if (n <= static_cast<uint32_t>(kSortCap)) keys = s[sort_lds(0, n)];
+	else {
+		unsigned long long* src = skeys0 + ob;
+		unsigned long long* dst = skeys1 + ob;
+		for (uint32_t c0 = 0; c0 < n; c0 += kSortCap) {
+			const uint32_t cn = min(static_cast<uint32_t>(kSortCap), n - c0);
+			__syncthreads();
+			const unsigned long long* v = s[sort_lds(c0, cn)];
+			for (uint32_t i = t; i < cn; i += kSortThreads) src[c0 + i] = v[i]; }
+		__syncthreads();
+		for (uint32_t run = kSortCap; run < n; run <<= 1) {
+			merge_runs(src, dst, n, run);
+			__syncthreads();
+			unsigned long long* x = src; src = dst; dst = x; }
+		keys = src; }
+	// the records in order and their masks, one wave per 64: a ballot per region
 	unsigned long long* const tm = masks + mask_word(ob, blk, maxRegions);
-	if (n <= static_cast<uint32_t>(kSortCap)) {
-		const unsigned long long* v = s[sort_lds(0, n)];
-		for (uint32_t i = t; i < n; i += kSortThreads) order[ob + i] = static_cast<uint32_t>(v[i]);
-		record_masks(n, ninl, d, ob, R, e.regionsX, e.regionsY, rec, crec, order, tm);
-		return; }
-	unsigned long long* src = skeys0 + ob;
-	unsigned long long* dst = skeys1 + ob;
-	for (uint32_t c0 = 0; c0 < n; c0 += kSortCap) {
-		const uint32_t cn = min(static_cast<uint32_t>(kSortCap), n - c0);
-		__syncthreads();
-		const unsigned long long* v = s[sort_lds(c0, cn)];
-		for (uint32_t i = t; i < cn; i += kSortThreads) src[c0 + i] = v[i]; }
-	__syncthreads();
-	for (uint32_t run = kSortCap; run < n; run <<= 1) {
-		merge_runs(src, dst, n, run);
-		__syncthreads();
-		unsigned long long* x = src; src = dst; dst = x; }
-	for (uint32_t i = t; i < n; i += kSortThreads) order[ob + i] = static_cast<uint32_t>(src[i]);
-	record_masks(n, ninl, d, ob, R, e.regionsX, e.regionsY, rec, crec, order, tm); }
+	const uint32_t nb = (n + 63) >> 6;
+	for (uint32_t k = t >> 6; k < nb; k += kSortThreads / 64) {   // uniform over the wave
+		int gx0 = 1, gx1 = 0, gy0 = 1, gy1 = 0;   // the regions the record's quads reach (none)
+		if (64 * k + lane < n) {
+			const uint32_t p = static_cast<uint32_t>(keys[64 * k + lane]);
+			const VisRec r = p < ninl ? rec[d.ib + p] : crec[d.cb + (p - ninl)];
+			const int minx = static_cast<int>(r.minxy & 0xffffu) - R.x0, miny = static_cast<int>(r.minxy >> 16) - R.y0;
+			const int nqx = static_cast<int>(r.nq & 0xffffu), nqy = static_cast<int>(r.nq >> 16);
+			if (nqx > 0 && nqy > 0) {
+				gx0 = minx / kRegionDim; gx1 = (minx + 2 * nqx - 1) / kRegionDim;
+				gy0 = miny / kRegionDim; gy1 = (miny + 2 * nqy - 1) / kRegionDim; }
+			sorted[ob + 64 * k + lane] = make_io_rec(r, lite, draws, b.nDraws, a.tvert, a.clipqOf); }
+		unsigned long long mine = 0;
+		int reg = 0;
+		for (int gy = 0; gy < e.regionsY; ++gy)
+			for (int gx = 0; gx < e.regionsX; ++gx, ++reg) {
+				const unsigned long long m = __ballot(gx0 <= gx && gx <= gx1 && gy0 <= gy && gy <= gy1);
+				if ((reg & 63) == static_cast<int>(lane)) mine = m;
+				if ((reg & 63) == 63) tm[static_cast<long long>(reg - 63 + static_cast<int>(lane)) * nb + k] = mine; }
+		const int rest = reg & 63;
+		if (static_cast<int>(lane) < rest) tm[static_cast<long long>(reg - rest + static_cast<int>(lane)) * nb + k] = mine; }}
 
 // the draw's program on one lane of a quad, the vertices' varyings loaded
 // with the triangle's vertex ids
@@ -220,16 +261,6 @@ __device__ inline uint32_t select_bit(unsigned long long m, uint32_t k) {
 		if (k >= c) { k -= c; at += h; w >>= h; }}
 	return at; }
 
-// what the coverage and shading read of a batch's triangle
-struct alignas(16) IoTri {
-	int32_t c1, c2, dx12, dy12, dx23, dy23;
-	uint32_t minxy;
-	float scale;
-	int32_t c3, dx31, dy31;   // coverage only
-	uint32_t slot;
-};
-static_assert(sizeof(IoTri) == 48, "three 16-byte rows");
-
 // A region's triangles come 64 at a time (the set bits of its record masks,
 // in order), and their (triangle, quad) pairs inside the region, at most 16
 // each, in windows of 64.  Cover: each lane takes one pair and lists its
@@ -252,19 +283,15 @@ static_assert(sizeof(IoTri) == 48, "three 16-byte rows");
 template <class L>
 __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs a, const IoFrame* __restrict__ io, int nIo,
 		const FrameDesc* __restrict__ frames, const FrameOp* __restrict__ ops, const DrawDesc* __restrict__ draws,
-		const DrawLite* __restrict__ lite, const VisTile* __restrict__ tileDesc, const VisRec* __restrict__ rec,
-		const VisRec* __restrict__ crec, const uint32_t* __restrict__ order, const unsigned long long* __restrict__ masks,
-		int maxRegions) {
+		const DrawLite* __restrict__ lite, const VisTile* __restrict__ tileDesc, const IoRec* __restrict__ sorted,
+		const unsigned long long* __restrict__ masks, int maxRegions) {
 	// 64 words of the region's record masks and the set bits before each
 	__shared__ unsigned long long smask[64];
 	__shared__ uint32_t spre[65];
-	// the batch's triangles: setup; draw | fragment state << 16 (bit 0 depth
-	// test, 1 depth write, 2-3 depth function, 4 colour write, 5 blend, 6
-	// early depth test, 7 the program runs); vertices (bit 31 of the first: in
-	// the clipped arrays); primitive id; pair rect in the region's quads (x0 |
-	// y0 << 4 | cx << 8)
-	__shared__ IoTri stri[64];
-	__shared__ uint32_t smeta[64], sv0[64], sv1[64], sv2[64], sprim[64], srect[64], qoff[64];
+	// the batch's triangles, and their pair rects in the region's quads (x0 |
+	// y0 << 4 | cx << 8) and first pairs
+	__shared__ IoRec stri[64];
+	__shared__ uint32_t srect[64], qoff[64];
 	// a window of pairs: its triangles and quads (x | y << 2), its covered
 	// fragments (pair | lane << 6), their depths, colours and whether the
 	// program kept them; per pixel of the region the pairs that cover it
@@ -304,12 +331,12 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	uint32_t pid = 0xffffffffu;
 	uint32_t frags = 0;
 	const VisTile vt = tileDesc[tile];
-	const uint32_t n = vt.ntot, ninl = vt.ninl, ob = vt.ib + vt.cb;
+	const uint32_t n = vt.ntot, ob = vt.ib + vt.cb;
 	uint32_t opi = static_cast<uint32_t>(f.opBase);
 	const uint32_t ope = static_cast<uint32_t>(f.opBase + f.nOps);
 	uint32_t nextOp = opi < ope ? ops[opi].pos : 0xffffffffu;   // the position of the next frame command
 
-	// the four lanes of a quad run it together
+	// every lane of the wave runs it (the downsampling store reads a quad's lanes)
 	auto apply_op = [&](const FrameOp& op) {
 		if (op.kind == kOpClear) {
 			if (op.bits & 1) { cr = op.color[0]; cg = op.color[1]; cb = op.color[2]; ca = op.color[3]; pid = 0xffffffffu; }
@@ -349,29 +376,32 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				static_cast<float4*>(op.ptr)[static_cast<long long>(y) * op.stride + x] = make_float4(cr, cg, cb, 0.0F);
 			else static_cast<uint32_t*>(op.ptr)[o] = pid; }};
 
-	auto apply_pair = [&](int w) {
+	auto apply_pairs = [&](unsigned long long todo) {
+	  while (todo) {
+		const int w = __ffsll(static_cast<long long>(todo)) - 1;
+		todo &= todo - 1;
 		const int j = wtri[w];
-		const uint32_t st = smeta[j] >> 16;
+		const uint32_t st = stri[j].meta >> 8;
 		const float fd = wfd[w][l];
 		const float4 c = wcol[w][l];
 		const bool keep = wkeep[w][l] != 0;   // gl_triMask after ShadeFragment
-		const bool pass = !(st & 1u) || depth_pass(static_cast<int>((st >> 2) & 3u), fd, dz);
+		const bool pass = !(st & kStDepthTest) || depth_pass(static_cast<int>((st >> kStDepthFunc) & 3u), fd, dz);
 		bool on;
-		if (st & 64u) {   // early depth test and write
-			if (pass && (st & 2u)) dz = fd;
+		if (st & kStEarlyZ) {   // early depth test and write
+			if (pass && (st & kStDepthWrite)) dz = fd;
 			on = pass && keep; }
 		else {
 			on = keep && pass;
-			if (on && (st & 2u)) dz = fd; }
+			if (on && (st & kStDepthWrite)) dz = fd; }
 		if (on) {
-			if (st & 16u) {
-				if (st & 32u) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
+			if (st & kStColor) {
+				if (st & kStBlend) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
 					const float al = c.w, om = 1.0F - al;
 					cr = c.x * al + cr * om;
 					cg = c.y * al + cg * om;
 					cb = c.z * al + cb * om; }
 				else { cr = c.x; cg = c.y; cb = c.z; }}
-			pid = sprim[j]; }};
+			pid = stri[j].prim; }}};
 
 	const uint32_t nb = (n + 63) >> 6;   // words of the region's record masks
 	const unsigned long long* rm = masks + mask_word(ob, e.tileStart + lt, maxRegions) + static_cast<long long>(reg) * nb;
@@ -389,52 +419,36 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 		spre[t + 1] = hits;
 		if (t == 0) spre[0] = 0;
 		__syncthreads();
+		// the region's h-th record of these words
+		auto record = [&](uint32_t h) {
+			uint32_t lo = 0;   // the word with spre[lo] <= h < spre[lo + 1]
+#pragma unroll
+			for (uint32_t st = 32; st > 0; st >>= 1) if (spre[lo + st] <= h) lo += st;
+			return sorted[ob + 64 * (k0 + lo) + select_bit(smask[lo], h - spre[lo])]; };
+		// each lane's record of the next batch is loaded while this one is drawn
+		IoRec rn;
+		if (static_cast<uint32_t>(t) < nh) rn = record(static_cast<uint32_t>(t));
 		for (uint32_t h0 = 0; h0 < nh; h0 += 64) {
-			// the batch: lane t takes the region's (h0 + t)-th record of these
+			// the batch: lane t takes the region's (h0 + t)-th record
 			const uint32_t cnt = min(64u, nh - h0);
 			uint32_t np = 0;
 			if (static_cast<uint32_t>(t) < cnt) {
-				const uint32_t h = h0 + static_cast<uint32_t>(t);
-				uint32_t lo = 0;   // the word with spre[lo] <= h < spre[lo + 1]
-#pragma unroll
-				for (uint32_t st = 32; st > 0; st >>= 1) if (spre[lo + st] <= h) lo += st;
-				const uint32_t p = order[ob + 64 * (k0 + lo) + select_bit(smask[lo], h - spre[lo])];
-				const VisRec rr = p < ninl ? rec[vt.ib + p] : crec[vt.cb + (p - ninl)];
-				stri[t] = IoTri{ rr.c1, rr.c2, rr.dx12, rr.dy12, rr.dx23, rr.dy23, rr.minxy, rr.scale, rr.c3, rr.dx31, rr.dy31, rr.slot };
-				const int di = find_draw_slot(lite, b.nDraws, rr.slot);
-				const DrawLite& dl = lite[di];
-				const uint32_t rel = rr.slot - dl.slotBase;
-				const uint32_t nTri = static_cast<uint32_t>(dl.tris) * static_cast<uint32_t>(dl.instances);
-				const uint32_t srcTri = rel < nTri ? rel : (rel - nTri) / kFanMax;
-				if (rel < nTri) {
-					const uint4 tv = a.tvert[dl.triBase + srcTri];
-					sv0[t] = tv.x; sv1[t] = tv.y; sv2[t] = tv.z; }
-				else {   // the fan triangle's vertices (clipped_verts)
-					const uint32_t v0 = a.clipqOf[dl.triBase + srcTri] * kClipVerts, fj = rel - nTri - srcTri * kFanMax;
-					sv0[t] = v0 | 0x80000000u; sv1[t] = v0 + fj + 1; sv2[t] = v0 + fj + 2; }
-				const DrawDesc& dd = draws[di];
-				const ProgramInfo info = program_info(dd.program);
-				smeta[t] = static_cast<uint32_t>(di) |
-				           ((dd.depthTest ? 1u : 0u) | (dd.depthWrite ? 2u : 0u) | (static_cast<uint32_t>(dd.depthFunc) << 2) |
-				            (dd.colorWrite ? 16u : 0u) | (dd.blend ? 32u : 0u) | (info.earlyZ ? 64u : 0u) |
-				            (dd.colorWrite || info.discard ? 128u : 0u)) << 16;
-				sprim[t] = dl.primBase + srcTri;
+				const IoRec r = rn;
+				stri[t] = r;
 				// its quads among the region's (both grids step 2 from even origins)
-				const int minx = static_cast<int>(rr.minxy & 0xffffu), miny = static_cast<int>(rr.minxy >> 16);
+				const int minx = static_cast<int>(r.minxy & 0xffffu), miny = static_cast<int>(r.minxy >> 16);
 				const int x0 = max(minx - rx0, 0) >> 1, y0 = max(miny - ry0, 0) >> 1;
-				const int x1 = min((minx - rx0) / 2 + static_cast<int>(rr.nq & 0xffffu), kRegionDim / 2);
-				const int y1 = min((miny - ry0) / 2 + static_cast<int>(rr.nq >> 16), kRegionDim / 2);
+				const int x1 = min((minx - rx0) / 2 + static_cast<int>((r.meta >> 16) & 0xffu), kRegionDim / 2);
+				const int y1 = min((miny - ry0) / 2 + static_cast<int>(r.meta >> 24), kRegionDim / 2);
 				np = static_cast<uint32_t>((x1 - x0) * (y1 - y0));
 				srect[t] = static_cast<uint32_t>(x0) | (static_cast<uint32_t>(y0) << 4) | (static_cast<uint32_t>(x1 - x0) << 8); }
+			if (h0 + 64 + static_cast<uint32_t>(t) < nh) rn = record(h0 + 64 + static_cast<uint32_t>(t));
 			uint32_t pend = np;   // pairs up to and with this lane's triangle
 			for (int o = 1; o < 64; o <<= 1) {
 				const uint32_t v = __shfl_up(pend, o, 64);
 				if (t >= o) pend += v; }
 			const uint32_t total = __shfl(pend, 63, 64), pbeg = pend - np;
 			qoff[t] = pbeg;
-			__syncthreads();
-			// a frame command at or before the batch's last triangle
-			const bool anyOp = __any(nextOp <= stri[cnt - 1].slot);
 			for (uint32_t w0 = 0; w0 < total; w0 += 64) {
 				// the window's pairs name their triangles
 				for (uint32_t p = max(pbeg, w0), pe = min(pend, w0 + 64u); p < pe; ++p) wtri[p - w0] = static_cast<uint8_t>(t);
@@ -448,19 +462,20 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 					const uint32_t wx = (rc & 15u) + k - iy * cx, wy = ((rc >> 4) & 15u) + iy;
 					wquad[t] = static_cast<uint8_t>(wx | (wy << 2));
 					const int px = rx0 + 2 * static_cast<int>(wx), py = ry0 + 2 * static_cast<int>(wy);
-					const IoTri r = stri[j];
+					const IoRec r = stri[j];
+					const int32_t dx31 = wsub(0, wadd(r.dx12, r.dx23)), dy31 = wsub(0, wadd(r.dy12, r.dy23));
 					const int kx = (px - static_cast<int>(r.minxy & 0xffffu)) >> 1, ky = (py - static_cast<int>(r.minxy >> 16)) >> 1;
 					// the quad's lanes (c, c+dy, c+dx, c+dx+dy), stepped as the
 					// rasteriser loops step (rglv_triangle.hxx:253-304)
 					const int32_t q1 = wadd(wadd(r.c1, wmul(kx, wmul(r.dy12, 2))), wmul(ky, wmul(r.dx12, 2)));
 					const int32_t q2 = wadd(wadd(r.c2, wmul(kx, wmul(r.dy23, 2))), wmul(ky, wmul(r.dx23, 2)));
-					const int32_t q3 = wadd(wadd(r.c3, wmul(kx, wmul(r.dy31, 2))), wmul(ky, wmul(r.dx31, 2)));
+					const int32_t q3 = wadd(wadd(r.c3, wmul(kx, wmul(dy31, 2))), wmul(ky, wmul(dx31, 2)));
 					const int32_t e1[4] = { q1, wadd(q1, r.dy12), wadd(q1, r.dx12), wadd(wadd(q1, r.dx12), r.dy12) };
 					const int32_t e2[4] = { q2, wadd(q2, r.dy23), wadd(q2, r.dx23), wadd(wadd(q2, r.dx23), r.dy23) };
-					const int32_t e3[4] = { q3, wadd(q3, r.dy31), wadd(q3, r.dx31), wadd(wadd(q3, r.dx31), r.dy31) };
+					const int32_t e3[4] = { q3, wadd(q3, dy31), wadd(q3, dx31), wadd(wadd(q3, dx31), dy31) };
 #pragma unroll
 					for (int i = 0; i < 4; ++i) live |= ((e1[i] | e2[i] | e3[i]) >= 0 ? 1u : 0u) << i;
-					const DrawLite& dl = lite[smeta[j] & 0xffffu];
+					const DrawLite& dl = lite[r.meta & 0xffu];
 					if (live && dl.scissorOn) {
 						// the scissor flags of the rasteriser loops mask exactly
 						// the lanes outside the clipped raster rect (tile origins
@@ -486,14 +501,13 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 					if (f0 + static_cast<uint32_t>(t) >= nf) continue;
 					const uint32_t en = flist[f0 + static_cast<uint32_t>(t)];
 					const int w = static_cast<int>(en & 63u), fl = static_cast<int>(en >> 6), j = wtri[w], wq = wquad[w];
-					const IoTri& r = stri[j];
+					const IoRec& r = stri[j];
 					TriSetup ts;
 					ts.c1 = r.c1; ts.c2 = r.c2; ts.dx12 = r.dx12; ts.dy12 = r.dy12; ts.dx23 = r.dx23; ts.dy23 = r.dy23;
 					ts.minx = static_cast<int>(r.minxy & 0xffffu); ts.miny = static_cast<int>(r.minxy >> 16); ts.scale = r.scale;
 					const int kx = (rx0 + 2 * (wq & 3) - ts.minx) >> 1, ky = (ry0 + 2 * (wq >> 2) - ts.miny) >> 1;
-					const uint32_t v0 = sv0[j];
-					const bool clipped = (v0 >> 31) != 0u;
-					const uint32_t vi[3] = { v0 & 0x7fffffffu, sv1[j], sv2[j] };
+					const bool clipped = (r.v0 >> 31) != 0u;
+					const uint32_t vi[3] = { r.v0 & 0x7fffffffu, r.v1, r.v2 };
 					const float4* vp = clipped ? a.cvpos : a.vpos;
 					TriVerts tr;
 					tr.clipped = clipped;
@@ -502,11 +516,11 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 						const float4 p = vp[vi[i]];
 						tr.z[i] = p.z; tr.w[i] = p.w;
 						tr.vary[i] = static_cast<long long>(vi[i]) * vs; }
-					const uint32_t meta = smeta[j];
-					const DrawDesc& dd = draws[meta & 0xffffu];
+					const uint32_t meta = r.meta;
+					const DrawDesc& dd = draws[meta & 0xffu];
 					float col[4] = { 0.0F, 0.0F, 0.0F, 0.0F }, fd;
 					bool keep = true;
-					if (meta & (128u << 16)) {
+					if (meta & (kStProgram << 8)) {
 						ShadeFrag sf{ dd, ts, tr, clipped ? a.cvvary : a.vvary, kx, ky, fl, f.H, col, 0.0F, true };
 						dispatch_program(dd.program, sf, L{});
 						fd = sf.depth; keep = sf.keep; }
@@ -528,22 +542,19 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				// and the masked colour store
 				unsigned long long todo = ppairs[t];
 				ppairs[t] = 0;
-				if (anyOp) {
-					// a quad's lanes meet the frame commands together: before the
-					// first pair of any of them that the command precedes
-					unsigned long long qt = todo | __shfl_xor(todo, 1, 64);
-					qt |= __shfl_xor(qt, 2, 64);
-					while (qt) {
-						const int w = __ffsll(static_cast<long long>(qt)) - 1;
-						qt &= qt - 1;
-						const uint32_t slot = stri[wtri[w]].slot;
-						while (nextOp <= slot) { apply_op(ops[opi]); ++opi; nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
-						if ((todo >> w) & 1ull) apply_pair(w); }}
-				else
-					while (todo) {
-						const int w = __ffsll(static_cast<long long>(todo)) - 1;
-						todo &= todo - 1;
-						apply_pair(w); }
+				// a command takes the whole wave between the pairs before and after
+				// it (in the same step: a command per pixel's own pairs made every
+				// quad fetch it again)
+				const uint32_t slot = w0 + static_cast<uint32_t>(t) < total ? stri[wtri[t]].slot : 0xffffffffu;
+				const uint32_t last = __builtin_amdgcn_readlane(slot, static_cast<int>(min(total - w0, 64u)) - 1);
+				while (nextOp <= last) {
+					const unsigned long long before = __ballot(slot < nextOp);
+					apply_pairs(todo & before);
+					todo &= ~before;
+					apply_op(ops[opi]);
+					++opi;
+					nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
+				apply_pairs(todo);
 				__syncthreads(); }
 			__syncthreads(); }}
 	while (opi < ope) { apply_op(ops[opi]); ++opi; }

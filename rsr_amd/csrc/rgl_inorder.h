@@ -264,18 +264,19 @@ __device__ inline uint32_t select_bit(unsigned long long m, uint32_t k) {
 // A region's triangles come 64 at a time (the set bits of its record masks,
 // in order), and their (triangle, quad) pairs inside the region, at most 16
 // each, in windows of 64.  Cover: each lane takes one pair and lists its
-// covered fragments.  Shade: each lane takes one fragment of the list and
-// runs the program (programs have no side effects, so this runs before the
-// depth test); its pair's bit goes into its pixel's word.  Apply: each lane
-// walks the set bits of its pixel, in slot order, with the frame's commands
-// between them.
+// covered fragments.  Rounds of 64 listed fragments follow.  Shade: each lane
+// takes one fragment and runs the program (programs have no side effects, so
+// this runs before the depth test); its bit goes into its pixel's word.
+// Apply: each lane walks the set bits of its pixel, in slot order, with the
+// frame's commands between them.
 //
-// Bound: VALU issue (the program per fragment), and the two dependent fetches
-// of a window (positions with varyings, texels) in the heaviest regions.
-// 327,680 blended triangles at 1920x1080 take 144 us; a lane per quad in
-// the shading, three of whose four lanes are often not covered, took 219 us,
-// and 16 x 16 regions that walked all triangles of a batch per quad and all
-// batches of the tile 471 us.
+// Bound: VALU issue (the program per fragment, about 60 of its 111 us on
+// 327,680 blended triangles at 1920x1080) and the two dependent fetches of a
+// round (positions with varyings, texels).  The LDS is kept to 8 KB, 19 waves
+// a CU, by holding one round's colours.  On the same frame: the colours of a
+// whole window (12 KB) 123 us, a lane per quad in the shading, three of whose
+// four lanes are often not covered, 219 us, and 16 x 16 regions that walked
+// all triangles of a batch per quad and all batches of the tile 471 us.
 //
 // L: the programs the draws may use (a frame of one program compiles only
 // that program's shading, which keeps the registers, and so the resident
@@ -292,14 +293,16 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	// y0 << 4 | cx << 8) and first pairs
 	__shared__ IoRec stri[64];
 	__shared__ uint32_t srect[64], qoff[64];
-	// a window of pairs: its triangles and quads (x | y << 2), its covered
-	// fragments (pair | lane << 6), their depths, colours and whether the
-	// program kept them; per pixel of the region the pairs that cover it
-	__shared__ uint8_t wtri[64], wquad[64], flist[256];
-	__shared__ uint8_t wkeep[64][4];
-	__shared__ float wfd[64][4];
-	__shared__ float4 wcol[64][4];
-	__shared__ unsigned long long ppairs[64];
+	// a window of pairs: its triangles; the covered fragments that wait to be
+	// shaded (triangle | pixel of the region << 6); a round of 64 of them:
+	// triangles, depths, colours, whether the program kept them, and per pixel
+	// the round's fragments
+	__shared__ uint8_t wtri[64];
+	__shared__ uint16_t flist[64 + 256];
+	__shared__ uint8_t rtri[64], rkeep[64];
+	__shared__ float rfd[64];
+	__shared__ float4 rcol[64];
+	__shared__ unsigned long long pfrags[64];
 	const int vs = a.varyStride;
 	// Workgroups are dealt round-robin over the eight XCDs: runs of 64 regions
 	// (a 64-pixel tile's) go to one XCD, whose L2 then reads the tile's
@@ -376,36 +379,98 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				static_cast<float4*>(op.ptr)[static_cast<long long>(y) * op.stride + x] = make_float4(cr, cg, cb, 0.0F);
 			else static_cast<uint32_t*>(op.ptr)[o] = pid; }};
 
-	auto apply_pairs = [&](unsigned long long todo) {
-	  while (todo) {
-		const int w = __ffsll(static_cast<long long>(todo)) - 1;
-		todo &= todo - 1;
-		const int j = wtri[w];
-		const uint32_t st = stri[j].meta >> 8;
-		const float fd = wfd[w][l];
-		const float4 c = wcol[w][l];
-		const bool keep = wkeep[w][l] != 0;   // gl_triMask after ShadeFragment
-		const bool pass = !(st & kStDepthTest) || depth_pass(static_cast<int>((st >> kStDepthFunc) & 3u), fd, dz);
-		bool on;
-		if (st & kStEarlyZ) {   // early depth test and write
-			if (pass && (st & kStDepthWrite)) dz = fd;
-			on = pass && keep; }
-		else {
-			on = keep && pass;
-			if (on && (st & kStDepthWrite)) dz = fd; }
-		if (on) {
-			if (st & kStColor) {
-				if (st & kStBlend) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
-					const float al = c.w, om = 1.0F - al;
-					cr = c.x * al + cr * om;
-					cg = c.y * al + cg * om;
-					cb = c.z * al + cb * om; }
-				else { cr = c.x; cg = c.y; cb = c.z; }}
-			pid = stri[j].prim; }}};
+	// the round's fragments of this pixel (bits of todo), in submission order
+	auto apply_frags = [&](unsigned long long todo) {
+		while (todo) {
+			const int w = __ffsll(static_cast<long long>(todo)) - 1;
+			todo &= todo - 1;
+			const int j = rtri[w];
+			const uint32_t st = stri[j].meta >> 8;
+			const float fd = rfd[w];
+			const float4 c = rcol[w];
+			const bool keep = rkeep[w] != 0;   // gl_triMask after ShadeFragment
+			const bool pass = !(st & kStDepthTest) || depth_pass(static_cast<int>((st >> kStDepthFunc) & 3u), fd, dz);
+			bool on;
+			if (st & kStEarlyZ) {   // early depth test and write
+				if (pass && (st & kStDepthWrite)) dz = fd;
+				on = pass && keep; }
+			else {
+				on = keep && pass;
+				if (on && (st & kStDepthWrite)) dz = fd; }
+			if (on) {
+				if (st & kStColor) {
+					if (st & kStBlend) {   // BlendAlpha (rglv_gpu_impl.hxx:80-84)
+						const float al = c.w, om = 1.0F - al;
+						cr = c.x * al + cr * om;
+						cg = c.y * al + cg * om;
+						cb = c.z * al + cb * om; }
+					else { cr = c.x; cg = c.y; cb = c.z; }}
+				pid = stri[j].prim; }}};
+
+	// one round: cnt of the listed fragments from f0 on (1 to 64), a lane each
+	auto round = [&](uint32_t f0, uint32_t cnt) {
+		uint32_t slot = 0xffffffffu;
+		if (static_cast<uint32_t>(t) < cnt) {
+			const uint32_t en = flist[f0 + static_cast<uint32_t>(t)];
+			const int j = static_cast<int>(en & 63u), fl = static_cast<int>((en >> 6) & 3u), wq = static_cast<int>(en >> 8);
+			const IoRec& r = stri[j];
+			TriSetup ts;
+			ts.c1 = r.c1; ts.c2 = r.c2; ts.dx12 = r.dx12; ts.dy12 = r.dy12; ts.dx23 = r.dx23; ts.dy23 = r.dy23;
+			ts.minx = static_cast<int>(r.minxy & 0xffffu); ts.miny = static_cast<int>(r.minxy >> 16); ts.scale = r.scale;
+			const int kx = (rx0 + 2 * (wq & 3) - ts.minx) >> 1, ky = (ry0 + 2 * (wq >> 2) - ts.miny) >> 1;
+			const bool clipped = (r.v0 >> 31) != 0u;
+			const uint32_t vi[3] = { r.v0 & 0x7fffffffu, r.v1, r.v2 };
+			const float4* vp = clipped ? a.cvpos : a.vpos;
+			TriVerts tr;
+			tr.clipped = clipped;
+#pragma unroll
+			for (int i = 0; i < 3; ++i) {
+				const float4 p = vp[vi[i]];
+				tr.z[i] = p.z; tr.w[i] = p.w;
+				tr.vary[i] = static_cast<long long>(vi[i]) * vs; }
+			const uint32_t meta = r.meta;
+			const DrawDesc& dd = draws[meta & 0xffu];
+			float col[4] = { 0.0F, 0.0F, 0.0F, 0.0F }, fd;
+			bool keep = true;
+			if (meta & (kStProgram << 8)) {
+				ShadeFrag sf{ dd, ts, tr, clipped ? a.cvvary : a.vvary, kx, ky, fl, f.H, col, 0.0F, true };
+				dispatch_program(dd.program, sf, L{});
+				fd = sf.depth; keep = sf.keep; }
+			else {   // neither its colour nor its discard is used: the depth alone
+				const int32_t q1 = wadd(wadd(ts.c1, wmul(kx, wmul(ts.dy12, 2))), wmul(ky, wmul(ts.dx12, 2)));
+				const int32_t q2 = wadd(wadd(ts.c2, wmul(kx, wmul(ts.dy23, 2))), wmul(ky, wmul(ts.dx23, 2)));
+				const int32_t e1 = wadd(q1, wadd((fl & 1) ? ts.dy12 : 0, (fl & 2) ? ts.dx12 : 0));
+				const int32_t e2 = wadd(q2, wadd((fl & 1) ? ts.dy23 : 0, (fl & 2) ? ts.dx23 : 0));
+				const float bx = itof(e2) * ts.scale, bz = itof(e1) * ts.scale, by = (1.0F - bx) - bz;
+				fd = (bx * tr.z[0] + by * tr.z[1]) + bz * tr.z[2]; }
+			rtri[t] = static_cast<uint8_t>(j);
+			rkeep[t] = keep ? 1 : 0;
+			rfd[t] = fd;
+			rcol[t] = make_float4(col[0], col[1], col[2], col[3]);
+			slot = r.slot;
+			atomicOr(&pfrags[en >> 6], 1ull << t); }
+		__syncthreads();
+		// apply: this pixel's fragments with the frame commands between them:
+		// TriangleProgram::Render's early or late depth test and depth write
+		// around the program, then blend and the masked colour store.  A
+		// command takes the whole wave between the fragments before and after
+		// it.
+		unsigned long long todo = pfrags[t];
+		pfrags[t] = 0;
+		const uint32_t last = __builtin_amdgcn_readlane(slot, static_cast<int>(cnt) - 1);
+		while (nextOp <= last) {
+			const unsigned long long before = __ballot(slot < nextOp);
+			apply_frags(todo & before);
+			todo &= ~before;
+			apply_op(ops[opi]);
+			++opi;
+			nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
+		apply_frags(todo);
+		__syncthreads(); };
 
 	const uint32_t nb = (n + 63) >> 6;   // words of the region's record masks
 	const unsigned long long* rm = masks + mask_word(ob, e.tileStart + lt, maxRegions) + static_cast<long long>(reg) * nb;
-	ppairs[t] = 0;
+	pfrags[t] = 0;
 	for (uint32_t k0 = 0; k0 < nb; k0 += 64) {   // 64 words, 4,096 records, at a time
 		const unsigned long long mw = k0 + t < nb ? rm[k0 + t] : 0ull;
 		uint32_t hits = static_cast<uint32_t>(__popcll(mw));
@@ -449,18 +514,19 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 				if (t >= o) pend += v; }
 			const uint32_t total = __shfl(pend, 63, 64), pbeg = pend - np;
 			qoff[t] = pbeg;
+			uint32_t nwait = 0;   // listed fragments
 			for (uint32_t w0 = 0; w0 < total; w0 += 64) {
 				// the window's pairs name their triangles
 				for (uint32_t p = max(pbeg, w0), pe = min(pend, w0 + 64u); p < pe; ++p) wtri[p - w0] = static_cast<uint8_t>(t);
 				__syncthreads();
 				// cover: lane t takes pair w0 + t
-				uint32_t live = 0;
+				uint32_t live = 0, entry = 0;
 				if (w0 + static_cast<uint32_t>(t) < total) {
 					const int j = wtri[t];
 					const uint32_t k = w0 + static_cast<uint32_t>(t) - qoff[j], rc = srect[j], cx = rc >> 8;
 					const uint32_t iy = (k * (cx == 3u ? 22u : 64u >> (cx >> 1))) >> 6;   // k / cx for k < 16, cx <= 4
 					const uint32_t wx = (rc & 15u) + k - iy * cx, wy = ((rc >> 4) & 15u) + iy;
-					wquad[t] = static_cast<uint8_t>(wx | (wy << 2));
+					entry = static_cast<uint32_t>(j) | (wx << 8) | (wy << 10);
 					const int px = rx0 + 2 * static_cast<int>(wx), py = ry0 + 2 * static_cast<int>(wy);
 					const IoRec r = stri[j];
 					const int32_t dx31 = wsub(0, wadd(r.dx12, r.dx23)), dy31 = wsub(0, wadd(r.dy12, r.dy23));
@@ -492,70 +558,23 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 					const uint32_t v = __shfl_up(fend, o, 64);
 					if (t >= o) fend += v; }
 				const uint32_t nf = __shfl(fend, 63, 64);
-				uint32_t fat = fend - nlive;
+				uint32_t fat = nwait + fend - nlive;
 #pragma unroll
-				for (int i = 0; i < 4; ++i) if ((live >> i) & 1u) flist[fat++] = static_cast<uint8_t>(t | (i << 6));
+				for (int i = 0; i < 4; ++i) if ((live >> i) & 1u) flist[fat++] = static_cast<uint16_t>(entry | (static_cast<uint32_t>(i) << 6));
+				nwait += nf;
 				__syncthreads();
-				// shade: lane t takes fragment f0 + t
-				for (uint32_t f0 = 0; f0 < nf; f0 += 64) {
-					if (f0 + static_cast<uint32_t>(t) >= nf) continue;
-					const uint32_t en = flist[f0 + static_cast<uint32_t>(t)];
-					const int w = static_cast<int>(en & 63u), fl = static_cast<int>(en >> 6), j = wtri[w], wq = wquad[w];
-					const IoRec& r = stri[j];
-					TriSetup ts;
-					ts.c1 = r.c1; ts.c2 = r.c2; ts.dx12 = r.dx12; ts.dy12 = r.dy12; ts.dx23 = r.dx23; ts.dy23 = r.dy23;
-					ts.minx = static_cast<int>(r.minxy & 0xffffu); ts.miny = static_cast<int>(r.minxy >> 16); ts.scale = r.scale;
-					const int kx = (rx0 + 2 * (wq & 3) - ts.minx) >> 1, ky = (ry0 + 2 * (wq >> 2) - ts.miny) >> 1;
-					const bool clipped = (r.v0 >> 31) != 0u;
-					const uint32_t vi[3] = { r.v0 & 0x7fffffffu, r.v1, r.v2 };
-					const float4* vp = clipped ? a.cvpos : a.vpos;
-					TriVerts tr;
-					tr.clipped = clipped;
-#pragma unroll
-					for (int i = 0; i < 3; ++i) {
-						const float4 p = vp[vi[i]];
-						tr.z[i] = p.z; tr.w[i] = p.w;
-						tr.vary[i] = static_cast<long long>(vi[i]) * vs; }
-					const uint32_t meta = r.meta;
-					const DrawDesc& dd = draws[meta & 0xffu];
-					float col[4] = { 0.0F, 0.0F, 0.0F, 0.0F }, fd;
-					bool keep = true;
-					if (meta & (kStProgram << 8)) {
-						ShadeFrag sf{ dd, ts, tr, clipped ? a.cvvary : a.vvary, kx, ky, fl, f.H, col, 0.0F, true };
-						dispatch_program(dd.program, sf, L{});
-						fd = sf.depth; keep = sf.keep; }
-					else {   // neither its colour nor its discard is used: the depth alone
-						const int32_t q1 = wadd(wadd(ts.c1, wmul(kx, wmul(ts.dy12, 2))), wmul(ky, wmul(ts.dx12, 2)));
-						const int32_t q2 = wadd(wadd(ts.c2, wmul(kx, wmul(ts.dy23, 2))), wmul(ky, wmul(ts.dx23, 2)));
-						const int32_t e1 = wadd(q1, wadd((fl & 1) ? ts.dy12 : 0, (fl & 2) ? ts.dx12 : 0));
-						const int32_t e2 = wadd(q2, wadd((fl & 1) ? ts.dy23 : 0, (fl & 2) ? ts.dx23 : 0));
-						const float bx = itof(e2) * ts.scale, bz = itof(e1) * ts.scale, by = (1.0F - bx) - bz;
-						fd = (bx * tr.z[0] + by * tr.z[1]) + bz * tr.z[2]; }
-					wkeep[w][fl] = keep ? 1 : 0;
-					wfd[w][fl] = fd;
-					wcol[w][fl] = make_float4(col[0], col[1], col[2], col[3]);
-					atomicOr(&ppairs[4 * wq + fl], 1ull << w); }
-				__syncthreads();
-				// apply: the pairs covering this pixel in triangle order with the
-				// frame commands between them: TriangleProgram::Render's early or
-				// late depth test and depth write around the program, then blend
-				// and the masked colour store
-				unsigned long long todo = ppairs[t];
-				ppairs[t] = 0;
-				// a command takes the whole wave between the pairs before and after
-				// it (in the same step: a command per pixel's own pairs made every
-				// quad fetch it again)
-				const uint32_t slot = w0 + static_cast<uint32_t>(t) < total ? stri[wtri[t]].slot : 0xffffffffu;
-				const uint32_t last = __builtin_amdgcn_readlane(slot, static_cast<int>(min(total - w0, 64u)) - 1);
-				while (nextOp <= last) {
-					const unsigned long long before = __ballot(slot < nextOp);
-					apply_pairs(todo & before);
-					todo &= ~before;
-					apply_op(ops[opi]);
-					++opi;
-					nextOp = opi < ope ? ops[opi].pos : 0xffffffffu; }
-				apply_pairs(todo);
-				__syncthreads(); }
+				// shade and apply whole rounds; what is left waits for the next
+				// window's fragments, or is the batch's last round
+				uint32_t f0 = 0;
+				for (; nwait - f0 >= 64; f0 += 64) round(f0, 64);
+				if (w0 + 64 >= total) {
+					if (nwait > f0) round(f0, nwait - f0);
+					nwait = 0; }
+				else if (f0 > 0) {
+					nwait -= f0;
+					const uint16_t en = flist[f0 + static_cast<uint32_t>(t)];
+					__syncthreads();
+					flist[t] = en; }}
 			__syncthreads(); }}
 	while (opi < ope) { apply_op(ops[opi]); ++opi; }
 	// fragments that reached the depth test, one atomic per region

@@ -100,3 +100,18 @@ def test_blended_config2_equals_the_key_path_frame():
     for name, a, b in (("colour", kc, bc), ("depth", kd, bd), ("prim", kp, bp)):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), name
     assert kst["fragments"] == bst["fragments"]
+
+
+@pytest.mark.parametrize("n,width,height", [(1, 8, 8), (1, 37, 23), (32, 64, 64), (33, 64, 64), (97, 61, 43), (2048, 16, 16),
+                                            (2049, 16, 16)])
+def test_record_counts(n, width, height):
+    # one tile of 2 n blended records: a region's batches of 64, the words of
+    # its record masks (64 records each, 64 words at a time) and the sort's
+    # runs of 64 and pieces of 4,096
+    import oracle_backend
+    from rsr_amd import rgl
+    from test_parity_gpu import _compare
+    from test_shared_tiles_gpu import _walls
+    sc = _walls(n, width, height)
+    sc.blend, sc.tile_blocks, sc.name = True, (8, 8), f"blended_{sc.name}"
+    _compare(sc.name, oracle_backend.render(sc, threads=8), rgl.render(sc))

@@ -210,6 +210,14 @@ int rgl_texture_pow2(const float* dev_src, int width, int height, float* dev_dst
    floats, base level in the first dim rows; one launch per level. */
 int rgl_texture_mipmap(float* dev_texels, int dim, void* hip_stream);
 
+/* The three above in one pass: dev_rgba8 = width*height decoded RGBA8
+   texels -> dev_texels = the dim x dim texture (dim a power of two of at
+   least the long edge; at most 16384 when it resamples), and when mip the
+   2*dim x dim buffer with the mip chain below it (dim at most 4096), texels
+   beside the chain zero. */
+int rgl_texture_prepare(const uint8_t* dev_rgba8, int width, int height, int premultiply, float* dev_texels, int dim,
+                        int mip, void* hip_stream);
+
 /* --- batches ----------------------------------------------------------- */
 /* No counterpart in the reference, which runs one GPU object per canvas
    (several at once for shadow passes, node/gllayer.cxx:152-181).  Draws

@@ -1562,6 +1562,17 @@ int rgl_texture_mipmap(float* buf, int dim, void* hip_stream) {
 		srcRow = dstRow; dstRow += size; }
 	return hipGetLastError() == hipSuccess ? 0 : RGL_E_HIP; }
 
+int rgl_texture_prepare(const uint8_t* src, int width, int height, int premultiply, float* dst, int dim, int mip, void* hip_stream) {
+	if (!src || !dst || width <= 0 || height <= 0 || dim < 2 || (dim & (dim - 1)) != 0 || dim < width || dim < height ||
+	    (mip ? dim > 4096 : dim > 16384 && (width != dim || height != dim))) return RGL_E_ARG;
+	const hipStream_t s = static_cast<hipStream_t>(hip_stream);
+	const unsigned n = static_cast<unsigned>((dim + kTexTile - 1) / kTexTile);
+	float4* d = reinterpret_cast<float4*>(dst);
+	hipLaunchKernelGGL(k_texture_prepare, dim3(n, n), dim3(256), 0, s, reinterpret_cast<const uchar4*>(src), width, height,
+	                   premultiply ? 1 : 0, d, dim, mip ? 1 : 0, srgb8_table());
+	if (mip && dim > kTexTile) hipLaunchKernelGGL(k_mip_tail, dim3(1), dim3(1024), 0, s, d, dim);
+	return hipGetLastError() == hipSuccess ? 0 : RGL_E_HIP; }
+
 /* ---- batches, graph replay and raster parameters (no reference counterpart) ---- */
 int rgl_gpu_run_batch(rgl_gpu* g, rgl_gpu* const* frames, int n, void* hip_stream) {
 	if (check(g)) return RGL_E_ARG;

@@ -85,6 +85,7 @@ def lib():
         L.rgl_texture_from_rgba8.argtypes = [vp, i, i, i, vp, vp]
         L.rgl_texture_pow2.argtypes = [vp, i, i, vp, i, vp]
         L.rgl_texture_mipmap.argtypes = [vp, i, vp]
+        L.rgl_texture_prepare.argtypes = [vp, i, i, i, vp, i, i, vp]
         L.rgl_gpu_run_batch.argtypes = [vp, ctypes.POINTER(vp), i, vp]
         L.rgl_gpu_set_graph.argtypes = [vp, i]
         L.rgl_gpu_set_double_buffer.argtypes = [vp, i]
@@ -118,6 +119,7 @@ EXPORTS = [
     "rgl_gl_clear", "rgl_gl_store_color_tc", "rgl_gl_store_depth", "rgl_gl_store_primitive_id",
     "rgl_gl_store_color_fp", "rgl_gl_store_color_quads", "rgl_kawase_blur",
     "rgl_gl_reset", "rgl_texture_make_mipmap", "rgl_texture_from_rgba8", "rgl_texture_pow2", "rgl_texture_mipmap",
+    "rgl_texture_prepare",
     "rgl_gpu_run_batch", "rgl_gpu_set_graph", "rgl_gpu_set_double_buffer", "rgl_gpu_wait_previous", "rgl_gpu_graph_captures", "rgl_gpu_set_raster_params",
     "rgl_gpu_set_guard_band",
     "rgl_mlp_param_count", "rgl_mlp_trainable_count", "rgl_gpu_set_learned_shading",
@@ -141,22 +143,10 @@ def texture_from_rgba8(rgba8, premultiply: bool = False, mip: bool = True):
     h, w = int(src.shape[0]), int(src.shape[1])
     s = torch.cuda.current_stream(src.device).cuda_stream
     L = lib()
-    f = torch.empty((h, w, 4), dtype=torch.float32, device=src.device)
-    if L.rgl_texture_from_rgba8(src.data_ptr(), w, h, int(premultiply), f.data_ptr(), s) != 0:
-        raise RglError("rgl_texture_from_rgba8 failed")
     dim = 1 << max(1, (max(w, h) - 1).bit_length())
-    if w == h and w == dim:
-        sq = f
-    else:
-        sq = torch.empty((dim, dim, 4), dtype=torch.float32, device=src.device)
-        if L.rgl_texture_pow2(f.data_ptr(), w, h, sq.data_ptr(), dim, s) != 0:
-            raise RglError("rgl_texture_pow2 failed")
-    if not mip:
-        return sq, dim
-    out = torch.zeros((2 * dim, dim, 4), dtype=torch.float32, device=src.device)
-    out[:dim] = sq
-    if L.rgl_texture_mipmap(out.data_ptr(), dim, s) != 0:
-        raise RglError("rgl_texture_mipmap failed")
+    out = torch.empty((2 * dim if mip else dim, dim, 4), dtype=torch.float32, device=src.device)
+    if L.rgl_texture_prepare(src.data_ptr(), w, h, int(premultiply), out.data_ptr(), dim, int(mip), s) != 0:
+        raise RglError("rgl_texture_prepare failed")
     return out, dim
 
 

@@ -67,3 +67,18 @@ def test_png_texture_drawn_matches_oracle():
         S.draw(sc, "sphere") + S.stores()
     sc.outputs = S.OUT3
     _check(sc)
+
+
+@pytest.mark.parametrize("h,w,pm", [(1, 1, False), (2, 2, True), (3, 4, False), (16, 16, False), (31, 32, True), (33, 64, False),
+                                    (65, 65, False), (128, 128, True), (130, 257, False), (777, 1000, True), (1024, 1024, False),
+                                    (9, 4096, False)])
+def test_texture_at_tile_and_level_edges(h, w, pm):
+    # dims 2 to 4096: levels within a wave (up to 16 texels), a workgroup (64)
+    # and the tail, ragged and square images
+    from rsr_amd import rgl
+    rgba8 = np.random.default_rng(7 * h + w).integers(0, 256, (h, w, 4), dtype=np.uint8)
+    got, dim = rgl.texture_from_rgba8(rgba8, premultiply=pm)
+    want, wdim = _host_texture(rgba8, pm)
+    assert dim == wdim and np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    base, _ = rgl.texture_from_rgba8(rgba8, premultiply=pm, mip=False)
+    assert np.array_equal(base.cpu().numpy().view(np.uint32), want[:dim].view(np.uint32))

@@ -1142,11 +1142,14 @@ struct rgl_gpu {
 			sa.clipq = clipq.p; sa.fcount = fcount.p; sa.frect = frect.p; sa.cvpos = cvpos.p; sa.clipCap = clipCap;
 			sa.clipCursor = clipCursor.p; sa.crec = crec.p; sa.clistCap = clistCap; sa.clipBlocks = kClipScatterBlocks;
 			sa.tileOff = tileOff.p; sa.clipOff = clipOff.p; sa.keys = keys.p; sa.ctr = dCtr;
+			// the units list their triangles where the list fits beside the window
+			const size_t winBytes = b.unitWindow * sizeof(uint32_t), listBytes = b.unitTris * sizeof(uint16_t);
+			sa.listed = !fusedScan && kScatterLdsBytes + winBytes + listBytes <= kUnitLdsBytes ? 1 : 0;
 			sa.fused = fusedScan ? 1 : 0; sa.tileCount = tileCount.p; sa.clipHist = clipHist.p;
 			sa.scan = so;
 			sa.scan.tileCursor = nullptr; sa.scan.clipCursor = nullptr;
-			k_scatter<<<(fusedScan ? 1 : 0) + b.units + kClipScatterBlocks + kResetBlocks, kUnitThreads, b.unitWindow * sizeof(uint32_t),
-				stream>>>(b, dLite.p, sa); }
+			k_scatter<<<(fusedScan ? 1 : 0) + b.units + kClipScatterBlocks + kResetBlocks, kUnitThreads,
+				winBytes + (sa.listed ? listBytes : 0), stream>>>(b, dLite.p, sa); }
 		Mark(5);
 		if (nIo < b.nFrames) {
 			// one workgroup per work item, sized from the last completed frame;
@@ -1210,6 +1213,7 @@ struct rgl_gpu {
 		return 0; }
 
 	static constexpr int kClipScatterBlocks = 32;   // k_scatter blocks that place the clipped fans
+	static constexpr size_t kScatterLdsBytes = 6 * 1024;  // k_scatter's own arrays, at most
 	static constexpr size_t kUnitLdsBytes = 160 * 1024;   // LDS per workgroup on gfx950
 	static constexpr int kResetBlocks = 128;        // k_scatter blocks that reset the keys of multi-segment tiles
 

@@ -26,6 +26,16 @@ def _walls(n, width, height):
     return sc
 
 
+def test_tiles_of_8_pixels():
+    # 32,400 tiles: the unit's tile window leaves no room for its list
+    import oracle_backend
+    from rsr_amd import rgl
+    from test_parity_gpu import _compare
+    sc = _walls(3, 1920, 1080)
+    sc.tile_blocks, sc.name = (1, 1), "walls3_1920x1080_tile8"
+    _compare(sc.name, oracle_backend.render(sc, threads=8), rgl.render(sc))
+
+
 @pytest.mark.parametrize("n,width,height", [(1, 333, 211), (128, 640, 360), (129, 640, 360), (300, 640, 360),
                                             (256, 2048, 1056), (300, 2048, 1056)])
 def test_walls(n, width, height):

@@ -96,7 +96,7 @@ __host__ __device__ inline int32_t imin(int32_t a, int32_t b) { return a < b ? a
 __host__ __device__ inline int32_t imax(int32_t a, int32_t b) { return a > b ? a : b; }
 
 // ryg float_to_srgb8_var2_SSE2 (3rdparty/ryg-srgb/ryg-srgb.h:183-219)
-__device__ inline uint32_t to_srgb8(float f) {
+__host__ __device__ inline uint32_t to_srgb8(float f) {
 	const float clamp1 = sse_max(f, u2f((127u - 13u) << 23));
 	const float clamp2 = sse_min(clamp1, u2f(0x3f7fffffu));
 	const uint32_t bits = f2u(clamp2);
@@ -113,7 +113,7 @@ __device__ inline uint32_t to_srgb8_tab(float f, const uint32_t* tab4) {
 	return ((tab & 0xffffu) * t + (tab >> 16) * 512u) >> 16; }
 
 // to_tc_basic (rglr_canvas_util.hxx:40-48)
-__device__ inline uint32_t to_linear8(float a) {
+__host__ __device__ inline uint32_t to_linear8(float a) {
 	float r = sse_min(a, 1.0F);
 	r = sse_max(r, 0.0F);
 	return static_cast<uint32_t>(cvtt(r * 255.0F)); }
@@ -289,6 +289,12 @@ struct FrameDesc {
 	uint32_t* outColor; int gamma; int postProgram; float exposure;
 	float* outDepth;
 	uint32_t* outPrim;
+	// log2 of the tile size when both are powers of two of at least 16 (a
+	// resolve block then lies in one tile) and the cleared pixel is the same
+	// everywhere (the IQ post program's is not), -1 otherwise; that pixel, and
+	// whether rows and outputs are 16-byte aligned
+	int shiftX, shiftY;
+	uint32_t clearPixel; int wideStores;
 	// 1: drawn by the in-order tile path (its commands opBase .. opBase +
 	// nOps of the batch's frame-command table apply in submission order)
 	int inOrder, opBase, nOps;
@@ -306,6 +312,7 @@ struct BatchDesc {
 	int nBlocks;             // resolve blocks, all frames
 	int segPairs;            // (triangle, tile) pairs per visibility work item
 	int splitQuads;          // quad work per quadrant from which it is cut in 2, and from twice this in 4 (0: never)
+	int skipEmpty;           // 1: tiles without records get no keys and resolve to the clear values (frames with shiftX >= 0)
 	int unitWindow;          // most tiles one binning unit's frames span (its LDS tile table)
 	const FrameDesc* frames; // device table, nFrames entries
 };

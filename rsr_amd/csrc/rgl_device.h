@@ -295,6 +295,8 @@ struct FrameDesc {
 	// whether rows and outputs are 16-byte aligned
 	int shiftX, shiftY;
 	uint32_t clearPixel; int wideStores;
+	int tileShiftX, tileShiftY;   // log2 of the tile's width and height, -1 where it is no power of two
+	uint32_t blocksMagic;         // lb / blocksX = mulhi(lb, blocksMagic) for the frame's block lb (0: divide)
 	// 1: drawn by the in-order tile path (its commands opBase .. opBase +
 	// nOps of the batch's frame-command table apply in submission order)
 	int inOrder, opBase, nOps;
@@ -316,6 +318,10 @@ struct BatchDesc {
 	int unitWindow;          // most tiles one binning unit's frames span (its LDS tile table)
 	const FrameDesc* frames; // device table, nFrames entries
 };
+
+// v / size, by a shift where the size is a power of two (shift >= 0): a
+// division by a value known at run time takes some 35 instructions
+__device__ inline int tile_of(int v, int size, int shift) { return shift >= 0 ? v >> shift : v / size; }
 
 // last k in [0, n) with base(k) <= v, for a nondecreasing table
 __device__ inline int find_base(const int* base, int n, int v) {

@@ -407,6 +407,8 @@ struct rgl_gpu {
 		f.W = W; f.H = H; f.tileW = tileW; f.tileH = tileH; f.tilesX = tilesX; f.tilesY = tilesY;
 		f.nTiles = tilesX * tilesY;
 		f.shiftX = f.shiftY = -1;
+		auto shift = [](int v) { return (v & (v - 1)) == 0 ? ilog2(static_cast<unsigned>(v)) : -1; };
+		f.tileShiftX = shift(tileW); f.tileShiftY = shift(tileH);
 		f.tileBase = tileBase;
 		f.depthFunc = -1;
 		f.drawEnabled = 1;
@@ -511,9 +513,8 @@ struct rgl_gpu {
 			if (clears == 0) { f.doClearColor = 0; f.doClearDepth = 0; }
 			if (f.depthFunc < 0) f.depthFunc = GL_LESS;
 			if (std::isnan(f.clearDepth)) f.drawEnabled = 0;
-			if (f.postProgram != 3 && tileW >= kResolveW && tileH >= kResolveH && (tileW & (tileW - 1)) == 0 && (tileH & (tileH - 1)) == 0) {
-				f.shiftX = ilog2(static_cast<unsigned>(tileW));
-				f.shiftY = ilog2(static_cast<unsigned>(tileH));
+			if (f.postProgram != 3 && tileW >= kResolveW && tileH >= kResolveH && f.tileShiftX >= 0 && f.tileShiftY >= 0) {
+				f.shiftX = f.tileShiftX; f.shiftY = f.tileShiftY;
 				// post_pixel of the clear colour
 				uint32_t px[3];
 				for (int ch = 0; ch < 3; ++ch) {
@@ -755,6 +756,9 @@ struct rgl_gpu {
 			FrameDesc& f = frames[i];
 			f.keyBase = keyBase; f.blockBase = blockBase;
 			f.blocksX = (f.W + kResolveW - 1) / kResolveW;
+			// exact while block * blocksX < 2^32
+			const unsigned long long bx = f.blocksX, blocks = bx * ((f.H + kResolveH - 1) / kResolveH);
+			f.blocksMagic = bx > 1 && blocks * bx < (1ull << 32) ? static_cast<uint32_t>(((1ull << 32) + bx - 1) / bx) : 0u;
 			tileBase += f.nTiles;
 			keyBase += static_cast<long long>(f.W) * f.H;
 			// frames drawn in order store their own pixels: no resolve blocks
@@ -1131,7 +1135,7 @@ struct rgl_gpu {
 		if (zeroHere) k_zero_counters<<<std::max(8, std::min((kCountGroups * b.nTiles + 255) / 256, 256)), 256, 0, stream>>>(za);
 		Mark(1);
 		if (b.units > 0) {
-			k_setup_count<<<b.units, kUnitThreads, dlBytes + b.unitWindow * sizeof(uint32_t), stream>>>(dDraws.p, b, vpos.p, vflags.p, trect.p, tvert.p,
+			k_setup_count<<<b.units, kUnitThreads, dlBytes + b.unitWindow * sizeof(uint32_t), stream>>>(dLite.p, b, vpos.p, vflags.p, trect.p, tvert.p,
 				tileCount.p, clipq.p, clipqOf.p, clipCap, dCtr); }
 		Mark(2);
 		// clipping: the clip queue is complete after setup; the clipped

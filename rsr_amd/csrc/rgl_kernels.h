@@ -79,6 +79,7 @@ struct alignas(16) DrawLite {
 	int tileW, tileH, tilesX, tilesY, tileBase;   // the draw's frame tile grid
 	int fW, fH;                                  // and its size
 	int scissorOn;                               // 1: the raster rect is the tile rect clipped by scissor[]
+	int tileShiftX, tileShiftY;                  // log2 of the tile's size, -1 where it is no power of two
 };
 
 __device__ inline int find_draw_ll(const DrawLite* dl, int nDraws, long long s) {
@@ -117,10 +118,15 @@ __host__ __device__ inline DrawLite make_lite(const DrawDesc& d) {
 	l.tileW = d.tileW; l.tileH = d.tileH; l.tilesX = d.tilesX; l.tilesY = d.tilesY; l.tileBase = d.tileBase;
 	l.fW = d.fW; l.fH = d.fH;
 	l.scissorOn = d.scissorOn;
+	auto shift = [](int v) { int s = 0; while ((1 << s) < v) ++s; return (1 << s) == v ? s : -1; };
+	l.tileShiftX = shift(d.tileW); l.tileShiftY = shift(d.tileH);
 	return l; }
 
-__device__ inline void load_lite(DrawLite* dl, const DrawDesc* draws, int nDraws) {
-	for (int k = threadIdx.x; k < nDraws; k += blockDim.x) dl[k] = make_lite(draws[k]); }
+// the compact draw table into LDS
+__device__ inline void load_lite(DrawLite* dl, const DrawLite* __restrict__ lite, int nDraws) {
+	static_assert(sizeof(DrawLite) % 16 == 0, "copied in 16-byte words");
+	const int n = nDraws * static_cast<int>(sizeof(DrawLite) / 16);
+	for (int k = threadIdx.x; k < n; k += blockDim.x) reinterpret_cast<uint4*>(dl)[k] = reinterpret_cast<const uint4*>(lite)[k]; }
 
 // LDS table of the frames' first tiles (n + 1 entries, the last = total)
 __device__ inline void load_tile_bases(int* ftb, const BatchDesc& b) {
@@ -159,9 +165,9 @@ template <class P>
 __device__ inline void vertex_one(const DrawDesc& d, long long gi, float4* __restrict__ vpos, uint8_t* __restrict__ vflags,
                                   float* __restrict__ vvary, int varyStride) {
 	if (d.program != P::kId) return;
-	const long long i = gi - d.vBase;
-	const int iid = static_cast<int>(i / d.verts);
-	const int v = static_cast<int>(i - static_cast<long long>(iid) * d.verts);
+	const uint32_t i = static_cast<uint32_t>(gi - d.vBase);   // below 65536 instances of 32768 vertices
+	const int iid = static_cast<int>(i / static_cast<uint32_t>(d.verts));
+	const int v = static_cast<int>(i - static_cast<uint32_t>(iid) * static_cast<uint32_t>(d.verts));
 	float pos[4], vo[P::kVary];
 	P::vertex(d, iid, v, pos, vo);
 	// ViewFrustum::Test, SIMD form with cmple (rglv_view_frustum.hxx:60-73)
@@ -206,7 +212,7 @@ __device__ inline uint2 pack_rect(int tx0, int ty0, int tx1, int ty1) {
 	                  static_cast<uint32_t>(ty0) | (static_cast<uint32_t>(ty1) << 16)); }
 __device__ inline const uint2 empty_rect() { return make_uint2(0x0000ffffu, 0x0000ffffu); }
 
-__global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawDesc* __restrict__ draws, BatchDesc b,
+__global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawLite* __restrict__ lite, BatchDesc b,
 		const float4* __restrict__ vpos, const uint8_t* __restrict__ vflags,
 		uint2* __restrict__ trect, uint4* __restrict__ tvert, uint32_t* __restrict__ tileCount,
 		uint32_t* __restrict__ clipq, uint32_t* __restrict__ clipqOf, uint32_t clipCap,
@@ -216,7 +222,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawDesc* __
 	DrawLite* dl = reinterpret_cast<DrawLite*>(dyn_lds);
 	uint32_t* lhist = reinterpret_cast<uint32_t*>(dl + b.nDraws);
 	const int u = blockIdx.x;
-	load_lite(dl, draws, b.nDraws);
+	load_lite(dl, lite, b.nDraws);
 	__syncthreads();
 	const TileWindow win = unit_window(dl, b, u);
 	if (win.n > b.unitWindow) {   // the host's window bound disagrees: flag it, touch nothing
@@ -236,9 +242,9 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawDesc* __
 		if (!q.live) return;
 		q.di = find_draw_ll(dl, b.nDraws, q.s);
 		const DrawLite& d = dl[q.di];
-		const long long n = q.s - d.triBase;
-		const int iid = static_cast<int>(n / d.tris);
-		const int t = static_cast<int>(n - static_cast<long long>(iid) * d.tris);
+		const uint32_t n = static_cast<uint32_t>(q.s - d.triBase);   // slots, 7 per triangle, fit 32 bits
+		const int iid = static_cast<int>(n / static_cast<uint32_t>(d.tris));
+		const int t = static_cast<int>(n - static_cast<uint32_t>(iid) * static_cast<uint32_t>(d.tris));
 		for (int k = 0; k < 3; ++k) q.ii[k] = d.elements ? d.indices[3 * t + k] : static_cast<uint32_t>(3 * t + k);
 		q.vb = d.vBase + static_cast<long long>(iid) * d.verts; };
 	auto vertices = [&](Tri& q) {
@@ -278,8 +284,8 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawDesc* __
 				const int32_t vmaxy = imin(wadd(imax(iy0, imax(iy1, iy2)), 1), d.scissor[3] - 1);
 				const bool notCulled = front ? d.keepFronts != 0 : d.keepBacks != 0;
 				if (notCulled && vmaxx > vminx && vmaxy > vminy) {
-					const int tx0 = vminx / d.tileW, ty0 = vminy / d.tileH;
-					const int tx1 = vmaxx / d.tileW, ty1 = vmaxy / d.tileH;
+					const int tx0 = tile_of(vminx, d.tileW, d.tileShiftX), ty0 = tile_of(vminy, d.tileH, d.tileShiftY);
+					const int tx1 = tile_of(vmaxx, d.tileW, d.tileShiftX), ty1 = tile_of(vmaxy, d.tileH, d.tileShiftY);
 					rect = pack_rect(tx0, ty0, tx1, ty1);
 					// backface reorder (:634-637); the 0x8000 flag is not needed
 					const uint32_t g0 = static_cast<uint32_t>(vb + (front ? ii[0] : ii[2]));
@@ -1370,7 +1376,7 @@ __device__ inline void resolve_draw(const FrameDesc& f, const RasterArgs& a, con
                                     int x, int y, uint32_t slot, const uint32_t* rcpTab, float col[3], float& dep, uint32_t& prim) {
 	const uint32_t rel = slot - d.slotBase;
 	const uint32_t nTri = static_cast<uint32_t>(d.tris) * static_cast<uint32_t>(d.instances);
-	const int tx = x / f.tileW, ty = y / f.tileH;
+	const int tx = tile_of(x, f.tileW, f.tileShiftX), ty = tile_of(y, f.tileH, f.tileShiftY);
 	Rect R;
 	R.x0 = tx * f.tileW; R.y0 = ty * f.tileH;
 	R.x1 = imin(R.x0 + f.tileW, f.W); R.y1 = imin(R.y0 + f.tileH, f.H);
@@ -1528,7 +1534,8 @@ __global__ __launch_bounds__(256, kResolveWaves<S>) void k_resolve(BatchDesc b, 
 		lo = __popcll(__ballot(base <= blk)) - 1;
 		const FrameDesc& f = frames[lo];
 		const int lb = blk - f.blockBase;
-		by = lb / f.blocksX; bx = lb - by * f.blocksX;
+		by = f.blocksMagic ? static_cast<int>(__umulhi(static_cast<uint32_t>(lb), f.blocksMagic)) : lb / f.blocksX;
+		bx = lb - by * f.blocksX;
 		if (b.skipEmpty && f.shiftX >= 0) tile = f.tileBase + ((by * kResolveH) >> f.shiftY) * f.tilesX + ((bx * kResolveW) >> f.shiftX); }
 	const FrameDesc f = frames[lo];
 	const int x = bx * kResolveW + static_cast<int>(threadIdx.x % kResolveW);
@@ -1674,9 +1681,8 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 					vis_quad(keys, w, q1, q2, q3, w.x0 + 2 * kx, w.y0 + 2 * ky, leq, frags); }}
 			__syncthreads(); }
 		// merge the region into the frame's key buffer
-		const int rw = S.x1 - S.x0, rh = S.y1 - S.y0;
-		for (int i = threadIdx.x; i < rw * rh; i += kRasterThreads) {
-			const int ly = i / rw, lx = i - ly * rw;
+		const int rw = S.x1 - S.x0, rh = S.y1 - S.y0, lx = static_cast<int>(threadIdx.x) % kSubDim;
+		for (int ly = static_cast<int>(threadIdx.x) / kSubDim; lx < rw && ly < rh; ly += kRasterThreads / kSubDim) {
 			const unsigned long long k = keys[ly * kSubDim + lx];
 			unsigned long long* dst = a.keys + f.keyBase + static_cast<long long>(S.y0 + ly) * f.W + S.x0 + lx;
 			if (!multiSeg) *dst = k;

@@ -315,7 +315,7 @@ __device__ inline bool resolve_inputs(const BatchDesc& b, const FrameDesc& f, co
 	const DrawLite& dd = dl[di];
 	const uint32_t rel = slot - dd.slotBase;
 	const uint32_t nTri = static_cast<uint32_t>(dd.tris) * static_cast<uint32_t>(dd.instances);
-	const int tx = x / f.tileW, ty = y / f.tileH;
+	const int tx = tile_of(x, f.tileW, f.tileShiftX), ty = tile_of(y, f.tileH, f.tileShiftY);
 	Rect R;
 	R.x0 = tx * f.tileW; R.y0 = ty * f.tileH;
 	R.x1 = imin(R.x0 + f.tileW, f.W); R.y1 = imin(R.y0 + f.tileH, f.H);
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void k_mlp_gather(BatchDesc b, RasterArgs a, f
 	DrawLite* dl = reinterpret_cast<DrawLite*>(dyn_lds);
 	__shared__ int fbb[kMaxFrames + 1];
 	const int blk = static_cast<int>(blockIdx.x);
-	load_lite(dl, a.draws, b.nDraws);
+	load_lite(dl, a.lite, b.nDraws);
 	if (blk < probeBlocks) load_tile_bases(fbb, b);
 	else load_block_bases(fbb, b);
 	__syncthreads();
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(256) void k_mlp_fallback(BatchDesc b, RasterArgs a,
 	const int per = subX * subY;
 	const uint32_t item = blockIdx.x / static_cast<uint32_t>(per);
 	if (item >= *count) return;   // uniform over the block
-	load_lite(dl, a.draws, b.nDraws);
+	load_lite(dl, a.lite, b.nDraws);
 	load_tile_bases(ftb, b);
 	__syncthreads();
 	const uint32_t id = list[item];
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(256) void k_mlp_samples(BatchDesc b, RasterArgs a, 
 	extern __shared__ uint4 dyn_lds[];   // the batch's draws
 	DrawLite* dl = reinterpret_cast<DrawLite*>(dyn_lds);
 	__shared__ int fbb[kMaxFrames + 1];
-	load_lite(dl, a.draws, b.nDraws);
+	load_lite(dl, a.lite, b.nDraws);
 	load_block_bases(fbb, b);
 	__syncthreads();
 	const BlockPixel bp = block_pixel(b, fbb);

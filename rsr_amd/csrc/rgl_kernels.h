@@ -383,6 +383,16 @@ __device__ inline uint32_t vis_regions(const BatchDesc& b, uint32_t cost, uint32
 	const uint32_t per = cost / (nseg * kQuadrants), s = static_cast<uint32_t>(b.splitQuads);
 	return per > 2 * s ? 4 * kQuadrants : per > s ? 2 * kQuadrants : kQuadrants; }
 
+// The work items of a tile of `pairs` records: none where it needs no keys
+// (no record, and the resolve tells so from the tile's bit).  A workgroup
+// that starts only to find its tile empty still costs its launch, the item's
+// and the tile's loads and the region's arithmetic: in four 4096^2 frames
+// two of three tiles are empty, and k_vis takes 238 us without their items
+// (265 with them, of which a part is the descriptor's: frame, regions and
+// tile position come ready, with no division an item).
+__device__ inline uint32_t vis_items(const BatchDesc& b, const FrameDesc& f, uint32_t pairs, uint32_t nseg, uint32_t nreg) {
+	return pairs == 0u && b.skipEmpty && f.shiftX >= 0 ? 0u : nseg * nreg; }
+
 constexpr int kCostClasses = 33;   // cost 0, then [2^(c-1), 2^c) for c = 1 .. 32
 constexpr int kScanSplitTiles = 2 * kScanThreads;   // tiles above which the scan takes three launches
 __device__ inline int cost_class(uint32_t cost) { return cost ? 32 - __clz(cost) : 0; }
@@ -392,12 +402,17 @@ __device__ inline int cost_class(uint32_t cost) { return cost ? 32 - __clz(cost)
 // chain of table lookups.
 struct alignas(16) VisTile {
 	uint32_t item0;        // the tile's first work item
-	uint32_t frame;
+	uint32_t flags;        // frame | log2(regions per segment) << 8 | several segments (regions merge with atomic min) << 12
 	uint32_t ib, cb;       // the tile's first inline and clipped records (clamped to the capacities)
 	uint32_t ninl, ntot;   // the tile's inline records, and inline + clipped
-	uint32_t nreg;         // regions per segment
-	uint32_t multiSeg;     // 1: the tile has several segments (regions merge with atomic min)
+	uint32_t xy;           // its column | row << 16 in the frame's tile grid
+	uint32_t pad;
 };
+__device__ inline uint32_t vis_flags(uint32_t frame, uint32_t nreg, uint32_t nseg) {
+	return frame | (static_cast<uint32_t>(31 - __clz(nreg)) << 8) | ((nseg > 1 ? 1u : 0u) << 12); }
+__device__ inline uint32_t tile_xy(const FrameDesc& f, int tile) {
+	const int ty = tile / f.tilesX;
+	return static_cast<uint32_t>(tile - ty * f.tilesX) | (static_cast<uint32_t>(ty) << 16); }
 static_assert(sizeof(VisTile) == 32, "two 16-byte loads");
 
 // One block: per tile the list offset (exclusive scan of the tiles' pair
@@ -431,6 +446,7 @@ __device__ inline void col_scan_block(const BatchDesc& b, const uint32_t* __rest
 		if (it * kThreads >= nT) break;   // uniform: no tile left for any thread
 		const int t = it * kThreads + threadIdx.x;
 		uint32_t col = 0, v = 0, items = 0, nseg = 1, nreg = kQuadrants, cost = 0;
+		int fr = 0;
 		uint32_t grp[kCountGroups];
 #pragma unroll
 		for (int g = 0; g < kCountGroups; ++g) {
@@ -441,7 +457,8 @@ __device__ inline void col_scan_block(const BatchDesc& b, const uint32_t* __rest
 			cost = o.tileCost[t];
 			nseg = vis_segments(b, col + v);
 			nreg = vis_regions(b, cost, nseg);
-			items = nseg * nreg;
+			fr = find_base(ftb, b.nFrames, t);
+			items = vis_items(b, b.frames[fr], col + v, nseg, nreg);
 			o.tileCost[t] = 0u; }
 		uint32_t tot, ctot;
 		const uint32_t ex = block_exclusive_scan(col, sh, tot);
@@ -457,13 +474,13 @@ __device__ inline void col_scan_block(const BatchDesc& b, const uint32_t* __rest
 			if (o.clipCursor) o.clipCursor[t] = ccarry + cex;
 			VisTile& d = mine[it];
 			d.item0 = items;   // the item count until the ordering below
-			d.frame = static_cast<uint32_t>(find_base(ftb, b.nFrames, t));
+			d.flags = vis_flags(static_cast<uint32_t>(fr), nreg, nseg);
+			d.xy = tile_xy(b.frames[fr], t - b.frames[fr].tileBase);
+			d.pad = 0u;
 			d.ib = min(carry + ex, o.listCap);
 			d.cb = min(ccarry + cex, o.clistCap);
 			d.ninl = min(carry + ex + col, o.listCap) - d.ib;
 			d.ntot = d.ninl + (min(ccarry + cex + v, o.clistCap) - d.cb);
-			d.nreg = nreg;
-			d.multiSeg = nseg > 1 ? 1u : 0u;
 			atomicAdd(&classItems[mcls[it]], items); }
 		carry += tot; ccarry += ctot; }
 	// Work-item order: by the tiles' previous-frame quad work, heaviest
@@ -539,13 +556,15 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_local(BatchDesc b, const 
 		tileCost[t] = 0u;
 		const uint32_t nseg = vis_segments(b, col + v), nreg = vis_regions(b, cost, nseg);
 		const int cls = cost_class(cost);
-		atomicAdd(&classItems[cls], nseg * nreg);
-		VisTile d;   // provisional: local prefixes, counts and the cost class
-		d.item0 = nseg * nreg;
-		d.frame = static_cast<uint32_t>(find_base(ftb, b.nFrames, t));
+		const int fr = find_base(ftb, b.nFrames, t);
+		const FrameDesc& f = b.frames[fr];
+		VisTile d;   // provisional: local prefixes, counts and (pad) the cost class
+		d.item0 = vis_items(b, f, col + v, nseg, nreg);
+		atomicAdd(&classItems[cls], d.item0);
+		d.flags = vis_flags(static_cast<uint32_t>(fr), nreg, nseg);
 		d.ib = ex; d.cb = cex; d.ninl = col; d.ntot = v;
-		d.nreg = nreg;
-		d.multiSeg = (nseg > 1 ? 1u : 0u) | (static_cast<uint32_t>(cls) << 1);
+		d.xy = tile_xy(f, t - f.tileBase);
+		d.pad = static_cast<uint32_t>(cls);
 		tileDesc[t] = d; }
 	__syncthreads();
 	ScanPart& P = part[blockIdx.x];
@@ -601,14 +620,13 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_final(BatchDesc b, const 
 		tileCursor[static_cast<long long>(g) * nT + t] = run;
 		run += tileCount[static_cast<long long>(g) * nT + t]; }
 	clipOff[t] = coff; clipCursor[t] = coff;
-	const uint32_t item0 = atomicAdd(&classCursor[d.multiSeg >> 1], items);
+	const uint32_t item0 = atomicAdd(&classCursor[d.pad], items);
 	for (uint32_t j = item0, je = min(j + items, itemCap); j < je; ++j) itemTile[j] = static_cast<uint32_t>(t);
 	d.item0 = item0;
 	d.ib = min(off, listCap);
 	d.cb = min(coff, clistCap);
 	d.ninl = min(off + col, listCap) - d.ib;
 	d.ntot = d.ninl + (min(coff + v, clistCap) - d.cb);
-	d.multiSeg &= 1u;
 	tileDesc[t] = d;
 	const unsigned long long bits = __ballot(d.ntot != 0u);   // lanes past the last tile have left
 	if ((threadIdx.x & 63u) == 0) tileBits[t >> 6] = bits; }
@@ -1581,17 +1599,18 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 		const uint32_t item = wi < full ? wi / kGroup * kGroup + (wi % kXcds) * 4u + (wi / kXcds) % 4u : wi;
 		const int tile = static_cast<int>(itemTile[item]);
 		const VisTile it = tileDesc[tile];
-		const uint32_t local = item - it.item0;
-		const uint32_t nreg = it.nreg, seg = local / nreg, reg = local - seg * nreg;
-		const bool multiSeg = it.multiSeg != 0u;
+		const uint32_t local = item - it.item0, regShift = (it.flags >> 8) & 15u;
+		const uint32_t seg = local >> regShift, reg = local & ((1u << regShift) - 1u);
+		const bool multiSeg = (it.flags >> 12) != 0u;
 		// the frame table is read-only (restrict): its fields come by scalar loads
-		const FrameDesc& f = frames[it.frame];
+		const FrameDesc& f = frames[it.flags & 0xffu];
 		if (f.inOrder) continue;   // drawn by the in-order tile path (uniform)
-		if (it.ntot == 0u && b.skipEmpty && f.shiftX >= 0) continue;   // resolved without keys (uniform)
 		const bool leq = f.depthFunc == 1;
-		const Rect R = tile_rect(f, tile - f.tileBase);
+		Rect R;
+		R.x0 = static_cast<int>(it.xy & 0xffffu) * f.tileW; R.y0 = static_cast<int>(it.xy >> 16) * f.tileH;
+		R.x1 = imin(R.x0 + f.tileW, f.W); R.y1 = imin(R.y0 + f.tileH, f.H);
 		// the item's region: a quadrant, or its half or quarter
-		const uint32_t per = max(1u, nreg / kQuadrants), quad = reg / per, sub = reg - quad * per;
+		const uint32_t perShift = regShift - 2u, per = 1u << perShift, quad = reg >> perShift, sub = reg & (per - 1u);
 		Rect S;
 		S.x0 = R.x0 + static_cast<int>(quad & 1) * kSubDim; S.y0 = R.y0 + static_cast<int>(quad >> 1) * kSubDim;
 		int sw = kSubDim, sh = kSubDim;

@@ -339,24 +339,29 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawLite* __
 // n+1 entries are written: out[n] = total.
 // ---------------------------------------------------------------------------
 
+// inclusive sum over the wave's lanes (all active) with DPP row shifts and
+// row broadcasts: registers only, where shuffles go through the LDS crossbar
+__device__ inline uint32_t wave_inclusive_scan(uint32_t v) {
+	int x = static_cast<int>(v);
+	x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+	x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);   // row_shr:2
+	x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);   // row_shr:4
+	x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);   // row_shr:8
+	x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+	x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+	return static_cast<uint32_t>(x); }
+
 __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* sh, uint32_t& total) {
-	// sh: blockDim.x + 32 entries; Hillis-Steele over waves then lanes
+	// sh: an entry per wave; every thread of the block calls it
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-	uint32_t x = v;
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t y = __shfl_up(x, o, 64);
-		if (lane >= o) x += y; }
+	const uint32_t x = wave_inclusive_scan(v);
 	if (lane == 63) sh[wave] = x;
 	__syncthreads();
-	if (threadIdx.x == 0) {
-		uint32_t acc = 0;
-		for (int w = 0; w < nw; ++w) { const uint32_t t = sh[w]; sh[w] = acc; acc += t; }
-		sh[nw] = acc; }
+	uint32_t base = 0, sum = 0;
+	for (int w = 0; w < nw; ++w) { const uint32_t t = sh[w]; base += w < wave ? t : 0u; sum += t; }
 	__syncthreads();
-	const uint32_t r = sh[wave] + x - v;
-	total = sh[nw];
-	__syncthreads();
-	return r; }
+	total = sum;
+	return base + x - v; }
 
 // The list is tile-major: tile t's inline pairs take list positions
 // [tileOff[t], tileOff[t + 1]), laid out by count group (the units u with
@@ -1229,45 +1234,48 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 // region into the per-pixel key buffer: a plain store when the tile is one
 // segment, a 64-bit atomic min otherwise.
 // ---------------------------------------------------------------------------
-struct alignas(16) VisSetup {
-	int32_t c1, c2, c3;   // edge values at the triangle's first quad in the quadrant
-	int32_t x0, y0;       // that quad's top-left pixel, quadrant-relative
-	int32_t dx12, dy12, dx23, dy23, dx31, dy31;
-	uint32_t nx;          // quads across inside the quadrant
-	float invNx;          // 1 / nx: row = floor((k + 0.5) / nx), exact for k < 2^16
-	float scale;
-	float z0, z1, z2;
-	uint32_t slot;
-	uint32_t small;       // 1: every quad step fits 23 bits, 24-bit multiplies are exact
-	uint32_t pad;
-};
-static_assert(sizeof(VisSetup) % 16 == 0, "VisSetup rows are read with aligned 16-byte loads");
+constexpr int kQuadWindow = 2048;   // quads mapped to their triangle per pass
+constexpr int kCullSpan = 2048;     // records tested against the region per pass
 
-
-constexpr int kQuadWindow = 2048;   // quad items mapped to their triangle per pass
+// A record prepared for a region, as the quad loop reads it: one of four
+// 16-byte columns per table, so that lanes of neighbouring triangles read
+// neighbouring addresses.
+//   0: edge values at the triangle's first quad in the region, and packed
+//      that quad's x | y << 6 in the region | quads across << 12 | its first
+//      quad's number (mod 2^15) << 17
+//   1: dx12 dy12 dx23 dy23   2: dx31 dy31 1/across scale   3: z0 z1 z2 slot
+struct VisRows { uint4 c[4][kRasterThreads]; };
 
 __device__ inline VisRec vis_record(const VisRec* __restrict__ rec, const VisRec* __restrict__ crec, uint32_t ib, uint32_t cb,
                                     uint32_t ninl, uint32_t p) {
 	return p < ninl ? rec[ib + p] : crec[cb + (p - ninl)]; }
+// the record's box alone (minxy, nq)
+__device__ inline uint2 vis_box(const VisRec* __restrict__ rec, const VisRec* __restrict__ crec, uint32_t ib, uint32_t cb,
+                                uint32_t ninl, uint32_t p) {
+	const VisRec* r = p < ninl ? rec + ib + p : crec + cb + (p - ninl);
+	return make_uint2(r->minxy, r->nq); }
 
 // one quad of a triangle: the four lanes (c, c+dy, c+dx, c+dx+dy)
 // (rglv_triangle.hxx:253-258) with their depth keys merged by a 64-bit LDS
-// min; q1..q3 are the edge values at the quad's top-left pixel (lx, ly),
-// quadrant-relative
-__device__ inline void vis_quad(unsigned long long* keys, const VisSetup& v, int32_t q1, int32_t q2, int32_t q3,
-                                int lx, int ly, bool leq, uint32_t& frags) {
+// min; q1..q3 are the edge values at the quad's top-left pixel, whose key
+// `k0` is.  Returns the wave's covered fragments.
+struct VisSteps { int32_t dx12, dy12, dx23, dy23, dx31, dy31; };
+__device__ inline uint32_t vis_quad(unsigned long long* k0, const VisSteps& v, float scale, float z0, float z1, float z2, uint32_t slot,
+                                    int32_t q1, int32_t q2, int32_t q3, bool leq, bool active) {
+	uint32_t frags = 0;
 #pragma unroll
 	for (int l = 0; l < 4; ++l) {
 		const int32_t e1 = (l & 2) ? wadd((l & 1) ? wadd(q1, v.dx12) : q1, (l & 1) ? v.dy12 : v.dx12) : ((l & 1) ? wadd(q1, v.dy12) : q1);
 		const int32_t e2 = (l & 2) ? wadd((l & 1) ? wadd(q2, v.dx23) : q2, (l & 1) ? v.dy23 : v.dx23) : ((l & 1) ? wadd(q2, v.dy23) : q2);
 		const int32_t e3 = (l & 2) ? wadd((l & 1) ? wadd(q3, v.dx31) : q3, (l & 1) ? v.dy31 : v.dx31) : ((l & 1) ? wadd(q3, v.dy31) : q3);
-		const bool cov = (e1 | e2 | e3) >= 0;
-		frags += cov ? 1u : 0u;
-		const float bx = itof(e2) * v.scale;
-		const float bz = itof(e1) * v.scale;
+		const bool cov = active && (e1 | e2 | e3) >= 0;
+		frags += static_cast<uint32_t>(__popcll(__ballot(cov)));
+		const float bx = itof(e2) * scale;
+		const float bz = itof(e1) * scale;
 		const float by = (1.0F - bx) - bz;
-		const float dz = (bx*v.z0 + by*v.z1) + bz*v.z2;
-		if (cov && dz == dz) atomicMin(&keys[(ly + (l >> 1)) * kSubDim + (lx + (l & 1))], frag_key(dz, v.slot, leq)); }}
+		const float dz = (bx*z0 + by*z1) + bz*z2;
+		if (cov && dz == dz) atomicMin(&k0[(l >> 1) * kSubDim + (l & 1)], frag_key(dz, slot, leq)); }
+	return frags; }
 
 // one lane of a quad of a triangle setup: perspective-correct barycentrics
 // BP and depth (TriangleProgram::Render, rglv_gpu_impl.hxx:169-191)
@@ -1581,11 +1589,17 @@ __global__ __launch_bounds__(256, kResolveWaves<S>) void k_resolve(BatchDesc b, 
 __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs a, const VisRec* __restrict__ rec,
                                                        const VisRec* __restrict__ crec, const uint32_t* __restrict__ itemTile,
                                                        const VisTile* __restrict__ tileDesc, const FrameDesc* __restrict__ frames) {
+	constexpr int kWords = kQuadWindow / 64;
 	__shared__ unsigned long long keys[kSubDim * kSubDim];
-	__shared__ VisSetup ts[kRasterThreads];
-	__shared__ uint32_t qoff[kRasterThreads + 1];
-	__shared__ uint32_t scan_sh[kRasterThreads / 64 + 1];
-	__shared__ uint8_t owner[kQuadWindow];
+	__shared__ VisRows rows;
+	__shared__ unsigned long long starts[2][kWords];   // per 64 quads: bit q - 1 set where a triangle's quads begin at q > 0
+	__shared__ uint8_t first[kWords];                  // per 64 quads: the row of the first one's triangle
+	__shared__ uint32_t waveSum[2][kRasterThreads / 64];
+	__shared__ uint32_t waveRows[2][kRasterThreads / 64];
+	__shared__ uint32_t nList;
+	__shared__ uint16_t list[kCullSpan];
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	if (threadIdx.x < 2 * kWords) (&starts[0][0])[threadIdx.x] = 0;
 	uint32_t frags = 0;
 	const uint32_t nItems = a.ctr->workItems;
 	// Workgroups are dealt round-robin over the eight XCDs.  A tile's items
@@ -1620,85 +1634,134 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 		if (S.x0 >= S.x1 || S.y0 >= S.y1) continue;   // region outside the screen (uniform)
 		for (int i = threadIdx.x; i < kSubDim * kSubDim; i += kRasterThreads) keys[i] = kKeySentinel;
 		const uint32_t ib = it.ib, cb = it.cb, ninl = it.ninl, ntot = it.ntot;
-		const uint32_t pbeg = seg * static_cast<uint32_t>(b.segPairs), pend = min(pbeg + static_cast<uint32_t>(b.segPairs), ntot);
+		const uint32_t pbeg = seg * static_cast<uint32_t>(b.segPairs);
+		const uint32_t pend = f.drawEnabled ? min(pbeg + static_cast<uint32_t>(b.segPairs), ntot) : pbeg;
 		uint32_t itemQuads = 0;   // quads dealt out over the workgroup: the item's cost for the next frame's split
-		__syncthreads();
-		// each thread holds one pair's record; the next batch's record is
-		// loaded while this batch rasterises
-		VisRec rn;
-		if (f.drawEnabled && pbeg + threadIdx.x < pend) rn = vis_record(rec, crec, ib, cb, ninl, pbeg + threadIdx.x);
-		for (uint32_t b0 = pbeg; f.drawEnabled && b0 < pend; b0 += kRasterThreads) {
-			const uint32_t p = b0 + threadIdx.x;
-			const VisRec r = rn;
-			if (p + kRasterThreads < pend) rn = vis_record(rec, crec, ib, cb, ninl, p + kRasterThreads);
-			uint32_t nq = 0;
-			VisSetup v;
-			if (p < pend) {
-				const int minx = static_cast<int>(r.minxy & 0xffffu), miny = static_cast<int>(r.minxy >> 16);
-				const int nqx = static_cast<int>(r.nq & 0xffffu), nqy = static_cast<int>(r.nq >> 16);
-				// the triangle's quads inside the quadrant
-				const int kx0 = imax(0, (S.x0 - minx) >> 1), ky0 = imax(0, (S.y0 - miny) >> 1);
-				const int kx1 = imin(nqx, (S.x1 - minx + 1) >> 1), ky1 = imin(nqy, (S.y1 - miny + 1) >> 1);
-				const int nx = imax(0, kx1 - kx0), ny = imax(0, ky1 - ky0);
-				// edge values at the first quad, stepped exactly as the rasteriser loops do
-				v.c1 = wadd(wadd(r.c1, wmul(kx0, wmul(r.dy12, 2))), wmul(ky0, wmul(r.dx12, 2)));
-				v.c2 = wadd(wadd(r.c2, wmul(kx0, wmul(r.dy23, 2))), wmul(ky0, wmul(r.dx23, 2)));
-				v.c3 = wadd(wadd(r.c3, wmul(kx0, wmul(r.dy31, 2))), wmul(ky0, wmul(r.dx31, 2)));
-				v.dx12 = r.dx12; v.dy12 = r.dy12; v.dx23 = r.dx23; v.dy23 = r.dy23; v.dx31 = r.dx31; v.dy31 = r.dy31;
-				const int32_t lim = 1 << 21;   // 2 * |d| < 2^22
-				v.small = (r.dx12 > -lim && r.dx12 < lim && r.dy12 > -lim && r.dy12 < lim &&
-				           r.dx23 > -lim && r.dx23 < lim && r.dy23 > -lim && r.dy23 < lim &&
-				           r.dx31 > -lim && r.dx31 < lim && r.dy31 > -lim && r.dy31 < lim) ? 1u : 0u;
-				v.pad = 0u;
-				v.x0 = minx + 2 * kx0 - S.x0; v.y0 = miny + 2 * ky0 - S.y0;
-				v.nx = static_cast<uint32_t>(nx);
-				v.invNx = nx > 0 ? 1.0F / static_cast<float>(nx) : 0.0F;
-				v.scale = r.scale; v.z0 = r.z0; v.z1 = r.z1; v.z2 = r.z2; v.slot = r.slot;
-				nq = static_cast<uint32_t>(nx) * static_cast<uint32_t>(ny); }
-			// the triangles' quads are dealt out over the block
-			const bool coop = nq != 0u;
-			if (coop) ts[threadIdx.x] = v;
-			// 24-bit step products are exact when every dealt-out triangle's
-			// steps fit 23 bits (nearly always); decided for the whole batch
-			// so that the quad loop does not diverge on it
-			const bool allSmall = __syncthreads_and(!coop || v.small != 0u) != 0;
-			const uint32_t cq = coop ? nq : 0u;
-			uint32_t total;
-			const uint32_t ex = block_exclusive_scan(cq, scan_sh, total);
-			itemQuads += total;
-			qoff[threadIdx.x] = ex;
-			for (uint32_t win0 = 0; win0 < total; win0 += kQuadWindow) {
-				// owner table: which triangle each quad item of the window belongs to
+		uint32_t par = 0;   // the sums' buffer: a round without quads has one barrier only
+		for (uint32_t p0 = pbeg; p0 < pend; p0 += kCullSpan) {
+			// Most records of a dense tile miss the region (four regions read
+			// them all).  Where there are more than one round of them, their
+			// boxes alone are tested first and the rounds are made up of
+			// those that hit; a single round takes them as they are, without
+			// the extra pass.
+			const uint32_t p1 = min(pend, p0 + kCullSpan);
+			uint32_t n = p1 - p0;
+			const bool listed = n > static_cast<uint32_t>(kRasterThreads);
+			if (listed) {
+				if (threadIdx.x == 0) nList = 0;
 				__syncthreads();
-				{
-					const uint32_t s0 = max(ex, win0), s1 = min(ex + cq, win0 + kQuadWindow);
-					for (uint32_t q = s0; q < s1; ++q) owner[q - win0] = static_cast<uint8_t>(threadIdx.x);
-				}
-				__syncthreads();
-				const uint32_t wend = min(total, win0 + kQuadWindow);
-				for (uint32_t it = win0 + threadIdx.x; it < wend; it += kRasterThreads) {
-					const int j = owner[it - win0];
-					// the owner's setup row, read whole into registers
-					VisSetup w;
-					const uint4* src = reinterpret_cast<const uint4*>(&ts[j]);
-					uint4* dstw = reinterpret_cast<uint4*>(&w);
+				for (uint32_t q = p0; q < p1; q += 2 * kRasterThreads) {
+					uint2 bx[2];
 #pragma unroll
-					for (int c = 0; c < static_cast<int>(sizeof(VisSetup) / 16); ++c) dstw[c] = src[c];
-					const uint32_t k = it - qoff[j];
-					const uint32_t kyr = static_cast<uint32_t>((static_cast<float>(k) + 0.5F) * w.invNx);
-					const uint32_t kxr = k - __umul24(kyr, w.nx);
-					const int32_t kx = static_cast<int32_t>(kxr), ky = static_cast<int32_t>(kyr);
-					int32_t q1, q2, q3;
-					if (allSmall) {
-						q1 = wadd(wadd(w.c1, __mul24(kx, shl(w.dy12, 1))), __mul24(ky, shl(w.dx12, 1)));
-						q2 = wadd(wadd(w.c2, __mul24(kx, shl(w.dy23, 1))), __mul24(ky, shl(w.dx23, 1)));
-						q3 = wadd(wadd(w.c3, __mul24(kx, shl(w.dy31, 1))), __mul24(ky, shl(w.dx31, 1))); }
-					else {
-						q1 = wadd(wadd(w.c1, wmul(kx, shl(w.dy12, 1))), wmul(ky, shl(w.dx12, 1)));
-						q2 = wadd(wadd(w.c2, wmul(kx, shl(w.dy23, 1))), wmul(ky, shl(w.dx23, 1)));
-						q3 = wadd(wadd(w.c3, wmul(kx, shl(w.dy31, 1))), wmul(ky, shl(w.dx31, 1))); }
-					vis_quad(keys, w, q1, q2, q3, w.x0 + 2 * kx, w.y0 + 2 * ky, leq, frags); }}
-			__syncthreads(); }
+					for (int u = 0; u < 2; ++u) {
+						const uint32_t p = q + u * kRasterThreads + threadIdx.x;
+						bx[u] = p < p1 ? vis_box(rec, crec, ib, cb, ninl, p) : make_uint2(0u, 0u); }
+#pragma unroll
+					for (int u = 0; u < 2; ++u) {
+						const int minx = static_cast<int>(bx[u].x & 0xffffu), miny = static_cast<int>(bx[u].x >> 16);
+						const int ex = minx + 2 * static_cast<int>(bx[u].y & 0xffffu), ey = miny + 2 * static_cast<int>(bx[u].y >> 16);
+						const bool hit = minx < S.x1 && miny < S.y1 && ex > S.x0 && ey > S.y0;   // no quads: ex = ey = 0
+						const unsigned long long m = __ballot(hit);
+						uint32_t base = 0;
+						if (lane == 0 && m) base = atomicAdd(&nList, static_cast<uint32_t>(__popcll(m)));
+						base = __builtin_amdgcn_readfirstlane(base);
+						if (hit)
+							list[base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u))] =
+								static_cast<uint16_t>(q - p0 + u * kRasterThreads + threadIdx.x); }}
+				__syncthreads();
+				n = nList; }
+			// each thread holds one pair's record; the next round's record is
+			// loaded while this round rasterises
+			VisRec rn;
+			if (threadIdx.x < n) rn = vis_record(rec, crec, ib, cb, ninl, p0 + (listed ? list[threadIdx.x] : threadIdx.x));
+			for (uint32_t b0 = 0; b0 < n; b0 += kRasterThreads, par ^= 1u) {
+				const uint32_t i = b0 + threadIdx.x;
+				const VisRec r = rn;
+				if (i + kRasterThreads < n) rn = vis_record(rec, crec, ib, cb, ninl, p0 + (listed ? list[i + kRasterThreads] : i + kRasterThreads));
+				uint32_t nq = 0, nx = 0, x0 = 0, y0 = 0;
+				int32_t c1 = 0, c2 = 0, c3 = 0;
+				bool small = true;
+				if (i < n) {
+					const int minx = static_cast<int>(r.minxy & 0xffffu), miny = static_cast<int>(r.minxy >> 16);
+					const int nqx = static_cast<int>(r.nq & 0xffffu), nqy = static_cast<int>(r.nq >> 16);
+					// the triangle's quads inside the region
+					const int kx0 = imax(0, (S.x0 - minx) >> 1), ky0 = imax(0, (S.y0 - miny) >> 1);
+					const int kx1 = imin(nqx, (S.x1 - minx + 1) >> 1), ky1 = imin(nqy, (S.y1 - miny + 1) >> 1);
+					nx = static_cast<uint32_t>(imax(0, kx1 - kx0));
+					nq = __umul24(nx, static_cast<uint32_t>(imax(0, ky1 - ky0)));
+					// edge values at the first quad, stepped exactly as the rasteriser loops do
+					c1 = wadd(wadd(r.c1, wmul(2 * kx0, r.dy12)), wmul(2 * ky0, r.dx12));
+					c2 = wadd(wadd(r.c2, wmul(2 * kx0, r.dy23)), wmul(2 * ky0, r.dx23));
+					c3 = wadd(wadd(r.c3, wmul(2 * kx0, r.dy31)), wmul(2 * ky0, r.dx31));
+					const int32_t lim = 1 << 23;
+					small = r.dx12 >= -lim && r.dx12 < lim && r.dy12 >= -lim && r.dy12 < lim &&
+					        r.dx23 >= -lim && r.dx23 < lim && r.dy23 >= -lim && r.dy23 < lim &&
+					        r.dx31 >= -lim && r.dx31 < lim && r.dy31 >= -lim && r.dy31 < lim;
+					x0 = static_cast<uint32_t>(minx + 2 * kx0 - S.x0); y0 = static_cast<uint32_t>(miny + 2 * ky0 - S.y0); }
+				// the triangles' quads are dealt out over the workgroup: a scan
+				// numbers them, a ballot numbers the triangles that have any.
+				// 24-bit step products are exact when every dealt-out
+				// triangle's steps fit 24 bits (nearly always); decided for the
+				// whole round so that the quad loop does not diverge on it
+				const unsigned long long has = __ballot(nq != 0u);
+				const uint32_t incl = wave_inclusive_scan(nq);
+				const bool waveSmall = __ballot(nq != 0u && !small) == 0ull;
+				if (lane == 63) waveSum[par][wave] = incl;
+				if (lane == 0) waveRows[par][wave] = static_cast<uint32_t>(__popcll(has)) | (waveSmall ? 0u : 0x10000u);
+				__syncthreads();
+				uint32_t ex = incl - nq, total = 0, rowBase = 0, flags = 0;
+#pragma unroll
+				for (int w = 0; w < kRasterThreads / 64; ++w) {
+					const uint32_t ts = waveSum[par][w], tr = waveRows[par][w];
+					ex += w < wave ? ts : 0u; total += ts;
+					rowBase += w < wave ? tr & 0xffffu : 0u; flags |= tr; }
+				const bool allSmall = __builtin_amdgcn_readfirstlane(flags) < 0x10000u;
+				total = __builtin_amdgcn_readfirstlane(total);
+				itemQuads += total;
+				const uint32_t row = rowBase + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(has >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(has), 0u));
+				if (nq != 0u) {
+					// 1 / nx: row = floor((k + 0.5) / nx) is off an integer by at
+					// least 0.5 / 17 of at most 17: an approximate reciprocal is exact there
+					rows.c[0][row] = make_uint4(static_cast<uint32_t>(c1), static_cast<uint32_t>(c2), static_cast<uint32_t>(c3),
+					                            x0 | (y0 << 6) | (nx << 12) | (ex << 17));
+					rows.c[1][row] = make_uint4(static_cast<uint32_t>(r.dx12), static_cast<uint32_t>(r.dy12),
+					                            static_cast<uint32_t>(r.dx23), static_cast<uint32_t>(r.dy23));
+					rows.c[2][row] = make_uint4(static_cast<uint32_t>(r.dx31), static_cast<uint32_t>(r.dy31),
+					                            f2u(__builtin_amdgcn_rcpf(static_cast<float>(nx))), f2u(r.scale));
+					rows.c[3][row] = make_uint4(f2u(r.z0), f2u(r.z1), f2u(r.z2), r.slot); }
+				for (uint32_t win0 = 0, buf = 0; win0 < total; win0 += kQuadWindow, buf ^= 1u) {
+					// which triangle each quad of the window belongs to: a bit where one begins, and the row at every 64th
+					if (nq != 0u && ex < win0 + kQuadWindow && ex + nq > win0) {
+						if (ex >= win0 && (ex & 63u)) atomicOr(&starts[buf][(ex - win0) >> 6], 1ull << ((ex & 63u) - 1u));
+						const uint32_t w1 = min(ex + nq - win0 - 1u, kQuadWindow - 1u) >> 6;
+						for (uint32_t w = ex > win0 ? (ex - win0 + 63u) >> 6 : 0u; w <= w1; ++w) first[w] = static_cast<uint8_t>(row); }
+					__syncthreads();
+					const uint32_t left = min(total - win0, static_cast<uint32_t>(kQuadWindow));
+					for (uint32_t w = wave; w * 64u < left; w += kRasterThreads / 64) {
+						const unsigned long long st = starts[buf][w];
+						const uint32_t j = first[w] + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(st >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(st), 0u));
+						const uint4 r0 = rows.c[0][j], r1 = rows.c[1][j], r2 = rows.c[2][j], r3 = rows.c[3][j];
+						const uint32_t k = (win0 + w * 64u + lane - (r0.w >> 17)) & 0x7fffu;
+						const uint32_t ky = static_cast<uint32_t>((static_cast<float>(k) + 0.5F) * u2f(r2.z));
+						const uint32_t kx = k - __umul24(ky, (r0.w >> 12) & 31u);
+						const int32_t kx2 = static_cast<int32_t>(kx * 2u), ky2 = static_cast<int32_t>(ky * 2u);
+						const VisSteps d{ static_cast<int32_t>(r1.x), static_cast<int32_t>(r1.y), static_cast<int32_t>(r1.z), static_cast<int32_t>(r1.w),
+						                  static_cast<int32_t>(r2.x), static_cast<int32_t>(r2.y) };
+						int32_t q1 = static_cast<int32_t>(r0.x), q2 = static_cast<int32_t>(r0.y), q3 = static_cast<int32_t>(r0.z);
+						if (allSmall) {
+							q1 = wadd(wadd(q1, __mul24(kx2, d.dy12)), __mul24(ky2, d.dx12));
+							q2 = wadd(wadd(q2, __mul24(kx2, d.dy23)), __mul24(ky2, d.dx23));
+							q3 = wadd(wadd(q3, __mul24(kx2, d.dy31)), __mul24(ky2, d.dx31)); }
+						else {
+							q1 = wadd(wadd(q1, wmul(kx2, d.dy12)), wmul(ky2, d.dx12));
+							q2 = wadd(wadd(q2, wmul(kx2, d.dy23)), wmul(ky2, d.dx23));
+							q3 = wadd(wadd(q3, wmul(kx2, d.dy31)), wmul(ky2, d.dx31)); }
+						const uint32_t px = (r0.w & 63u) + static_cast<uint32_t>(kx2), py = ((r0.w >> 6) & 63u) + static_cast<uint32_t>(ky2);
+						frags += vis_quad(&keys[py * kSubDim + px], d, u2f(r2.w), u2f(r3.x), u2f(r3.y), u2f(r3.z), r3.w, q1, q2, q3, leq,
+						                  w * 64u + lane < left); }
+					__syncthreads();
+					if (threadIdx.x < kWords) starts[buf][threadIdx.x] = 0; }}}
+		__syncthreads();
 		// merge the region into the frame's key buffer
 		const int rw = S.x1 - S.x0, rh = S.y1 - S.y0, lx = static_cast<int>(threadIdx.x) % kSubDim;
 		for (int ly = static_cast<int>(threadIdx.x) / kSubDim; lx < rw && ly < rh; ly += kRasterThreads / kSubDim) {
@@ -1707,13 +1770,12 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 			if (!multiSeg) *dst = k;
 			else if (k != kKeySentinel) atomicMin(dst, k); }
 		if (threadIdx.x == 0 && itemQuads) atomicAdd(&a.tileCost[tile], itemQuads); }
-	for (int o = 32; o > 0; o >>= 1) frags += __shfl_xor(frags, o, 64);
 	__syncthreads();
-	if ((threadIdx.x & 63) == 0) scan_sh[threadIdx.x >> 6] = frags;
+	if (lane == 0) waveRows[0][wave] = frags;
 	__syncthreads();
 	if (threadIdx.x == 0) {
 		unsigned long long sum = 0;
-		for (int w = 0; w < kRasterThreads / 64; ++w) sum += scan_sh[w];
+		for (int w = 0; w < kRasterThreads / 64; ++w) sum += waveRows[0][w];
 		if (sum) atomicAdd(&a.ctr->slot[blockIdx.x % kCtrSlots].fragments, sum); }}
 
 __global__ void k_fill_u32(uint32_t* p, long long n, uint32_t v) {

@@ -217,9 +217,28 @@ __device__ inline void xform3w0(const float* f, const float b[3], float o[3]) {
 	o[1] = (f[1]*b[0] + f[5]*b[1]) + f[ 9]*b[2];
 	o[2] = (f[2]*b[0] + f[6]*b[1]) + f[10]*b[2]; }
 
+// 1 / x and 1 / sqrt(x), correctly rounded as the operators are, in a
+// third of their instructions: the compiler's expansions scale and fix up
+// for the whole range of exponents, these correct the hardware's estimate
+// by FMAs where no step can leave the normal range and take the operators
+// elsewhere (zero, subnormal, huge, infinite, NaN).  Compared with the
+// operators for each of the 2^31 floats of one sign: no difference for
+// 2^-126 <= x < 2^126 and 2^-102 <= x respectively.
+__device__ inline float recip(float x) {
+	if (__builtin_expect(!(__builtin_fabsf(x) >= 0x1p-126F && __builtin_fabsf(x) < 0x1p126F), 0)) return 1.0F / x;
+	const float y = __builtin_amdgcn_rcpf(x);
+	return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0F), y, y); }
+
+__device__ inline float recip_sqrt(float x) {
+	if (__builtin_expect(!(x >= 0x1p-102F && x < 0x1p127F), 0)) return 1.0F / __builtin_sqrtf(x);
+	const float y = __builtin_amdgcn_rsqf(x);
+	const float q = x * y, s = __builtin_fmaf(__builtin_fmaf(-q, q, x), 0.5F * y, q);
+	const float z = __builtin_amdgcn_rcpf(s);
+	return __builtin_fmaf(__builtin_fmaf(-s, z, 1.0F), z, z); }
+
 __device__ inline void normalize3(float& x, float& y, float& z) {
 	const float len2 = (x*x + y*y) + z*z;
-	const float inv = 1.0F / __builtin_sqrtf(len2);
+	const float inv = recip_sqrt(len2);
 	x = x * inv; y = y * inv; z = z * inv; }
 
 // depth ordering key: float order as unsigned, -0 == +0

@@ -797,7 +797,7 @@ __device__ inline void setup_vector(const Rect& r, const int32_t X[3], const int
 	t.c1 = wsub(wadd(c1, tl12), 1) >> 4;
 	t.c2 = wsub(wadd(c2, tl23), 1) >> 4;
 	t.c3 = wsub(wadd(c3, tl31), 1) >> 4;
-	t.scale = 1.0F / itof(wadd(wadd(t.c1, t.c2), t.c3));
+	t.scale = recip(itof(wadd(wadd(t.c1, t.c2), t.c3)));
 	t.minx = minx; t.miny = miny;
 	t.nqx = maxx > minx ? (maxx - minx + 1) >> 1 : 0;
 	t.nqy = maxy > miny ? (maxy - miny + 1) >> 1 : 0; }
@@ -828,7 +828,7 @@ __device__ inline void setup_scalar(const Rect& r, const int32_t X[3], const int
 	t.dx12 = static_cast<int32_t>(dx12); t.dy12 = static_cast<int32_t>(dy12);
 	t.dx23 = static_cast<int32_t>(dx23); t.dy23 = static_cast<int32_t>(dy23);
 	t.dx31 = static_cast<int32_t>(dx31); t.dy31 = static_cast<int32_t>(dy31);
-	t.scale = 1.0F / static_cast<float>(c1 + c2 + c3);
+	t.scale = recip(static_cast<float>(c1 + c2 + c3));
 	t.minx = minx; t.miny = miny;
 	t.nqx = endx > minx ? (endx - minx + 1) >> 1 : 0;
 	t.nqy = endy > miny ? (endy - miny + 1) >> 1 : 0; }

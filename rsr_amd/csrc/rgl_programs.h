@@ -231,7 +231,7 @@ __device__ inline void ggx_shade(const DrawDesc& d, const ShadeInput& s, float c
 		const float* L = lights + 8 * i;
 		float lx = L[0] - s.p[0], ly = L[1] - s.p[1], lz = L[2] - s.p[2];
 		const float d2 = (lx*lx + ly*ly) + lz*lz;
-		const float inv = 1.0F / __builtin_sqrtf(d2);
+		const float inv = recip_sqrt(d2);
 		lx = lx * inv; ly = ly * inv; lz = lz * inv;
 		const float ndl = (s.n[0]*lx + s.n[1]*ly) + s.n[2]*lz;
 		if (!(ndl > 0.0F)) continue;
@@ -248,7 +248,7 @@ __device__ inline void ggx_shade(const DrawDesc& d, const ShadeInput& s, float c
 		const float F = 0.04F + 0.96F * f5;
 		const float spec = (((D * gl) * gv) * F) / ((4.0F * ndl) * ndv);
 		const float kd = (1.0F - F) * kInvPi;
-		const float id2 = 1.0F / d2;
+		const float id2 = recip(d2);
 #pragma unroll
 		for (int c = 0; c < 3; ++c) acc[c] = acc[c] + ((s.albedo[c] * kd + spec) * (L[4 + c] * id2)) * ndl; }
 	// environment: 8 taps spread around the reflection vector by roughness

@@ -248,7 +248,9 @@ struct rgl_gpu {
 	size_t costReady = 0;          // tileCost entries cleared since allocation
 	uint32_t itemCap = 0;
 	DevArray<unsigned long long> keys;
-	DevArray<VisRec> rec, crec;
+	DevArray<uint4> pairIds;        // inline (triangle, tile) pairs
+	DevArray<uint32_t> pairBoxes;
+	DevArray<VisRec> crec;          // clipped fans' pairs
 	size_t keysReady = 0;           // pixels of keys holding the sentinel
 	DevArray<DrawDesc> dDraws;
 	DevArray<DrawLite> dLite;
@@ -355,7 +357,7 @@ struct rgl_gpu {
 	~rgl_gpu() {
 		for (auto* a : { &qCount, &tileCount, &tileCursor, &tileOff, &clipq, &clipqOf, &clipHist, &clipOff, &clipCursor, &itemTile, &tileCost }) a->release();
 		tileDesc.release(); tileBits.release(); scanPart.release();
-		keys.release(); rec.release(); crec.release();
+		keys.release(); pairIds.release(); pairBoxes.release(); crec.release();
 		probeWant.release(); quadList.release();
 		for (auto* a : { &mlpQueue, &tPart, &tLoss }) a->release();
 		tImg.release();
@@ -672,7 +674,7 @@ struct rgl_gpu {
 		if ((e = Grow(tileCursor, static_cast<long long>(kCountGroups) * b.nTiles + 1)) != hipSuccess) return hipfail(e, "hipMalloc tile cursors");
 		if ((e = Grow(tileOff, b.nTiles + 1)) != hipSuccess) return hipfail(e, "hipMalloc tile offsets");
 		if (listCap < 2 * S + 4096) listCap = static_cast<uint32_t>(std::min<long long>(2 * S + 4096, 0x7fffffffLL));
-		if ((e = Grow(rec, listCap)) != hipSuccess) return hipfail(e, "hipMalloc setup records");
+		if ((e = Grow(pairIds, listCap)) != hipSuccess || (e = Grow(pairBoxes, listCap)) != hipSuccess) return hipfail(e, "hipMalloc pair lists");
 		if (clipCap < std::min<long long>(S, 4096)) clipCap = static_cast<uint32_t>(std::min<long long>(S, 4096));
 		if ((e = Grow(clipq, clipCap)) != hipSuccess) return hipfail(e, "hipMalloc clipq");
 		if ((e = Grow(clipqOf, S)) != hipSuccess) return hipfail(e, "hipMalloc clipqOf");
@@ -1041,7 +1043,7 @@ struct rgl_gpu {
 		mix(lastIo.data(), lastIo.size());
 		const void* ptrs[] = { vpos.p, vflags.p, vvary.p, trect.p, tvert.p, tileCount.p, tileCursor.p, tileOff.p, clipq.p, clipqOf.p,
 		                       cvpos.p, cvvary.p, fcount.p, frect.p, clipHist.p, clipOff.p, clipCursor.p, itemTile.p, tileDesc.p, tileBits.p, scanPart.p, tileCost.p,
-		                       keys.p, rec.p, crec.p, mlpImg.p, probeWant.p, quadList.p, mlpQueue.p, qCount.p, mlpParams,
+		                       keys.p, pairIds.p, pairBoxes.p, crec.p, mlpImg.p, probeWant.p, quadList.p, mlpQueue.p, qCount.p, mlpParams,
 		                       dOps.p, dIo.p, ioRec.p, ioMasks.p, skeys0.p, skeys1.p };
 		mix(ptrs, sizeof(ptrs));
 		const uint32_t caps[] = { listCap, clipCap, clistCap, mlpSegCap, static_cast<uint32_t>(items), learned ? 1u : 0u,
@@ -1164,7 +1166,7 @@ struct rgl_gpu {
 		ra.hostCtr = learned ? nullptr : hCtrDev;
 		if (b.units > 0) {
 			ScatterArgs sa;
-			sa.trect = trect.p; sa.tvert = tvert.p; sa.vpos = vpos.p; sa.cursor = tileCursor.p; sa.rec = rec.p; sa.listCap = listCap;
+			sa.trect = trect.p; sa.tvert = tvert.p; sa.cursor = tileCursor.p; sa.ids = pairIds.p; sa.boxes = pairBoxes.p; sa.listCap = listCap;
 			sa.clipq = clipq.p; sa.fcount = fcount.p; sa.frect = frect.p; sa.cvpos = cvpos.p; sa.clipCap = clipCap;
 			sa.clipCursor = clipCursor.p; sa.crec = crec.p; sa.clistCap = clistCap; sa.clipBlocks = kClipScatterBlocks;
 			sa.tileOff = tileOff.p; sa.clipOff = clipOff.p; sa.keys = keys.p; sa.ctr = dCtr;
@@ -1177,17 +1179,18 @@ struct rgl_gpu {
 			k_scatter<<<(fusedScan ? 1 : 0) + b.units + kClipScatterBlocks + kResetBlocks, kUnitThreads,
 				winBytes + (sa.listed ? listBytes : 0), stream>>>(b, dLite.p, sa); }
 		Mark(5);
+		const PairLists pl{ pairIds.p, pairBoxes.p, vpos.p, dLite.p, b.nDraws };
 		if (nIo < b.nFrames) {
 			// one workgroup per work item, sized from the last completed frame;
 			// the kernel strides over any remainder
 			Dispatch(0, k_vis, dim3(std::min(items, 1 << 20)), dim3(kRasterThreads), 0, b, ra,
-			         static_cast<const VisRec*>(rec.p), static_cast<const VisRec*>(crec.p), static_cast<const uint32_t*>(itemTile.p),
+			         pl, pl.ids, pl.boxes, static_cast<const VisRec*>(crec.p), static_cast<const uint32_t*>(itemTile.p),
 			         static_cast<const VisTile*>(tileDesc.p), b.frames); }
 		// frames drawn in order: the tiles' records sorted by slot, then
 		// every tile region walks them (before k_resolve, whose first block
 		// publishes the frame's counters)
 		if (nIo > 0)
-			k_tile_order<<<nIoTiles, kSortThreads, 0, stream>>>(b, ra, dIo.p, nIo, b.frames, dDraws.p, dLite.p, tileDesc.p, rec.p, crec.p, ioRec.p,
+			k_tile_order<<<nIoTiles, kSortThreads, 0, stream>>>(b, ra, dIo.p, nIo, b.frames, dDraws.p, dLite.p, tileDesc.p, pl, crec.p, ioRec.p,
 				skeys0.p, skeys1.p, ioMasks.p, ioRegions);
 		// everything above writes this executor's buffers alone; what
 		// follows writes or samples the caller's, after the previous

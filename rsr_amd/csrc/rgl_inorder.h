@@ -123,7 +123,7 @@ static_assert(sizeof(IoRec) == 64 && kMaxDraws <= 256 && kMaxAnyTileDim / 2 <= 2
 // the program runs (its colour or its discard is used)
 constexpr uint32_t kStDepthTest = 1u, kStDepthWrite = 2u, kStDepthFunc = 2, kStColor = 16u, kStBlend = 32u, kStEarlyZ = 64u, kStProgram = 128u;
 
-__device__ inline IoRec make_io_rec(const VisRec& r, const DrawLite* __restrict__ lite, const DrawDesc* __restrict__ draws, int nDraws,
+__device__ inline IoRec make_io_rec(const TriSetup& r, const DrawLite* __restrict__ lite, const DrawDesc* __restrict__ draws, int nDraws,
                                     const uint4* __restrict__ tvert, const uint32_t* __restrict__ clipqOf) {
 	const int di = find_draw_slot(lite, nDraws, r.slot);
 	const DrawLite& dl = lite[di];
@@ -135,7 +135,7 @@ __device__ inline IoRec make_io_rec(const VisRec& r, const DrawLite* __restrict_
 	IoRec o;
 	o.c1 = r.c1; o.c2 = r.c2; o.c3 = r.c3;
 	o.dx12 = r.dx12; o.dy12 = r.dy12; o.dx23 = r.dx23; o.dy23 = r.dy23;
-	o.minxy = r.minxy; o.scale = r.scale; o.slot = r.slot;
+	o.minxy = static_cast<uint32_t>(r.minx & 0xffff) | (static_cast<uint32_t>(r.miny) << 16); o.scale = r.scale; o.slot = r.slot;
 	if (rel < nTri) {
 		const uint4 tv = tvert[dl.triBase + srcTri];
 		o.v0 = tv.x; o.v1 = tv.y; o.v2 = tv.z; }
@@ -145,7 +145,7 @@ __device__ inline IoRec make_io_rec(const VisRec& r, const DrawLite* __restrict_
 	const uint32_t st = (dd.depthTest ? kStDepthTest : 0u) | (dd.depthWrite ? kStDepthWrite : 0u) |
 	                    (static_cast<uint32_t>(dd.depthFunc) << kStDepthFunc) | (dd.colorWrite ? kStColor : 0u) |
 	                    (dd.blend ? kStBlend : 0u) | (info.earlyZ ? kStEarlyZ : 0u) | (dd.colorWrite || info.discard ? kStProgram : 0u);
-	o.meta = static_cast<uint32_t>(di) | (st << 8) | ((r.nq & 0xffu) << 16) | ((r.nq >> 16) << 24);
+	o.meta = static_cast<uint32_t>(di) | (st << 8) | ((static_cast<uint32_t>(r.nqx) & 0xffu) << 16) | (static_cast<uint32_t>(r.nqy) << 24);
 	o.prim = dl.primBase + srcTri;
 	o.pad = 0u;
 	return o; }
@@ -170,7 +170,7 @@ __device__ inline long long mask_word(uint32_t ob, int blk, int maxRegions) {
 // passes and barriers (71 -> 31 us with tiles of up to 1,800).
 __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, RasterArgs a, const IoFrame* __restrict__ io, int nIo,
 		const FrameDesc* __restrict__ frames, const DrawDesc* __restrict__ draws, const DrawLite* __restrict__ lite,
-		const VisTile* __restrict__ tileDesc, const VisRec* __restrict__ rec, const VisRec* __restrict__ crec,
+		const VisTile* __restrict__ tileDesc, PairLists pl, const VisRec* __restrict__ crec,
 		IoRec* __restrict__ sorted, unsigned long long* __restrict__ skeys0, unsigned long long* __restrict__ skeys1,
 		unsigned long long* __restrict__ masks, int maxRegions) {
 	__shared__ unsigned long long s[2][kSortCap];
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, Raster
 	const uint32_t n = d.ntot, ninl = d.ninl, ob = d.ib + d.cb;
 	const uint32_t t = threadIdx.x, lane = t & 63;
 	auto key_of = [&](uint32_t p) -> unsigned long long {
-		const uint32_t slot = p < ninl ? rec[d.ib + p].slot : crec[d.cb + (p - ninl)].slot;
+		const uint32_t slot = p < ninl ? pl.ids[d.ib + p].w : crec[d.cb + (p - ninl)].slot;
 		return (static_cast<unsigned long long>(slot) << 32) | p; };
 	// records c0 .. c0 + cn - 1 sorted in LDS; returns the buffer they end in
 	auto sort_lds = [&](uint32_t c0, uint32_t cn) {
@@ -217,9 +217,11 @@ __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, Raster
 		int gx0 = 1, gx1 = 0, gy0 = 1, gy1 = 0;   // the regions the record's quads reach (none)
 		if (64 * k + lane < n) {
 			const uint32_t p = static_cast<uint32_t>(keys[64 * k + lane]);
-			const VisRec r = p < ninl ? rec[d.ib + p] : crec[d.cb + (p - ninl)];
-			const int minx = static_cast<int>(r.minxy & 0xffffu) - R.x0, miny = static_cast<int>(r.minxy >> 16) - R.y0;
-			const int nqx = static_cast<int>(r.nq & 0xffffu), nqy = static_cast<int>(r.nq >> 16);
+			TriSetup r;
+			if (p < ninl) pair_setup(pl, pl.ids[d.ib + p], (pl.boxes[d.ib + p] & kBoxScissor) != 0u, R, r);
+			else rec_setup(crec[d.cb + (p - ninl)], r);
+			const int minx = r.minx - R.x0, miny = r.miny - R.y0;
+			const int nqx = r.nqx, nqy = r.nqy;
 			if (nqx > 0 && nqy > 0) {
 				gx0 = minx / kRegionDim; gx1 = (minx + 2 * nqx - 1) / kRegionDim;
 				gy0 = miny / kRegionDim; gy1 = (miny + 2 * nqy - 1) / kRegionDim; }

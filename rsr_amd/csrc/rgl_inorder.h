@@ -287,7 +287,7 @@ template <class L>
 __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs a, const IoFrame* __restrict__ io, int nIo,
 		const FrameDesc* __restrict__ frames, const FrameOp* __restrict__ ops, const DrawDesc* __restrict__ draws,
 		const DrawLite* __restrict__ lite, const VisTile* __restrict__ tileDesc, const IoRec* __restrict__ sorted,
-		const unsigned long long* __restrict__ masks, int maxRegions) {
+		const unsigned long long* __restrict__ masks, int maxRegions, const uint32_t* __restrict__ order) {
 	// 64 words of the region's record masks and the set bits before each
 	__shared__ unsigned long long smask[64];
 	__shared__ uint32_t spre[65];
@@ -312,12 +312,17 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	constexpr int kRun = 64 * kXcds;
 	const int wg = static_cast<int>(blockIdx.x);
 	const int blk = wg < static_cast<int>(gridDim.x) / kRun * kRun ? wg / kRun * kRun + (wg % kXcds) * 64 + (wg / kXcds) % 64 : wg;
-	const IoFrame e = io[find_io(io, nIo, blk, false)];
+	// With `order` (frames drawn in order alone, of one tile size) the tiles
+	// come as the scan ordered them, the most records first in classes of
+	// powers of two, so that the longest regions do not start last.
+	const IoFrame e0 = io[order ? 0 : find_io(io, nIo, blk, false)];
+	const int rpt = e0.regionsX * e0.regionsY;
+	const int lb = blk - e0.blockStart, ltn = lb / rpt, reg = lb - ltn * rpt;
+	const int tile = order ? static_cast<int>(order[ltn]) : frames[e0.frame].tileBase + ltn;
+	const VisTile vt = tileDesc[tile];
+	const IoFrame e = order && nIo > 1 ? io[vt.flags & 0xffu] : e0;
 	const FrameDesc& f = frames[e.frame];
-	const int rpt = e.regionsX * e.regionsY;
-	const int lb = blk - e.blockStart;
-	const int lt = lb / rpt, reg = lb - lt * rpt;
-	const int tile = f.tileBase + lt;
+	const int lt = tile - f.tileBase;
 	const Rect R = tile_rect(f, lt);
 	const int rgy = reg / e.regionsX, rgx = reg - rgy * e.regionsX;
 	const int rx0 = R.x0 + rgx * kRegionDim, ry0 = R.y0 + rgy * kRegionDim;
@@ -335,7 +340,6 @@ __global__ __launch_bounds__(kIoThreads) void k_inorder(BatchDesc b, RasterArgs 
 	float ca = 0.0F;   // RB_RGBAF32's alpha: set by clears, never drawn
 	uint32_t pid = 0xffffffffu;
 	uint32_t frags = 0;
-	const VisTile vt = tileDesc[tile];
 	const uint32_t n = vt.ntot, ob = vt.ib + vt.cb;
 	uint32_t opi = static_cast<uint32_t>(f.opBase);
 	const uint32_t ope = static_cast<uint32_t>(f.opBase + f.nOps);

@@ -448,7 +448,10 @@ __device__ inline uint32_t vis_regions(const BatchDesc& b, uint32_t cost, uint32
 // two of three tiles are empty, and k_vis takes 238 us without their items
 // (265 with them, of which a part is the descriptor's: frame, regions and
 // tile position come ready, with no division an item).
+// A tile of an in-order frame is one item: k_vis passes over it, and
+// k_inorder takes its tiles in the items' order.
 __device__ inline uint32_t vis_items(const BatchDesc& b, const FrameDesc& f, uint32_t pairs, uint32_t nseg, uint32_t nreg) {
+	if (f.inOrder) return 1u;
 	return pairs == 0u && b.skipEmpty && f.shiftX >= 0 ? 0u : nseg * nreg; }
 
 constexpr int kCostClasses = 33;   // cost 0, then [2^(c-1), 2^c) for c = 1 .. 32
@@ -512,10 +515,10 @@ __device__ inline void col_scan_block(const BatchDesc& b, const uint32_t* __rest
 			col += grp[g]; }
 		if (t < nT) {
 			v = clipHist[t];
-			cost = o.tileCost[t];
+			fr = find_base(ftb, b.nFrames, t);
+			cost = b.frames[fr].inOrder ? col + v : o.tileCost[t];   // in order: this frame's records
 			nseg = vis_segments(b, col + v);
 			nreg = vis_regions(b, cost, nseg);
-			fr = find_base(ftb, b.nFrames, t);
 			items = vis_items(b, b.frames[fr], col + v, nseg, nreg);
 			o.tileCost[t] = 0u; }
 		uint32_t tot, ctot;
@@ -610,12 +613,12 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_local(BatchDesc b, const 
 	const uint32_t ex = block_exclusive_scan(col, sh, tot);
 	const uint32_t cex = block_exclusive_scan(v, sh, ctot);
 	if (t < nT) {
-		const uint32_t cost = tileCost[t];
+		const int fr = find_base(ftb, b.nFrames, t);
+		const FrameDesc& f = b.frames[fr];
+		const uint32_t cost = f.inOrder ? col + v : tileCost[t];   // in order: this frame's records
 		tileCost[t] = 0u;
 		const uint32_t nseg = vis_segments(b, col + v), nreg = vis_regions(b, cost, nseg);
 		const int cls = cost_class(cost);
-		const int fr = find_base(ftb, b.nFrames, t);
-		const FrameDesc& f = b.frames[fr];
 		VisTile d;   // provisional: local prefixes, counts and (pad) the cost class
 		d.item0 = vis_items(b, f, col + v, nseg, nreg);
 		atomicAdd(&classItems[cls], d.item0);

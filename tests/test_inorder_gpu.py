@@ -115,3 +115,27 @@ def test_record_counts(n, width, height):
     sc = _walls(n, width, height)
     sc.blend, sc.tile_blocks, sc.name = True, (8, 8), f"blended_{sc.name}"
     _compare(sc.name, oracle_backend.render(sc, threads=8), rgl.render(sc))
+
+
+@pytest.mark.parametrize("frames", [[(512, 512, 8)], [(520, 512, 8)], [(400, 360, 8), (401, 377, 8)], [(400, 360, 8), (401, 377, 4)]],
+                         ids=str)
+def test_tiles_by_their_records(frames):
+    # 4,096 regions, row by row; 4,608 in one frame and 5,376 in two, tiles
+    # with the most records first; two tile sizes, row by row again
+    import dataclasses
+    from oracle_backend import render as oracle_render
+    from rsr_amd import rgl, scenes
+    from test_batch_gpu import _recorders
+    from test_parity_gpu import _compare
+    scs = [dataclasses.replace(scenes.scene_icospheres(w, h, instances=24 + k, tex_dim=256), blend=True, tile_blocks=(tb, tb),
+                               name=f"ordered_{w}x{h}_{tb}") for k, (w, h, tb) in enumerate(frames)]
+    recs = _recorders(scs)
+    ex = rgl.GPU(0)
+    ex.run_batch_and_wait([g for g, _ in recs], torch.cuda.current_stream().cuda_stream)
+    refs = [oracle_render(sc, threads=8) for sc in scs]
+    for (g, ds), sc, ref in zip(recs, scs, refs):
+        _compare(sc.name, ref, (*ds.outputs(), ref[3]))
+    assert ex.stats()["fragments"] == sum(r[3]["fragments"] for r in refs)
+    ex.close()
+    for g, _ in recs:
+        g.close()

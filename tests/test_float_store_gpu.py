@@ -36,3 +36,25 @@ def test_kawase_passes_match_oracle(h, w):
         got = dst.cpu().numpy()
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), d
         src, cur = dst, want
+
+
+@pytest.mark.parametrize("h,w", [(1, 1), (16, 32), (17, 33), (47, 65)])
+@pytest.mark.parametrize("d", [0, 1, 4, 5, 6, 40])
+def test_kawase_tiles_match_oracle(h, w, d):
+    # tiles of 32 x 16 pixels up to d = 5, a thread per pixel beyond; rows
+    # wider than the canvas; infinities and NaN where they land
+    from oracle_backend import lib as olib
+    from rsr_amd import rgl
+    rng = np.random.default_rng(100 * h + d)
+    img = rng.uniform(-1, 1, (h, w, 4)).astype(np.float32)
+    img[h // 2, w // 2] = (np.inf, -0.0, 3e38, 1e-45)
+    wide = torch.full((h, w + 3, 4), 7.0, device="cuda")
+    src, dst = wide.clone(), wide.clone()
+    src[:, :w] = torch.from_numpy(img).cuda()
+    rgl.kawase_blur(src[:, :w], dst[:, :w], d)
+    torch.cuda.synchronize()
+    want = np.full_like(img, 5.0)
+    olib().rglo_kawase_blur(img.ctypes.data, want.ctypes.data, w, h, w, w, d)
+    got = dst.cpu().numpy()
+    assert np.array_equal(got[:, :w].view(np.uint32), want.view(np.uint32))
+    assert (got[:, w:] == 7.0).all()

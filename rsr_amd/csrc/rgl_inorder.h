@@ -88,19 +88,30 @@ __device__ inline unsigned long long wave_sort(unsigned long long v) {
 			if ((low == up) ? o < v : o > v) v = o; }
 	return v; }
 
-// one merge pass over n distinct keys in sorted runs of `run`: each key's
-// place in its merged run of 2 run is its index in its own run plus its
-// rank (binary search) in the other
+// one merge pass over n distinct keys in sorted runs of `run` (a power of
+// two): each key's place in its merged run of 2 run is its index in its own
+// run plus its rank in the other.  A thread searches for two keys at a time,
+// so that one's loads fill the other's latency.
 __device__ inline void merge_runs(const unsigned long long* src, unsigned long long* dst, uint32_t n, uint32_t run) {
-	for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-		const uint32_t a0 = i & ~(2 * run - 1);
-		const uint32_t a1 = min(a0 + run, n), b1 = min(a0 + 2 * run, n);
-		const unsigned long long key = src[i];
-		const bool inA = i < a1;
-		uint32_t lo = inA ? a1 : a0, hi = inA ? b1 : a1;
-		const uint32_t own = inA ? i - a0 : i - a1, base = lo;
-		while (lo < hi) { const uint32_t mid = (lo + hi) >> 1; if (src[mid] < key) lo = mid + 1; else hi = mid; }
-		dst[a0 + own + (lo - base)] = key; }}
+	for (uint32_t i = threadIdx.x; i < n; i += 2 * blockDim.x) {
+		unsigned long long key[2];
+		uint32_t other[2], len[2], rank[2] = { 0, 0 }, out[2];
+#pragma unroll
+		for (uint32_t k = 0; k < 2; ++k) {
+			const uint32_t j = min(i + k * blockDim.x, n - 1);   // past the last key: that key again, not stored
+			const uint32_t a0 = j & ~(2 * run - 1), a1 = min(a0 + run, n), b1 = min(a0 + 2 * run, n);
+			const bool inA = j < a1;
+			key[k] = src[j];
+			other[k] = inA ? a1 : a0; len[k] = inA ? b1 - a1 : a1 - a0;
+			out[k] = inA ? j : j - run; }   // the place without the other run's keys
+		for (uint32_t s = run; s > 0; s >>= 1)
+#pragma unroll
+			for (uint32_t k = 0; k < 2; ++k) {
+				const uint32_t at = rank[k] + s;
+				if (at <= len[k] && src[other[k] + at - 1] < key[k]) rank[k] = at; }
+#pragma unroll
+		for (uint32_t k = 0; k < 2; ++k)
+			if (i + k * blockDim.x < n) dst[out[k] + rank[k]] = key[k]; }}
 
 // A tile's record as k_inorder reads it: the setup (dx31 = -(dx12 + dx23)
 // and dy31 likewise, in the wrapping arithmetic of the setup), its
@@ -167,7 +178,9 @@ __device__ inline long long mask_word(uint32_t ob, int blk, int maxRegions) {
 // the lanes of a wave, then merged in LDS (up to kSortCap records, and above
 // that in global memory), each pass a binary search per key: six passes of
 // LDS latency for 4,096 records, where a bitonic network in LDS took 78
-// passes and barriers (71 -> 31 us with tiles of up to 1,800).
+// passes and barriers (71 -> 31 us with tiles of up to 1,800).  With the
+// pairs set up here 38.2 us; 34.5 with two keys a thread searched together
+// and a record's regions from 8 + 8 ballots instead of 64.
 __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, RasterArgs a, const IoFrame* __restrict__ io, int nIo,
 		const FrameDesc* __restrict__ frames, const DrawDesc* __restrict__ draws, const DrawLite* __restrict__ lite,
 		const VisTile* __restrict__ tileDesc, PairLists pl, const VisRec* __restrict__ crec,
@@ -226,15 +239,14 @@ __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, Raster
 				gx0 = minx / kRegionDim; gx1 = (minx + 2 * nqx - 1) / kRegionDim;
 				gy0 = miny / kRegionDim; gy1 = (miny + 2 * nqy - 1) / kRegionDim; }
 			sorted[ob + 64 * k + lane] = make_io_rec(r, lite, draws, b.nDraws, a.tvert, a.clipqOf); }
-		unsigned long long mine = 0;
-		int reg = 0;
-		for (int gy = 0; gy < e.regionsY; ++gy)
-			for (int gx = 0; gx < e.regionsX; ++gx, ++reg) {
-				const unsigned long long m = __ballot(gx0 <= gx && gx <= gx1 && gy0 <= gy && gy <= gy1);
-				if ((reg & 63) == static_cast<int>(lane)) mine = m;
-				if ((reg & 63) == 63) tm[static_cast<long long>(reg - 63 + static_cast<int>(lane)) * nb + k] = mine; }
-		const int rest = reg & 63;
-		if (static_cast<int>(lane) < rest) tm[static_cast<long long>(reg - rest + static_cast<int>(lane)) * nb + k] = mine; }}
+		// a lane per region, its word the ballots of its column and its row
+		const int regions = e.regionsX * e.regionsY;
+		for (int reg0 = 0; reg0 < regions; reg0 += 64) {
+			const int reg = reg0 + static_cast<int>(lane), ry = reg / e.regionsX, rx = reg - ry * e.regionsX;
+			unsigned long long col = 0, rowm = 0;
+			for (int g = 0; g < e.regionsX; ++g) { const unsigned long long m = __ballot(gx0 <= g && g <= gx1); if (rx == g) col = m; }
+			for (int g = 0; g < e.regionsY; ++g) { const unsigned long long m = __ballot(gy0 <= g && g <= gy1); if (ry == g) rowm = m; }
+			if (reg < regions) tm[static_cast<long long>(reg) * nb + k] = col & rowm; }}}
 
 // the draw's program on one lane of a quad, the vertices' varyings loaded
 // with the triangle's vertex ids

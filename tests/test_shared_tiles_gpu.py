@@ -46,3 +46,24 @@ def test_walls(n, width, height):
     ref = oracle_backend.render(sc, threads=8)
     # the first frame may report a full list: render() draws it again
     _compare(sc.name, ref, rgl.render(sc))
+
+
+@pytest.mark.parametrize("n,width,height,blocks,cull", [(1, 64, 40, (8, 8), False), (7, 131, 77, (5, 3), False), (63, 200, 120, (3, 8), True),
+                                                        (1025, 120, 72, (4, 4), False), (2050, 97, 61, (8, 8), True)])
+def test_triangles_around_the_camera(n, width, height, blocks, cull):
+    # triangles that cross several clipping planes (polygons of three to eight
+    # vertices, parts left of and above the frame), tiles that are no power of
+    # two, more triangles than the clipping launch has waves
+    import oracle_backend
+    from rsr_amd import rgl
+    from test_parity_gpu import _compare
+    sc = scenes.scene_clip_floor(width, height, 2)
+    rng = np.random.RandomState(n)
+    pos = rng.uniform(-4, 4, (3 * n, 3)).astype(np.float32)
+    nrm = np.tile(np.array([[0, 0, 1]], np.float32), (3 * n, 1))
+    uv = rng.uniform(-1, 2, (3 * n, 2)).astype(np.float32)
+    sc.meshes = [scenes.Mesh(scenes._mesh_buffers(pos, nrm, uv), np.arange(3 * n, dtype=np.uint16))]
+    sc.tile_blocks, sc.cull, sc.name = blocks, cull, f"around{n}_{width}x{height}"
+    ref = oracle_backend.render(sc, threads=8)
+    assert n == 1 or ref[3]["clipped"] > n // 2
+    _compare(sc.name, ref, rgl.render(sc))

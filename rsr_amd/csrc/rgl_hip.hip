@@ -804,8 +804,13 @@ struct rgl_gpu {
 			b.unitTris = kUnitTris * std::min(32, b.unitWindow / (2 * kUnitTris));
 			b.unitWindow = UnitWindow(draws, triBase, b.unitTris, b.unitDraws); }
 		b.units = static_cast<int>((triBase + b.unitTris - 1) / b.unitTris);
-		// the setup's LDS holds the draw table and the unit's tile window
-		if (sizeof(DrawLite) * draws.size() + sizeof(uint32_t) * static_cast<size_t>(b.unitWindow) > kUnitLdsBytes)
+		// the unit's tile window lies in LDS, in the setup beside the unit's
+		// draws (the bound counts the batch's) and in the scatter beside its
+		// own arrays: a launch that asks for more than a workgroup has fails,
+		// and the kernels after it would read lists that were never written
+		const size_t winBytes = sizeof(uint32_t) * static_cast<size_t>(b.unitWindow);
+		if (sizeof(DrawLite) * draws.size() + winBytes > kUnitLdsBytes ||
+		    kScatterLdsBytes + winBytes + (FusedScan(b) ? kFusedBytes : 0) > kUnitLdsBytes)
 			return fail(RGL_E_UNSUPPORTED, "a binning unit's frames span too many tiles for its LDS table; use larger tiles");
 		b.nBlocks = blockBase; b.segPairs = segPairs; b.splitQuads = splitQuads; b.skipEmpty = 0; b.frames = nullptr;
 		long long vtot = 0;
@@ -1127,8 +1132,7 @@ struct rgl_gpu {
 	           const std::vector<SampleReq>& reqs) {
 		hipError_t e;
 		const size_t dlBytes = sizeof(DrawLite) * static_cast<size_t>(std::max(b.nDraws, 1));
-		// small batches scan inside k_scatter (kFusedScanTiles)
-		const bool fusedScan = b.nTiles <= kFusedScanTiles && b.units > 0;
+		const bool fusedScan = FusedScan(b);
 		const ZeroArgs za{ dCtr, clipHist.p, b.nTiles, tileCount.p, qCount.p, fusedScan ? tileCursor.p : nullptr,
 		                   fusedScan ? clipCursor.p : nullptr };
 		// a double-buffered frame reads the caller's buffers only after the
@@ -1150,7 +1154,9 @@ struct rgl_gpu {
 		Mark(1);
 		if (b.units > 0) {
 			k_setup_count<<<b.units, kUnitThreads, b.unitDraws * sizeof(DrawLite) + b.unitWindow * sizeof(uint32_t), stream>>>(dLite.p, b, vpos.p, vflags.p, trect.p, tvert.p,
-				tileCount.p, clipq.p, clipqOf.p, clipCap, dCtr); }
+				tileCount.p, clipq.p, clipqOf.p, clipCap, dCtr);
+			// what follows indexes by what this wrote: nothing does without it
+			if ((e = hipGetLastError()) != hipSuccess) return hipfail(e, "setup launch"); }
 		Mark(2);
 		// clipping: the clip queue is complete after setup; the clipped
 		// per-tile counts feed the scan below
@@ -1189,7 +1195,8 @@ struct rgl_gpu {
 			sa.scan = so;
 			sa.scan.tileCursor = nullptr; sa.scan.clipCursor = nullptr;
 			k_scatter<<<(fusedScan ? 1 : 0) + b.units + kClipScatterBlocks + kResetBlocks, kUnitThreads,
-				winBytes + (sa.listed ? listBytes : 0), stream>>>(b, dLite.p, sa); }
+				winBytes + (fusedScan ? kFusedBytes : sa.listed ? listBytes : 0), stream>>>(b, dLite.p, sa);
+			if ((e = hipGetLastError()) != hipSuccess) return hipfail(e, "scatter launch"); }
 		Mark(5);
 		const PairLists pl{ pairIds.p, pairBoxes.p, vpos.p, dLite.p, b.nDraws };
 		if (nIo < b.nFrames) {
@@ -1262,8 +1269,11 @@ struct rgl_gpu {
 		return 0; }
 
 	static constexpr int kClipScatterBlocks = 32;   // k_scatter blocks that place the clipped fans
-	static constexpr size_t kScatterLdsBytes = 6 * 1024;  // k_scatter's own arrays, at most
+	static constexpr size_t kScatterLdsBytes = (sizeof(ScatterLds) + 15) / 16 * 16;   // k_scatter's own arrays; the dynamic part starts 16-byte aligned
+	static constexpr size_t kFusedBytes = kFusedScanTiles * sizeof(uint32_t);         // the fused scan's tile bases
 	static constexpr size_t kUnitLdsBytes = 160 * 1024;   // LDS per workgroup on gfx950
+	// small batches scan inside k_scatter (kFusedScanTiles)
+	static bool FusedScan(const BatchDesc& b) { return b.nTiles <= kFusedScanTiles && b.units > 0; }
 	static constexpr int kResetBlocks = 128;        // k_scatter blocks that reset the keys of multi-segment tiles
 
 	// ---- learned shading: one forward + backward pass over a batch ----

@@ -488,18 +488,26 @@ struct ScanOut {
 	unsigned long long* tileBits;   // a bit per tile with records (64 tiles a word)
 };
 
+template <int kThreads>
+struct ScanLds {
+	uint32_t sh[kThreads / 64 + 1];
+	int ftb[kMaxFrames + 1];
+	uint32_t classItems[kCostClasses], classCursor[kCostClasses];
+};
+
 template <int kThreads, int kTiles>
 __device__ inline void col_scan_block(const BatchDesc& b, const uint32_t* __restrict__ tileCount,
-		const uint32_t* __restrict__ clipHist, const ScanOut& o) {
-	__shared__ uint32_t sh[kThreads / 64 + 1];
-	__shared__ int ftb[kMaxFrames + 1];
+		const uint32_t* __restrict__ clipHist, const ScanOut& o, ScanLds<kThreads>& lds) {
+	uint32_t* const sh = lds.sh;
+	int* const ftb = lds.ftb;
+	uint32_t* const classItems = lds.classItems;
+	uint32_t* const classCursor = lds.classCursor;
 	load_tile_bases(ftb, b);
 	__syncthreads();
 	const int nT = b.nTiles;   // at most kTiles: each thread keeps its tiles' descriptors in registers
 	constexpr int kPer = kTiles / kThreads;
 	VisTile mine[kPer];
 	int mcls[kPer];
-	__shared__ uint32_t classItems[kCostClasses], classCursor[kCostClasses];
 	for (int c = threadIdx.x; c < kCostClasses; c += kThreads) classItems[c] = 0u;
 	uint32_t carry = 0, ccarry = 0;
 #pragma unroll
@@ -578,7 +586,8 @@ __device__ inline void col_scan_block(const BatchDesc& b, const uint32_t* __rest
 
 __global__ __launch_bounds__(kScanThreads) void k_col_scan(BatchDesc b, const uint32_t* __restrict__ tileCount,
 		const uint32_t* __restrict__ clipHist, ScanOut o) {
-	col_scan_block<kScanThreads, kScanSplitTiles>(b, tileCount, clipHist, o); }
+	__shared__ ScanLds<kScanThreads> lds;
+	col_scan_block<kScanThreads, kScanSplitTiles>(b, tileCount, clipHist, o, lds); }
 
 // Large batches scan in three launches instead of one block: per block of
 // kScanThreads tiles the local prefixes and per-class item counts
@@ -1174,6 +1183,16 @@ __device__ inline void reset_keys(const BatchDesc& b, const int* ftb, int rb, in
 constexpr uint32_t kSharedTiles = 4;
 constexpr int kBigCap = 512;   // such triangles a unit lists; with more than these its lanes walk them all
 
+// k_scatter's own LDS.  The host adds the launch's dynamic part (the unit's
+// tile window and, after it, the fused scan's tile bases or the unit's list)
+// and refuses a batch whose sum a workgroup cannot have.
+struct ScatterLds {
+	ScanLds<kUnitThreads> scan;      // block 0 of the fused scan; the others use its frame table and scan words
+	uint32_t cpre[kUnitThreads];     // clip blocks and large triangles: pair prefixes
+	uint16_t big[kBigCap];           // the unit's large triangles
+	uint32_t nbig, nlist;
+};
+
 // With the fused scan, block 0 is the scan's and the others shift by one.
 // Blocks [0, units): one binning unit each.  The unit counts its pairs per
 // tile in LDS, reserves one block of list positions per tile it touches
@@ -1182,20 +1201,23 @@ constexpr int kBigCap = 512;   // such triangles a unit lists; with more than th
 // writes the pair's entries.  Blocks [units, units + clipBlocks): the
 // clipped fans.  The rest: key resets.
 __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const DrawLite* __restrict__ dl, ScatterArgs a) {
-	// dynamic LDS: the unit's tile-window counts, then write cursors; the
-	// draw table is read through the caches
+	// dynamic LDS: the unit's tile-window counts, then write cursors; after
+	// them the tile bases (fused) or the unit's list (listed); the draw table
+	// is read through the caches
 	extern __shared__ uint4 dyn_lds[];
-	__shared__ int ftb[kMaxFrames + 1];
-	__shared__ uint32_t fbase[kFusedScanTiles];   // fused: per tile, this block's list (or clipped-list) base
-	__shared__ uint32_t fsh[kUnitThreads / 64 + 1];
-	__shared__ uint32_t cpre[kUnitThreads];      // clip blocks and large triangles: pair prefixes
-	__shared__ uint16_t big[kBigCap];            // the unit's large triangles
-	__shared__ uint32_t nbig, nlist;
+	__shared__ ScatterLds lds;
+	int* const ftb = lds.scan.ftb;
+	uint32_t* const fsh = lds.scan.sh;
+	uint32_t* const cpre = lds.cpre;
+	uint16_t* const big = lds.big;
+	uint32_t& nbig = lds.nbig;
+	uint32_t& nlist = lds.nlist;
 	uint32_t* base = reinterpret_cast<uint32_t*>(dyn_lds);
+	uint32_t* const fbase = base + b.unitWindow;   // fused: per tile, this block's list (or clipped-list) base
 	int u = blockIdx.x;
 	int nblk = static_cast<int>(gridDim.x);
 	if (a.fused) {
-		if (u == 0) { col_scan_block<kUnitThreads, kFusedScanTiles>(b, a.tileCount, a.clipHist, a.scan); return; }
+		if (u == 0) { col_scan_block<kUnitThreads, kFusedScanTiles>(b, a.tileCount, a.clipHist, a.scan, lds.scan); return; }
 		--u; --nblk; }
 	if (u >= b.units + a.clipBlocks) {
 		load_tile_bases(ftb, b);

@@ -15,6 +15,8 @@
 // have (same tile-clamped edge start values, same barycentric scale).
 #pragma once
 
+#include <type_traits>
+
 #include "rgl_programs.h"
 
 namespace rgl {
@@ -1662,14 +1664,20 @@ __device__ inline void clear_block(uint32_t* outColor, uint32_t* outDepth, uint3
 	if (outPrim) outPrim[o] = 0xffffffffu; }
 
 // Waves per SIMD the resolve is compiled for.  It waits on memory half of its
-// time, so a program's resolve takes the registers that leave eight waves
-// (64) rather than the few more the compiler would like: icospheres at
-// 1920x1080 25.6 -> 23.3 us, 64 scenes 143 -> 126.  The heavy shader's long
-// arithmetic would spill (285 -> 305 us on four 4K views), and the resolve of
-// mixed programs holds them all.
-template <class S> constexpr int kResolveWaves = 8;
-template <> constexpr int kResolveWaves<ShadeOne<ProgGGXEnv>> = 1;
-template <> constexpr int kResolveWaves<ShadeAny> = 1;
+// time, so where a program's own registers leave eight waves (64), or miss
+// them by one, its resolve is held to them: icospheres at 1920x1080 25.6 ->
+// 23.3 us, 64 scenes 143 -> 126 (a register over), a frame of the textured
+// sphere and ground 88.8 -> 86.3, of the pattern 68.4 -> 67.7.  Programs that
+// need more spill under the bound and take the compiler's choice: 1080p
+// frames of the mesh programs 70.1 us (OBJ2, 69 registers; 75.0 bound, 31
+// spills) and 75.4 (OBJ2S, 79; 96.1 bound, 127 spills), the heavy shader's
+// resolve of four 4K views 285 (83; 305 bound).  So do programs this list
+// does not name: what they need is not known here.
+template <class P, class... Ps> constexpr bool kOneOf = (std::is_same_v<P, Ps> || ...);
+template <class S> constexpr int kResolveWaves = 1;
+template <class P> constexpr int kResolveWaves<ShadeOne<P>> =
+	kOneOf<P, ProgBase, ProgAmy, ProgMany, ProgLambertTex, ProgManyBlinnPhong, ProgAlphaTexture, ProgText, ProgDepth, ProgPattern, ProgOBJ1,
+	       ProgEnvmap> ? 8 : 1;
 
 // What places a resolve block: the frames' first blocks, and, so that a
 // batch of one frame needs no load for it, that frame's tile grid (its grid

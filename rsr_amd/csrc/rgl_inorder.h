@@ -231,7 +231,9 @@ __global__ __launch_bounds__(kSortThreads) void k_tile_order(BatchDesc b, Raster
 		if (64 * k + lane < n) {
 			const uint32_t p = static_cast<uint32_t>(keys[64 * k + lane]);
 			TriSetup r;
-			if (p < ninl) pair_setup(pl, pl.ids[d.ib + p], (pl.boxes[d.ib + p] & kBoxScissor) != 0u, R, r);
+			if (p < ninl) {
+				const uint4 id = pl.ids[d.ib + p];
+				pair_setup(pl, id, pair_rect(pl, id, pl.boxes[d.ib + p], R), r); }
 			else rec_setup(crec[d.cb + (p - ninl)], r);
 			const int minx = r.minx - R.x0, miny = r.miny - R.y0;
 			const int nqx = r.nqx, nqy = r.nqy;

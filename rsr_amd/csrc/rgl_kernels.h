@@ -1350,9 +1350,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 // ---------------------------------------------------------------------------
 constexpr int kQuadWindow = 2048;   // quads mapped to their triangle per pass
 constexpr int kCullSpan = 2048;     // pairs tested against the region per pass
-constexpr uint32_t kPairScissor = 0x80000000u;
-constexpr uint32_t kListScissor = 0x8000u;   // a listed pair's draw has a scissor rectangle
-static_assert(kCullSpan <= 0x8000, "a listed pair's number and its flag share 16 bits");
+static_assert(kCullSpan <= 0x10000, "a listed pair's number in its pass has 16 bits");
 constexpr uint32_t kWholeTile = (0x7fu << 7) | (0x7fu << 21);   // a box that reaches every region
 
 // A record prepared for a region, as the quad loop reads it: one of four
@@ -1365,18 +1363,23 @@ constexpr uint32_t kWholeTile = (0x7fu << 7) | (0x7fu << 21);   // a box that re
 //   1: dx12 dy12 dx23 dy23   2: dx31 dy31 1/across scale   3: z0 z1 z2 slot
 struct VisRows { uint4 c[4][kRasterThreads]; };
 
-// an inline pair's setup against its tile's rectangle R
-__device__ inline void pair_setup(const PairLists& l, const uint4& id, bool scissored, const Rect& R, TriSetup& t) {
+// an inline pair's setup against R, its tile's rectangle (cut by the draw's
+// scissor rectangle, where it has one: pair_rect)
+__device__ inline void pair_setup(const PairLists& l, const uint4& id, const Rect& R, TriSetup& t) {
 	TriVerts tr;
 	inline_verts(id, l.vpos, tr);
+	setup_vector(R, tr.X, tr.Y, t);
+	t.z0 = tr.z[0]; t.z1 = tr.z[1]; t.z2 = tr.z[2];
+	t.slot = id.w; }
+// Draws with a scissor rectangle are drawn in order: k_tile_order asks, k_vis
+// takes the tile's rectangle.
+__device__ inline Rect pair_rect(const PairLists& l, const uint4& id, uint32_t box, const Rect& R) {
 	Rect r = R;
-	if (scissored) {
+	if (box & kBoxScissor) {
 		const DrawLite& d = l.lite[find_draw_slot(l.lite, l.nDraws, id.w)];
 		r.x0 = imax(r.x0, d.scissor[0]); r.y0 = imax(r.y0, d.scissor[1]);
 		r.x1 = imin(r.x1, d.scissor[2]); r.y1 = imin(r.y1, d.scissor[3]); }
-	setup_vector(r, tr.X, tr.Y, t);
-	t.z0 = tr.z[0]; t.z1 = tr.z[1]; t.z2 = tr.z[2];
-	t.slot = id.w; }
+	return r; }
 __device__ inline void rec_setup(const VisRec& r, TriSetup& t) {
 	t.c1 = r.c1; t.c2 = r.c2; t.c3 = r.c3;
 	t.dx12 = r.dx12; t.dy12 = r.dy12; t.dx23 = r.dx23; t.dy23 = r.dy23; t.dx31 = r.dx31; t.dy31 = r.dy31;
@@ -1817,33 +1820,29 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 						base = __builtin_amdgcn_readfirstlane(base);
 						if (hit)
 							list[base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u))] =
-								static_cast<uint16_t>((q - p0 + u * kRasterThreads + threadIdx.x) | (bx[u] & kBoxScissor ? kListScissor : 0u)); }}
+								static_cast<uint16_t>(q - p0 + u * kRasterThreads + threadIdx.x); }}
 				__syncthreads();
 				n = nList; }
 			// each thread holds one pair's vertices; the next round's are
 			// loaded while this round rasterises
 			uint4 idn;
-			uint32_t pn = 0;   // the pair's number in the tile | kPairScissor
+			uint32_t pn = 0;   // the pair's number in the tile
 			auto fetch = [&](uint32_t i) {
 				if (i >= n) return;
-				uint32_t sc;
-				if (listed) { const uint32_t e = list[i]; pn = p0 + (e & ~kListScissor); sc = e & kListScissor; }
-				else { pn = p0 + i; sc = pn < ninl ? boxes[ib + pn] & kBoxScissor : 0u; }
-				if (pn < ninl) idn = ids[ib + pn];
-				if (sc) pn |= kPairScissor; };
+				pn = p0 + (listed ? list[i] : i);
+				if (pn < ninl) idn = ids[ib + pn]; };
 			fetch(threadIdx.x);
 			for (uint32_t b0 = 0; b0 < n; b0 += kRasterThreads, par ^= 1u) {
 				const uint32_t i = b0 + threadIdx.x;
 				const uint4 id = idn;
-				const uint32_t p = pn & ~kPairScissor;
-				const bool scissored = (pn & kPairScissor) != 0u;
+				const uint32_t p = pn;
 				fetch(i + kRasterThreads);
 				uint32_t nq = 0, nx = 0, x0 = 0, y0 = 0;
 				int32_t c1 = 0, c2 = 0, c3 = 0;
 				bool small = true;
 				TriSetup r;
 				if (i < n) {
-					if (p < ninl) pair_setup(pl, id, scissored, R, r);
+					if (p < ninl) pair_setup(pl, id, R, r);
 					else rec_setup(crec[cb + (p - ninl)], r);
 					const int minx = r.minx, miny = r.miny, nqx = r.nqx, nqy = r.nqy;
 					// the triangle's quads inside the region

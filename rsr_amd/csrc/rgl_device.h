@@ -330,6 +330,7 @@ struct BatchDesc {
 	int segPairs;            // (triangle, tile) pairs per visibility work item
 	int splitQuads;          // quad work per quadrant from which it is cut in 2, and from twice this in 4 (0: never)
 	int skipEmpty;           // 1: tiles without records get no keys and resolve to the clear values (frames with shiftX >= 0)
+	int ioOrdered;           // 1: k_inorder takes the tiles in the work items' order (every frame is drawn in order)
 	int unitDraws;           // most draws one binning unit's triangles lie in
 	int unitWindow;          // most tiles one binning unit's frames span (its LDS tile table)
 	const FrameDesc* frames; // device table, nFrames entries

@@ -793,6 +793,7 @@ struct rgl_gpu {
 		ioSame = static_cast<int>(io.size()) == n && ioBlocks > kIoOrderBlocks;
 		for (const IoFrame& e : io) ioSame = ioSame && e.regionsX == io[0].regionsX && e.regionsY == io[0].regionsY;
 		BatchDesc b;
+		std::memset(&b, 0, sizeof(b));   // GraphKey hashes its bytes
 		b.nFrames = n; b.nTiles = tileBase; b.nDraws = static_cast<int>(draws.size());
 		// binning units: kUnitTris triangles, grown in steps of kUnitTris
 		// when the tiles a unit's frames span (its LDS table, cleared and
@@ -812,7 +813,7 @@ struct rgl_gpu {
 		if (sizeof(DrawLite) * draws.size() + winBytes > kUnitLdsBytes ||
 		    kScatterLdsBytes + winBytes + (FusedScan(b) ? kFusedBytes : 0) > kUnitLdsBytes)
 			return fail(RGL_E_UNSUPPORTED, "a binning unit's frames span too many tiles for its LDS table; use larger tiles");
-		b.nBlocks = blockBase; b.segPairs = segPairs; b.splitQuads = splitQuads; b.skipEmpty = 0; b.frames = nullptr;
+		b.nBlocks = blockBase; b.segPairs = segPairs; b.splitQuads = splitQuads; b.skipEmpty = 0; b.ioOrdered = ioSame ? 1 : 0; b.frames = nullptr;
 		long long vtot = 0;
 		for (const auto& d : draws) vtot += static_cast<long long>(d.instances) * d.verts;
 		hipError_t e;

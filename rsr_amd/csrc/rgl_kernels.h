@@ -450,10 +450,11 @@ __device__ inline uint32_t vis_regions(const BatchDesc& b, uint32_t cost, uint32
 // two of three tiles are empty, and k_vis takes 238 us without their items
 // (265 with them, of which a part is the descriptor's: frame, regions and
 // tile position come ready, with no division an item).
-// A tile of an in-order frame is one item: k_vis passes over it, and
-// k_inorder takes its tiles in the items' order.
+// A tile of an in-order frame has none for k_vis.  Where k_inorder takes the
+// tiles in the items' order (every frame is drawn in order: k_vis isn't
+// launched), it is one.
 __device__ inline uint32_t vis_items(const BatchDesc& b, const FrameDesc& f, uint32_t pairs, uint32_t nseg, uint32_t nreg) {
-	if (f.inOrder) return 1u;
+	if (f.inOrder) return b.ioOrdered ? 1u : 0u;
 	return pairs == 0u && b.skipEmpty && f.shiftX >= 0 ? 0u : nseg * nreg; }
 
 constexpr int kCostClasses = 33;   // cost 0, then [2^(c-1), 2^c) for c = 1 .. 32
@@ -1770,7 +1771,6 @@ __global__ __launch_bounds__(kRasterThreads) void k_vis(BatchDesc b, RasterArgs 
 		const bool multiSeg = (it.flags >> 12) != 0u;
 		// the frame table is read-only (restrict): its fields come by scalar loads
 		const FrameDesc& f = frames[it.flags & 0xffu];
-		if (f.inOrder) continue;   // drawn by the in-order tile path (uniform)
 		const bool leq = f.depthFunc == 1;
 		Rect R;
 		R.x0 = static_cast<int>(it.xy & 0xffffu) * f.tileW; R.y0 = static_cast<int>(it.xy >> 16) * f.tileH;

@@ -21,6 +21,8 @@ import sys
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "librgl_hip.so")
+TESTS = os.path.join(os.path.dirname(PKG), "tests")
+CHECKS_LIB = os.path.join(TESTS, "libdevice_checks.so")   # exhaustive checks of device functions, for the tests
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("RGL_OFFLOAD_ARCH", "gfx950")
 
@@ -36,13 +38,21 @@ FLAGS = [
 def build(verbose: bool = False, programs: str | None = None, out: str = LIB) -> str:
     """Compiles the library to *out*; *programs* names a header of user
     programs to add to the built-in ones."""
-    src = os.path.join(CSRC, "rgl_hip.hip")
     extra = []
     if programs is not None:
         header = os.path.abspath(programs)
         if not os.path.isfile(header):
             raise FileNotFoundError(header)
         extra = [f'-DRGL_USER_PROGRAMS="{header}"']
+    return _compile(os.path.join(CSRC, "rgl_hip.hip"), out, extra, verbose)
+
+
+def build_checks(verbose: bool = False) -> str:
+    """Compiles the tests' library of device checks, with the same flags."""
+    return _compile(os.path.join(TESTS, "device_checks.hip"), CHECKS_LIB, [], verbose)
+
+
+def _compile(src: str, out: str, extra: list, verbose: bool) -> str:
     cmd = [HIPCC, *FLAGS, *extra, "-o", out + ".tmp", src]
     if verbose:
         print(" ".join(cmd), flush=True)

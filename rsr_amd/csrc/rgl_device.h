@@ -218,9 +218,8 @@ __device__ inline void xform3w0(const float* f, const float b[3], float o[3]) {
 // third of their instructions: the compiler's expansions scale and fix up
 // for the whole range of exponents, these correct the hardware's estimate
 // by FMAs where no step can leave the normal range and take the operators
-// elsewhere (zero, subnormal, huge, infinite, NaN).  Compared with the
-// operators for each of the 2^31 floats of one sign: no difference for
-// 2^-126 <= x < 2^126 and 2^-102 <= x respectively.
+// elsewhere (zero, subnormal, huge, infinite, NaN).  Equal to the operators
+// for every float (tests/test_device_functions_gpu.py).
 __device__ inline float recip(float x) {
 	if (__builtin_expect(!(__builtin_fabsf(x) >= 0x1p-126F && __builtin_fabsf(x) < 0x1p126F), 0)) return 1.0F / x;
 	const float y = __builtin_amdgcn_rcpf(x);

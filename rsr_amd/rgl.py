@@ -307,20 +307,22 @@ class GPU:
         return self._check(self.L.rgl_gl_use_buffer(self.h, slot, dev_ptr, count if dev_ptr else 0))
 
     def __getattr__(self, name):
-        # a gl_ method's first use: it becomes a method of the class.  Looked
-        # up here and wrapped anew at each call, the recording of the viewer's
-        # three frames (171 calls) took 295 us; with render_calls' arguments
-        # resolved in one loop it takes 213
+        # a gl_ method's first use: it becomes a method of the class, which
+        # calls the library of the object it is called on.  Looked up here and
+        # wrapped anew at each call, the recording of the viewer's three frames
+        # (171 calls) took 295 us; with render_calls' arguments resolved in one
+        # loop it takes 213
         if not name.startswith("gl_"):
             raise AttributeError(name)
-        fn = getattr(self.L, "rgl_" + name)
+        L, symbol = self.L, "rgl_" + name
+        fn = getattr(L, symbol)
 
         def call(self, *args):
             for a in args:
                 if isinstance(a, (np.ndarray, bool)):
                     args = [self._arg(a) for a in args]
                     break
-            rc = fn(self.h, *args)
+            rc = (fn if self.L is L else getattr(self.L, symbol))(self.h, *args)
             return rc if rc >= 0 else self._check(rc)
         call.__name__ = name
         setattr(GPU, name, call)

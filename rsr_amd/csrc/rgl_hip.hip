@@ -872,7 +872,8 @@ struct rgl_gpu {
 			costReady = tileCost.cap; }
 		if (keysReady < keys.cap) {
 			// defined contents after allocation; each frame then resets the
-			// keys of multi-segment tiles in k_pair_setup and overwrites the rest
+			// keys of multi-segment tiles in k_scatter and overwrites the rest, or
+			// in large batches leaves those of empty tiles, which it does not read
 			k_fill_u64<<<1024, 256, 0, stream>>>(keys.p, static_cast<long long>(keys.cap), kKeySentinel);
 			keysReady = keys.cap; }
 		int pid = draws.empty() ? ProgManyBlinnPhong::kId : draws[0].program;

@@ -8,11 +8,11 @@
 // between draws (a depth-only clear for a shadow pass, a store followed by
 // more drawing).
 //
-//   k_tile_order  one workgroup per tile: the tile's (triangle, tile) setup
-//                 records, inline and clipped, sorted by submission slot and
-//                 written in that order with their draw's state and vertices,
-//                 and per region of the tile a bit per sorted record that can
-//                 touch it.
+//   k_tile_order  one workgroup per tile: the tile's (triangle, tile) pairs,
+//                 inline (set up here) and clipped (setup records), sorted by
+//                 submission slot and written in that order as records with
+//                 their draw's state and vertices, and per region of the tile
+//                 a bit per sorted record that can touch it.
 //   k_inorder     one wave per 8 x 8-pixel region of a tile, one lane per
 //                 pixel: the pixel's colour, depth and primitive id stay in
 //                 registers while the wave steps through the region's

@@ -36,6 +36,8 @@ constexpr int kMaxOps = 1024;     // clears and stores per batch
 // Pixels of a batch from which tiles without records get no keys: the
 // resolve's look at the tile's bit costs a small frame half a microsecond
 // (640 x 360: 6.4 -> 6.9 us), and saves a large one 16 B for each such pixel.
+// Between the two the line is drawn by caution: one sphere at 1920 x 1080
+// would take 42.2 us without it (47.0 with), at 2560 x 1440 47.3 (61.0).
 constexpr long long kSkipPixels = 4 << 20;
 
 // Regions of an in-order batch from which k_inorder takes its tiles with the

@@ -1234,7 +1234,7 @@ __global__ __launch_bounds__(kUnitThreads) void k_scatter(BatchDesc b, const Dra
 	const UnitDraws ud = unit_draws(dl, b, u);
 	dl += ud.lo;
 	const TileWindow win = unit_window(dl, ud.n);
-	if (win.n > b.unitWindow) return;   // flagged by the setup
+	if (ud.n > b.unitDraws || win.n > b.unitWindow) return;   // flagged by the setup, which wrote nothing
 	const int grp = u % kCountGroups;
 	if (a.fused) {
 		// per tile: its list offset (the scan of all groups' counts) plus
